@@ -175,7 +175,16 @@ int launch_init(const Sys& s, int64_t W, const jqmc_walkers* wk, void* workspace
     T* S1 = static_cast<T*>(workspace);
     T* S2 = S1 + W * s.n_el * s.n_ao;
     k_init_jsums<T><<<grid_for(W * s.n_ao, B), B, 0, st>>>(s, W, k, S1, S2);
-    k_init_jfield<T><<<grid_for(W * s.n_el * s.n_ao, B), B, 0, st>>>(s, W, k, S1, S2);
+    if constexpr (std::is_same<T, double>::value) {
+      const int64_t n_rt = (W * s.n_el + JG_TILE - 1) / JG_TILE;
+      const int n_ct = (s.n_ao + JG_TILE - 1) / JG_TILE;
+      const int64_t blocks = (n_rt + 7) / 8 * 8 * n_ct;
+      if (blocks > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+      k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, W * s.n_el, S1, S2, k.jfield, n_ct, n_rt);
+    } else {
+      // the mixed form keeps its FP32 sums in AO order: its Markov chains are functions of their rounding
+      k_init_jfield<T><<<grid_for(W * s.n_el * s.n_ao, B), B, 0, st>>>(s, W, k, S1, S2);
+    }
   }
   k_init_jastrow<T><<<grid_for(W, 4), 4 * WAVE, 0, st>>>(s, W, k, 4);
   HIP_TRY(hipGetLastError());

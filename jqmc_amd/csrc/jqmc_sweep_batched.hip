@@ -399,6 +399,97 @@ struct JfMfma<float> {
   static __device__ __forceinline__ int row(int q, int ih) { return 4 * ih + q; }
 };
 
+// J3 fields of every electron of every walker from the prefix sums of k_init_jsums as one FP64 GEMM on
+// the matrix cores: rows = the M = W n_el electrons, G[m, a] = j1[a] + sum_b S1[m, b] J3T[b, a] +
+// sum_b S2[m, b] J3[b, a] (jastrow_factor.py:4121-4135); a symmetric J3 takes one product with S1 + S2.
+// Bound by the FP64 matrix rate (4 n_ao^2 flops per electron): 64 x 64 output tiles, 16-deep slices of
+// both operands through LDS with the next slice in registers, four waves of 2 x 2 MFMA tiles each.
+// The column tiles of a row tile are eight blocks apart, so they run on one XCD and share the rows in
+// its L2.  512 benzene walkers (15360 x 228): 1389 us with one thread per output and n_ao dependent
+// steps, 98 us as this GEMM (33 TFLOP/s).
+constexpr int JG_TILE = 64, JG_KC = 16;
+constexpr int JG_A_LD = JG_KC + 1;    // doubles per LDS row of S: 34 banks apart, no conflict over 16 rows
+constexpr int JG_B_LD = JG_TILE + 8;  // the four 16-lane groups read rows 16 banks apart
+
+__global__ void __launch_bounds__(256) k_init_jfield_mfma(Sys s, int64_t M, const double* __restrict__ S1,
+                                                          const double* __restrict__ S2, double* __restrict__ G,
+                                                          int n_ct, int64_t n_rt) {
+  using MF = JfMfma<double>;
+  __shared__ double a_s[JG_TILE][JG_A_LD];
+  __shared__ double b_s[JG_KC][JG_B_LD];
+  const int64_t blk = blockIdx.x;
+  const int64_t rt = (blk / (8 * n_ct)) * 8 + blk % 8;
+  const int ct = (int)((blk / 8) % n_ct);
+  if (rt >= n_rt) return;  // uniform across the block
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, il = lane & 15, ih = lane >> 4;
+  const int na = s.n_ao, a0 = ct * JG_TILE;
+  const int64_t m0 = rt * JG_TILE;
+  const bool sym = s.j3_sym != 0;
+  const int wr = 32 * (wave >> 1), wc = 32 * (wave & 1);
+  const int n_k = (na + JG_KC - 1) / JG_KC, n_stage = sym ? n_k : 2 * n_k;
+  double pa[4], pb[4];
+  // thread t stages column b0 + t % 16 of rows t / 16 + 16 r of S, and column t % 64 of rows
+  // t / 64 + 4 r of J
+  auto fetch = [&](int st) {
+    const bool second = st >= n_k;
+    const int b0 = (second ? st - n_k : st) * JG_KC;
+    const double* __restrict__ S = second ? S2 : S1;
+    const double* __restrict__ J = second ? s.td.j3 : s.td.j3T;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t m = m0 + (t >> 4) + 16 * r;
+      const int b = b0 + (t & 15);
+      const bool ok = m < M && b < na;
+      pa[r] = ok ? S[m * na + b] : 0.0;
+      if (sym && ok) pa[r] += S2[m * na + b];
+      const int bb = b0 + (t >> 6) + 4 * r, a = a0 + (t & 63);
+      pb[r] = (bb < na && a < na) ? J[(int64_t)bb * na + a] : 0.0;
+    }
+  };
+  MF::v4 acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) acc[x][y] = MF::v4{0, 0, 0, 0};
+  fetch(0);
+  for (int st = 0; st < n_stage; ++st) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      a_s[(t >> 4) + 16 * r][t & 15] = pa[r];
+      b_s[(t >> 6) + 4 * r][t & 63] = pb[r];
+    }
+    __syncthreads();
+    if (st + 1 < n_stage) fetch(st + 1);
+#pragma unroll
+    for (int kk = 0; kk < JG_KC; kk += 4) {
+      double fa[2], fb[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        fa[x] = a_s[wr + 16 * x + il][kk + ih];
+        fb[x] = b_s[kk + ih][wc + 16 * x + il];
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = MF::mma(fa[x], fb[y], acc[x][y]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const int a = a0 + wc + 16 * y + il;
+    if (a >= na) continue;
+    const double j1 = s.td.j3v[a];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t m = m0 + wr + 16 * x + MF::row(q, ih);
+        if (m < M) G[m * na + a] = j1 + acc[x][y][q];
+      }
+  }
+}
+
 // [T1 | T2] = [J3 dA | J3^T dA] on AO rows a0..a0+63 (a0 = 64 blockIdx.x) for the 32 walkers
 // blockIdx.y of the block that accepted, then the field increments on those rows: an up move of
 // e gives t1 to up f < e and t2 to every other electron; a dn move gives t1 to every up electron
