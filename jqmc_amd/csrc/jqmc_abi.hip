@@ -58,6 +58,9 @@ struct jqmc_system {
   // FP64 guard of the mixed form's local energy (jqmc_system_set_mixed_guard)
   double guard_e_ref = 0.0;
   double guard_width = 1.0e4;
+  // shell starts, AO scales and packed AO words kept while the system is built (build_pieces)
+  std::vector<int32_t> host_sh0, host_meta;
+  std::vector<double> host_scale;
   // pinned host words the GFMC_t projections read their active-walker counts into
   int* host_flags = nullptr;
 };
@@ -82,6 +85,106 @@ int upload_f32(jqmc_system* sys, const double* host, size_t count, const float**
   std::vector<float> f(count);
   for (size_t i = 0; i < count; ++i) f[i] = (float)host[i];
   return upload(sys, f.data(), count, dev_out);
+}
+
+// The piece and chunk tables and the packed MO coefficients of the flattened local energy (Sys::pc64 ff.).
+int build_pieces(jqmc_system* sys, const jqmc_system_desc* d) {
+  Sys& s = sys->s;
+  const bool mixed = s.precision == JQMC_PRECISION_MIXED_FP32;
+  std::vector<PieceRec<double>> r64;
+  std::vector<PieceRec<float>> r32;
+  std::vector<PieceMore<double>> m64;
+  std::vector<PieceMore<float>> m32;
+  std::vector<int32_t> chunks;
+  std::vector<double> scale;
+  int in_chunk = 0;
+  for (int k = 0; k < s.n_shell; ++k) {
+    const int s0 = sys->host_sh0[k], s1 = sys->host_sh0[k + 1];
+    const int p0 = d->ao_prim_ptr[s0], np = d->ao_prim_ptr[s0 + 1] - p0;
+    for (int a0 = s0; a0 < s1; a0 += EL_CH) {
+      const int n = std::min(s1 - a0, EL_CH);
+      int l = 0;
+      while (l < 4 && (l + 1) * (l + 2) / 2 < n) ++l;
+      bool fast = l <= 3 && (l + 1) * (l + 2) / 2 == n && s1 - s0 == n;
+      for (int nx = l, i = 0; nx >= 0 && fast; --nx)
+        for (int ny = l - nx; ny >= 0 && fast; --ny, ++i) {
+          const int m = sys->host_meta[a0 + i];
+          fast = (m & AO_UNIT_TERM) && ((m >> 16) & 15) == nx && ((m >> 20) & 15) == ny && ((m >> 24) & 15) == l - nx - ny;
+        }
+      PieceRec<double> x{};
+      PieceRec<float> y{};
+      PieceMore<double> xm{};
+      PieceMore<float> ym{};
+      for (int c = 0; c < 3; ++c) x.c[c] = y.c[c] = d->nuc_pos[3 * d->ao_nuc[a0] + c];
+      const int ni = std::min(np, PIECE_P);
+      x.info = y.info = (fast && np >= 1 && np <= PIECE_P ? np | (l << 4) : PIECE_ANY) | (n << 16);
+      x.a0 = y.a0 = a0;
+      for (int q = 0; q < ni; ++q) {
+        x.zc[2 * q] = -d->prim_exp[p0 + q] * 1.4426950408889634;
+        x.zc[2 * q + 1] = d->prim_coef[p0 + q];
+        y.zc[2 * q] = (float)d->prim_exp[p0 + q];
+        y.zc[2 * q + 1] = (float)d->prim_coef[p0 + q];
+      }
+      if (fast)
+        for (int i = 0; i < n; ++i) {
+          xm.sc[i] = sys->host_scale[a0 + i];
+          ym.sc[i] = (float)sys->host_scale[a0 + i];
+        }
+      xm.p0 = ym.p0 = p0;
+      xm.p1 = ym.p1 = p0 + np;
+      if (chunks.empty() || in_chunk + n > EL_CH) {
+        chunks.insert(chunks.end(), {(int32_t)r64.size(), 0, a0, 0});
+        scale.resize(scale.size() + EL_CH, 0.0);
+        in_chunk = 0;
+      }
+      for (int i = 0; i < n; ++i) scale[scale.size() - EL_CH + in_chunk + i] = sys->host_scale[a0 + i];
+      in_chunk += n;
+      r64.push_back(x);
+      r32.push_back(y);
+      m64.push_back(xm);
+      m32.push_back(ym);
+      chunks[chunks.size() - 3] = (int32_t)r64.size();
+      chunks[chunks.size() - 1] = in_chunk;
+    }
+  }
+  s.n_chunk = (int)(chunks.size() / 4);
+  r64.emplace_back();  // read ahead of the last piece
+  r32.emplace_back();
+  int rc = upload(sys, r64.data(), r64.size(), &s.pc64);
+  if (rc == JQMC_OK) rc = upload(sys, m64.data(), m64.size(), &s.pm64);
+  if (rc == JQMC_OK && mixed) rc = upload(sys, r32.data(), r32.size(), &s.pc32);
+  if (rc == JQMC_OK && mixed) rc = upload(sys, m32.data(), m32.size(), &s.pm32);
+  if (rc == JQMC_OK) rc = upload(sys, chunks.data(), chunks.size(), &s.el_chunks);
+  if (rc == JQMC_OK) rc = upload(sys, scale.data(), scale.size(), &s.el_scale);
+  if (rc != JQMC_OK) return rc;
+  s.el_ks = s.orb_is_mo && s.n_orb <= 64 ? (s.n_orb + 15) / 16 * 4 : 0;
+  s.mo_same = 1;
+  if (s.el_ks == 0) return JQMC_OK;
+  const size_t n_mo = (size_t)s.n_orb * s.n_ao;
+  s.mo_same = std::equal(d->mo_coef_up, d->mo_coef_up + n_mo, d->mo_coef_dn) ? 1 : 0;
+  auto pack = [&](const double* C, bool scaled, const double** out) {
+    std::vector<double> v((size_t)s.n_chunk * s.el_ks * 64, 0.0);
+    for (int c = 0; c < s.n_chunk; ++c)
+      for (int q = 0; q < s.el_ks; ++q)
+        for (int k = 0; k < 4; ++k)
+          for (int j = 0; j < chunks[4 * c + 3]; ++j) {
+            const int o = 4 * q + k;
+            if (o >= s.n_orb) continue;
+            v[((size_t)c * s.el_ks + q) * 64 + j + 16 * k] =
+                C[(size_t)o * s.n_ao + chunks[4 * c + 2] + j] * (scaled ? scale[(size_t)c * EL_CH + j] : 1.0);
+          }
+    return upload(sys, v.data(), v.size(), out);
+  };
+  rc = pack(d->mo_coef_up, true, &s.el_kup);
+  if (rc == JQMC_OK) rc = s.mo_same ? (s.el_kdn = s.el_kup, JQMC_OK) : pack(d->mo_coef_dn, true, &s.el_kdn);
+  if (rc == JQMC_OK && mixed) {
+    rc = pack(d->mo_coef_up, false, &s.el_cup);
+    if (rc == JQMC_OK) rc = s.mo_same ? (s.el_cdn = s.el_cup, JQMC_OK) : pack(d->mo_coef_dn, false, &s.el_cdn);
+  } else {
+    s.el_cup = s.el_kup;
+    s.el_cdn = s.el_kdn;
+  }
+  return rc;
 }
 
 #define UPLOAD(host, count, dst)                                  \
@@ -260,19 +363,22 @@ int launch_sweep_batched(const jqmc_system* sys, int64_t W, const jqmc_walkers* 
   return JQMC_OK;
 }
 
-// Layout of the local-energy workspace: the h rows (and q rows) of every walker, then for the mixed
-// form's FP64 guard the flagged count, the flagged list and GUARD_SLOTS scratch records.
+// Layout of the local-energy workspace: the flattened launches' buffers, then for the mixed form's
+// FP64 guard the flagged count, the flagged list and GUARD_SLOTS scratch records.
 struct ElWs {
-  double* hws;
+  ElBuf eb;
   int* count;
   int* list;
   double* scratch;
   int64_t rec;  // doubles per guard record
 };
 
+inline int64_t el_ws_doubles(const Sys& s, int64_t W) {
+  return W * el_buf_doubles(s, (int64_t)s.n_el * el_parts(s)) + 1;  // an even number of ints rounded up
+}
+
 inline int64_t el_ws_bytes(const Sys& s, int64_t W) {
-  const int64_t rows = s.n_ao + (el2_q_in_lds(s) ? 0 : s.n_orb);
-  int64_t b = W * (int64_t)s.n_el * rows * (int64_t)sizeof(double);
+  int64_t b = el_ws_doubles(s, W) * (int64_t)sizeof(double);
   if (s.precision == JQMC_PRECISION_MIXED_FP32) {
     b += 16 + ((W * (int64_t)sizeof(int) + 15) & ~(int64_t)15);
     b += GUARD_SLOTS * GuardRec::doubles(s) * (int64_t)sizeof(double);
@@ -283,9 +389,8 @@ inline int64_t el_ws_bytes(const Sys& s, int64_t W) {
 inline ElWs el_ws(const Sys& s, int64_t W, void* base) {
   ElWs x{};
   char* p = static_cast<char*>(base);
-  x.hws = reinterpret_cast<double*>(p);
-  const int64_t rows = s.n_ao + (el2_q_in_lds(s) ? 0 : s.n_orb);
-  p += W * (int64_t)s.n_el * rows * (int64_t)sizeof(double);
+  x.eb = el_buf(s, W, (int64_t)s.n_el * el_parts(s), reinterpret_cast<double*>(p));
+  p += el_ws_doubles(s, W) * (int64_t)sizeof(double);
   if (s.precision == JQMC_PRECISION_MIXED_FP32) {
     x.count = reinterpret_cast<int*>(p);
     p += 16;
@@ -297,15 +402,110 @@ inline ElWs el_ws(const Sys& s, int64_t W, void* base) {
   return x;
 }
 
+// ---- the flattened local energy: one launch of each kernel over up to EL_MAX_JOBS walker sets
+
+template <typename T>
+ElJob<T> el_job(const Sys* d_sys, const Sys& s, int64_t W, const WalkT<T>& wk, const ElBuf& B) {
+  ElJob<T> J{};
+  J.sys = d_sys;
+  J.wk = wk;
+  J.W = W;
+  J.Q = B.Q;
+  J.H = B.H;
+  J.te = B.te;
+  J.jc = B.jc;
+  J.jold = B.jold;
+  J.vpot = B.vpot;
+  J.val = B.val;
+  J.val_ld = B.ld_val;
+  J.elist = B.elist;
+  J.necp = B.necp;
+  return J;
+}
+
+// Waves of a k_el_kinetic block: four, or two where four would not leave room for two blocks per CU.
+constexpr int64_t kMaxKineticLds = 80 * 1024;
+template <typename T>
+int el_kin_waves(const Sys& s) {
+  return el_kin_lds<T>(s.n_orb, s.el_ks, EL_KIN_WAVES) <= kMaxKineticLds ? EL_KIN_WAVES : EL_KIN_WAVES / 2;
+}
+
+// The three launches for the jobs of systems host[k] (jobs and host in the same order).
+template <typename T>
+int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
+  int64_t n = 0;
+  for (int k = 0; k < M.n; ++k) {
+    ElJob<T>& J = M.job[k];
+    const Sys& s = *host[k];
+    const int64_t tiles = (s.n_up + 15) / 16 + (s.n_dn + 15) / 16;
+    J.prep0 = n;
+    J.q_blocks = (J.W * tiles + 3) / 4;
+    n += J.q_blocks + (J.W + 3) / 4;
+  }
+  if (n > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+  if (n == 0) return JQMC_OK;
+  k_el_prep<T><<<(unsigned)n, 256, 0, st>>>(M);
+  for (int k = 0; k < M.n; ++k)
+    if (el_h_rows(*host[k])) {
+      const Sys& s = *host[k];
+      const int64_t waves = M.job[k].W * ((s.n_up + 15) / 16 + (s.n_dn + 15) / 16);
+      k_el_hrows<T><<<(unsigned)((waves + 3) / 4), 256, 0, st>>>(M.job[k]);
+    }
+  for (int kq : {4, 8, 12, 16, 0}) {
+    ElJobs<T> G{};
+    int64_t nk = 0, np = 0, lds = 0;
+    int nw = EL_KIN_WAVES;
+    for (int k = 0; k < M.n; ++k) {
+      const Sys& s = *host[k];
+      if (s.el_ks != kq) continue;
+      ElJob<T>& J = G.job[G.n++];
+      J = M.job[k];
+      J.kin0 = nk;
+      nk += (J.W * s.n_el + EL_KIN_ROWS - 1) / EL_KIN_ROWS;
+      nw = std::min(nw, el_kin_waves<T>(s));
+      // points: lattice groups of ten electrons, then per four walkers the groups of listed electrons
+      const bool nonlocal = s.ecp_on && s.nv > 0;
+      const int parts = el_parts(s), per = s.nv > 0 ? std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)) : 1;
+      J.pts0 = np;
+      J.lat_groups = J.lr ? (J.W * s.n_el + EL_SLOTS - 1) / EL_SLOTS : 0;
+      J.ecp_groups = (4 * s.n_el * parts + per - 1) / per;
+      const int64_t ecp = nonlocal ? (J.W + 3) / 4 * J.ecp_groups : 0;
+      np += (J.lat_groups + ecp + 3) / 4;
+    }
+    if (G.n == 0) continue;
+    if (std::max(nk, np) > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+    for (int k = 0; k < M.n; ++k)
+      if (host[k]->el_ks == kq) lds = std::max(lds, el_kin_lds<T>(host[k]->n_orb, kq, nw));
+    const unsigned bk = (unsigned)nk, bp = (unsigned)np;
+    auto run = [&](auto K) {
+      constexpr int KQ = decltype(K)::value;
+      // more than 64 KiB of dynamic LDS has to be allowed once per kernel
+      static const hipError_t allowed =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(&k_el_kinetic<T, KQ>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxKineticLds);
+      (void)allowed;
+      k_el_kinetic<T, KQ><<<bk, nw * WAVE, lds, st>>>(G);
+      if (bp) k_el_points<T, KQ><<<bp, 256, 0, st>>>(G);
+    };
+    if (kq == 4)
+      run(std::integral_constant<int, 4>{});
+    else if (kq == 8)
+      run(std::integral_constant<int, 8>{});
+    else if (kq == 12)
+      run(std::integral_constant<int, 12>{});
+    else if (kq == 16)
+      run(std::integral_constant<int, 16>{});
+    else
+      run(std::integral_constant<int, 0>{});
+  }
+  return JQMC_OK;
+}
+
 template <typename T>
 int launch_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const double* RT, double* e_L,
                         double* kinetic, double* v_total, double* t_elec, void* workspace, hipStream_t st) {
   const Sys& s = sys->s;
-  const int64_t per_wave = el2_lds_bytes(s);
-  if (per_wave > kMaxLdsPerBlock) return fail(JQMC_ERR_UNSUPPORTED, "system too large for the E_L LDS budget");
-  const int wpb = tuned_wpb(per_wave, sys->tune_el_wpb);
-  const dim3 grid(grid_for(W, wpb)), block(wpb * WAVE);
-  const size_t lds = (size_t)wpb * per_wave;
+  if (el2_lds_bytes(s) > kMaxLdsPerBlock) return fail(JQMC_ERR_UNSUPPORTED, "system too large for the E_L LDS budget");
   const WalkT<T> k = to_walk<T>(wk);
   const ElWs ws = el_ws(s, W, workspace);
   ElGuard guard{nullptr, nullptr, 0.0, 0.0};
@@ -316,33 +516,24 @@ int launch_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* w
     guard = ElGuard{ws.list, ws.count, sys->guard_e_ref, sys->guard_width};
     k_zero_int<<<1, 64, 0, st>>>(ws.count);
   }
-  const int team = sys->tune_el_team;
-  if ((team == 2 || team == 4) && el2_lds_bytes(s, team) <= kMaxLdsPerBlock) {
-    if (W > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one block per walker");
-    if (team == 2)
-      k_local_energy_team<T, 2><<<(unsigned)W, 2 * WAVE, el2_lds_bytes(s, 2), st>>>(s, W, k, RT, e_L, kinetic, v_total,
-                                                                                  t_elec, ws.hws, guard);
-    else
-      k_local_energy_team<T, 4><<<(unsigned)W, 4 * WAVE, el2_lds_bytes(s, 4), st>>>(s, W, k, RT, e_L, kinetic, v_total,
-                                                                                  t_elec, ws.hws, guard);
-  } else if (wpb == 4)
-    k_local_energy_pts<T, 4><<<grid, block, lds, st>>>(s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.hws, guard,
-                                                       per_wave);
-  else if (wpb == 2)
-    k_local_energy_pts<T, 2><<<grid, block, lds, st>>>(s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.hws, guard,
-                                                       per_wave);
-  else
-    k_local_energy_pts<T, 1><<<grid, block, lds, st>>>(s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.hws, guard,
-                                                       per_wave);
+  ElJobs<T> M{};
+  M.n = 1;
+  M.job[0] = el_job<T>(sys->d_sys, s, W, k, ws.eb);
+  M.job[0].RT = RT;
+  M.job[0].t_elec = t_elec;
+  const Sys* host = &s;
+  const int rc = launch_el<T>(M, &host, st);
+  if (rc != JQMC_OK) return rc;
+  k_el_final<T><<<grid_for(W, 4), 256, 0, st>>>(M.job[0], e_L, kinetic, v_total, el_parts(s), guard);
   if constexpr (std::is_same<T, float>::value) {
     if (guarded) {
       const unsigned slots = (unsigned)std::min<int64_t>(GUARD_SLOTS, W);
       if (guard_lds_bytes(s, 8) <= kMaxLdsPerBlock)
         k_local_energy_guard<512><<<slots, 512, guard_lds_bytes(s, 8), st>>>(
-            s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.hws, ws.list, ws.count, ws.scratch, ws.rec);
+            s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.list, ws.count, ws.scratch, ws.rec);
       else
         k_local_energy_guard<256><<<slots, 256, guard_lds_bytes(s, 4), st>>>(
-            s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.hws, ws.list, ws.count, ws.scratch, ws.rec);
+            s, W, k, RT, e_L, kinetic, v_total, t_elec, ws.list, ws.count, ws.scratch, ws.rec);
     }
   }
   HIP_TRY(hipGetLastError());
@@ -403,19 +594,6 @@ int lr_poll(int* const* act, int n, int it, int* host, hipStream_t st, bool* don
   return JQMC_OK;
 }
 
-// Waves per walker of the LRDMC Hamiltonian launch: a team of LR_TEAM waves when W one-wave walkers
-// would leave fewer than 8 waves per SIMD of the 1024 (W < 8192), the walker has work enough to
-// share (n_el n_ao >= 4096: measured, the team loses on the 10- and 30-electron chains with 24 and
-// 120 AOs and wins from benzene's 30 x 228 up) and the team's LDS fits; else one wave.  A function
-// of the system and W only, so that the single and the multi-system launch take the same
-// arithmetic.
-template <typename T>
-int lr_team(const Sys& s, int64_t W) {
-  return (W < 8192 && (int64_t)s.n_el * s.n_ao >= 4096 && lr_ham_lds_bytes<T>(s, LR_TEAM) <= kMaxLdsPerBlock)
-             ? LR_TEAM
-             : 1;
-}
-
 // The LRDMC move's dA rows and movers in the form the J3 product kernel takes (no offsets).
 template <typename T>
 SweepWs<T> lr_jfield_ws(const LrState& S) {
@@ -425,26 +603,51 @@ SweepWs<T> lr_jfield_ws(const LrState& S) {
   return ws;
 }
 
-// One Hamiltonian launch, one move launch and (with J3) one J3 field launch per projection
-// (LR_MEASURE: the Hamiltonian only).
+// The local-energy job of projection `it` of a call (LR_MEASURE: at the given rotations).
 template <typename T>
-int launch_lrdmc(const Sys& s, int64_t W, const jqmc_walkers* wk, const LrArgs& A, int* host_flags, hipStream_t st) {
-  const int64_t per_ham = lr_ham_lds_bytes<T>(s), per_move = lr_move_lds_bytes<T>(s);
-  if (std::max(per_ham, per_move) > kMaxLdsPerBlock)
+ElJob<T> lr_job(const Sys* d_sys, const Sys& s, int64_t W, const WalkT<T>& wk, const LrArgs& A, int it) {
+  ElJob<T> J = el_job<T>(d_sys, s, W, wk, A.st.eb);
+  J.lr = 1;
+  J.measure = A.mode == LR_MEASURE;
+  J.RT = J.measure ? A.RT : A.st.RT;
+  J.RT_new = J.measure ? nullptr : A.st.RT;
+  J.RT_copy = J.measure ? nullptr : A.RT;
+  J.tau = A.st.tau;
+  J.nproj = A.st.nproj;
+  J.act = A.st.act;
+  J.tau0 = A.tau;
+  J.alat = A.alat;
+  J.seed = A.seed;
+  J.step = A.step0 + it;
+  J.dlt = A.dlt;
+  J.random_mesh = A.random_mesh;
+  J.it = it;
+  J.tau_mode = A.mode == LR_FIXED_TAU;
+  return J;
+}
+
+// The elements' launches, one move launch and (with J3) one J3 field launch per projection
+// (LR_MEASURE: the elements and their sums).
+template <typename T>
+int launch_lrdmc(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const LrArgs& A, int* host_flags,
+                 hipStream_t st) {
+  const Sys& s = sys->s;
+  const int64_t per_move = lr_move_lds_bytes<T>(s);
+  if (std::max(lr_ham_lds_bytes<T>(s), per_move) > kMaxLdsPerBlock)
     return fail(JQMC_ERR_UNSUPPORTED, "system too large for the LRDMC LDS budget");
-  const int wpb_h = walkers_per_block(per_ham), wpb_m = walkers_per_block(per_move);
-  const int team = lr_team<T>(s, W);
-  const int64_t team_ham = lr_ham_lds_bytes<T>(s, LR_TEAM);
+  const int wpb_m = walkers_per_block(per_move);
   const WalkT<T> k = to_walk<T>(wk);
   const int rounds = A.mode == LR_MEASURE ? 1 : A.n_steps;
+  const Sys* host = &s;
   for (int it = 0; it < rounds; ++it) {
-    if (team == LR_TEAM)
-      (lr_wide(s) ? k_lrdmc_ham_team<T, true> : k_lrdmc_ham_team<T, false>)<<<(unsigned)W, LR_TEAM * WAVE, team_ham,
-                                                                              st>>>(s, W, k, A, it);
-    else
-      (lr_wide(s) ? k_lrdmc_ham<T, true> : k_lrdmc_ham<T, false>)<<<grid_for(W, wpb_h), wpb_h * WAVE, wpb_h * per_ham,
-                                                                    st>>>(s, W, k, A, it, wpb_h, per_ham);
-    if (A.mode != LR_MEASURE) {
+    ElJobs<T> M{};
+    M.n = 1;
+    M.job[0] = lr_job<T>(sys->d_sys, s, W, k, A, it);
+    const int erc = launch_el<T>(M, &host, st);
+    if (erc != JQMC_OK) return erc;
+    if (A.mode == LR_MEASURE) {
+      k_lrdmc_measure<T><<<grid_for(W, 4), 256, 0, st>>>(s, W, k, A);
+    } else {
       k_lrdmc_move<T><<<grid_for(W, wpb_m), wpb_m * WAVE, wpb_m * per_move, st>>>(s, W, k, A, it, wpb_m, per_move);
       if (s.j3_on) {
         const dim3 jg(grid_for(s.n_ao, JF_ROWS), grid_for(W, JF_WALKERS));
@@ -462,6 +665,19 @@ int launch_lrdmc(const Sys& s, int64_t W, const jqmc_walkers* wk, const LrArgs& 
   }
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
+}
+
+// The elements' launches of every system of a multi-system call that is still projecting at round it.
+template <typename T>
+int lr_multi_elements(const LrMulti<T>& M, const Sys* const* hsys, int it, hipStream_t st) {
+  ElJobs<T> E{};
+  const Sys* host[LR_MAX_SYSTEMS];
+  for (int slot = 0; slot < M.n_sys; ++slot) {
+    if (M.sys[slot].W == 0 || it >= M.args[slot].n_steps) continue;
+    host[E.n] = hsys[slot];
+    E.job[E.n++] = lr_job<T>(M.sys[slot].sys, *hsys[slot], M.sys[slot].W, M.wk[slot], M.args[slot], it);
+  }
+  return launch_el<T>(E, host, st);
 }
 
 // The J3 field launch of every system of a multi-system move launch that has J3 and is still
@@ -705,6 +921,9 @@ int jqmc_system_create(const jqmc_system_desc* d, jqmc_system** out) {
       }
     }
     UPLOAD(rec.data(), rec.size(), s.shrec);
+    sys->host_sh0 = sh0;
+    sys->host_scale = scale;
+    sys->host_meta = meta;
   }
   UPLOAD_REAL(d->prim_exp, d->n_prim, prim_exp);
   UPLOAD_REAL(d->prim_coef, d->n_prim, prim_coef);
@@ -735,6 +954,14 @@ int jqmc_system_create(const jqmc_system_desc* d, jqmc_system** out) {
     UPLOAD_REAL(lp.data(), lp.size(), lam_p);
     UPLOAD_REAL(lpt.data(), lpt.size(), lam_pT);
     if (unp > 0) UPLOAD_REAL(lu.data(), (size_t)n_orb * unp, lam_u);
+  }
+
+  {
+    const int rc = build_pieces(sys, d);
+    if (rc != JQMC_OK) {
+      jqmc_system_destroy(sys);
+      return rc;
+    }
   }
 
   // J3 over the AO basis
@@ -990,8 +1217,8 @@ int jqmc_counter_add(int64_t* ctr, int64_t inc, void* stream) {
 int jqmc_local_energy_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes) {
   if (!sys || !bytes) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (W < 0) return fail(JQMC_ERR_SHAPE, "W < 0");
-  // the determinant field rows h_e of every electron (FP64), the q_e rows when they do not fit LDS,
-  // and in the mixed form the FP64 guard's list and scratch
+  // q_e (and, above 64 MOs, h_e) of every electron, its parts of e_L, and in the mixed form the FP64
+  // guard's list and scratch
   *bytes = el_ws_bytes(sys->s, W);
   return JQMC_OK;
 }
@@ -1073,10 +1300,9 @@ int lrdmc_check(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const
 }
 
 int lrdmc_launch(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const LrArgs& A, void* stream) {
-  const Sys& s = sys->s;
   hipStream_t st = (hipStream_t)stream;
-  return s.precision == JQMC_PRECISION_MIXED_FP32 ? launch_lrdmc<float>(s, W, wk, A, sys->host_flags, st)
-                                                  : launch_lrdmc<double>(s, W, wk, A, sys->host_flags, st);
+  return sys->s.precision == JQMC_PRECISION_MIXED_FP32 ? launch_lrdmc<float>(sys, W, wk, A, sys->host_flags, st)
+                                                       : launch_lrdmc<double>(sys, W, wk, A, sys->host_flags, st);
 }
 
 LrArgs lr_args(const jqmc_lrdmc_params* prm) {
@@ -1098,7 +1324,7 @@ extern "C" {
 int jqmc_lrdmc_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes) {
   if (!sys || !bytes) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (W < 0) return fail(JQMC_ERR_SHAPE, "W < 0");
-  *bytes = lr_ws_bytes(sys->s, W);  // determinant field rows (and q rows) of every walker
+  *bytes = lr_ws_bytes(sys->s, W);
   return JQMC_OK;
 }
 
@@ -1113,8 +1339,7 @@ int jqmc_lrdmc_projection(const jqmc_system* sys, int64_t W, const jqmc_walkers*
   if (!workspace || workspace_bytes < lr_ws_bytes(sys->s, W))
     return fail(JQMC_ERR_WORKSPACE, "workspace of %lld bytes required", (long long)lr_ws_bytes(sys->s, W));
   LrArgs A = lr_args(prm);
-  A.hws = static_cast<double*>(workspace);
-  A.st = lr_state(sys->s, W, A.hws);
+  A.st = lr_state(sys->s, W, static_cast<double*>(workspace));
   A.seed = seed;
   A.step0 = step0;
   A.w = w_L;
@@ -1136,8 +1361,7 @@ int jqmc_lrdmc_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walker
   if (!workspace || workspace_bytes < lr_ws_bytes(sys->s, W))
     return fail(JQMC_ERR_WORKSPACE, "workspace of %lld bytes required", (long long)lr_ws_bytes(sys->s, W));
   LrArgs A = lr_args(prm);
-  A.hws = static_cast<double*>(workspace);
-  A.st = lr_state(sys->s, W, A.hws);
+  A.st = lr_state(sys->s, W, static_cast<double*>(workspace));
   A.mode = LR_MEASURE;
   A.RT = const_cast<double*>(RT);
   A.V_diag = V_diag;
@@ -1156,9 +1380,8 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
   if (!systems || !W || !wks || !params || !step0 || !w_L || !workspaces || !workspace_bytes)
     return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   const int prec = systems[0] ? systems[0]->s.precision : -1;
-  // One walker per 64-thread block, so that a system whose walkers need a whole LDS / register
-  // budget does not leave the other SIMDs of a CU idle; the systems with the most work per walker
-  // take the first blocks (longest first), the smallest fill the tail.
+  // The systems with the most work per walker take the first blocks of every launch (longest first), the
+  // smallest fill the tail.
   std::vector<int> order(n_sys);
   std::vector<double> cost(n_sys, 0.0);
   for (int k = 0; k < n_sys; ++k) {
@@ -1171,7 +1394,7 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
   int64_t blocks = 0, lds_move = 0;
-  int rounds = 0, team[LR_MAX_SYSTEMS];
+  int rounds = 0;
   LrMulti<double> Md{};
   LrMulti<float> Mf{};
   Md.n_sys = Mf.n_sys = n_sys;
@@ -1185,15 +1408,11 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
     if (W[k] > 0 && (!workspaces[k] || workspace_bytes[k] < lr_ws_bytes(sys->s, W[k])))
       return fail(JQMC_ERR_WORKSPACE, "workspace %d: %lld bytes required", k, (long long)lr_ws_bytes(sys->s, W[k]));
     const bool mixed = prec == JQMC_PRECISION_MIXED_FP32;
-    const int64_t per_ham = mixed ? lr_ham_lds_bytes<float>(sys->s) : lr_ham_lds_bytes<double>(sys->s);
+    const int64_t per_ham = lr_ham_lds_bytes<double>(sys->s);
     const int64_t per_move = mixed ? lr_move_lds_bytes<float>(sys->s) : lr_move_lds_bytes<double>(sys->s);
     if (std::max(per_ham, per_move) > kMaxLdsPerBlock)
       return fail(JQMC_ERR_UNSUPPORTED, "system %d too large for the LRDMC LDS budget", k);
-    team[slot] = mixed ? lr_team<float>(sys->s, W[k]) : lr_team<double>(sys->s, W[k]);
-    const int64_t ham_lds = team[slot] == LR_TEAM ? (mixed ? lr_ham_lds_bytes<float>(sys->s, LR_TEAM)
-                                                           : lr_ham_lds_bytes<double>(sys->s, LR_TEAM))
-                                                  : per_ham;
-    LrSystem e{sys->d_sys, W[k], ham_lds, per_move, blocks};
+    LrSystem e{sys->d_sys, W[k], blocks};
     blocks += W[k];
     lds_move = std::max<int64_t>(lds_move, per_move);
     rounds = std::max(rounds, params[k].n_steps);
@@ -1206,8 +1425,7 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
     A.V_nondiag = V_nondiag ? V_nondiag[k] : nullptr;
     A.tau_left = tau_left ? tau_left[k] : nullptr;
     A.n_proj = n_proj ? n_proj[k] : nullptr;
-    A.hws = static_cast<double*>(workspaces[k]);
-    A.st = lr_state(sys->s, W[k], A.hws);
+    A.st = lr_state(sys->s, W[k], static_cast<double*>(workspaces[k]));
     Md.sys[slot] = Mf.sys[slot] = e;
     Md.args[slot] = Mf.args[slot] = A;
     Md.wk[slot] = to_walk<double>(&wks[k]);
@@ -1215,25 +1433,6 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
   }
   if (blocks == 0) return JQMC_OK;
   if (blocks > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers in one launch");
-  // the Hamiltonian launches: one per (team size, determinant-field form) present, each over its
-  // systems' walkers; group g = (one wave ? 1 : 0) + (lr_wide ? 2 : 0)
-  LrMulti<double> Hd[4]{};
-  LrMulti<float> Hf[4]{};
-  int64_t h_blocks[4] = {0, 0, 0, 0}, h_lds[4] = {0, 0, 0, 0};
-  for (int slot = 0; slot < n_sys; ++slot) {
-    const int g = (team[slot] == LR_TEAM ? 0 : 1) + (lr_wide(systems[order[slot]]->s) ? 2 : 0);
-    const int j = Hd[g].n_sys++;
-    Hf[g].n_sys = Hd[g].n_sys;
-    Hd[g].sys[j] = Md.sys[slot];
-    Hd[g].sys[j].block_start = h_blocks[g];
-    Hf[g].sys[j] = Hd[g].sys[j];
-    Hd[g].wk[j] = Md.wk[slot];
-    Hf[g].wk[j] = Mf.wk[slot];
-    Hd[g].args[j] = Md.args[slot];
-    Hf[g].args[j] = Mf.args[slot];
-    h_blocks[g] += Md.sys[slot].W;
-    h_lds[g] = std::max(h_lds[g], Md.sys[slot].lds_ham);
-  }
   const Sys* hsys[LR_MAX_SYSTEMS];  // host copies of the systems, in slot order
   for (int slot = 0; slot < n_sys; ++slot) hsys[slot] = &systems[order[slot]]->s;
   hipStream_t st = (hipStream_t)stream;
@@ -1245,17 +1444,13 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
   }
   for (int it = 0; it < rounds; ++it) {
     if (prec == JQMC_PRECISION_MIXED_FP32) {
-      if (h_blocks[0]) k_lrdmc_ham_multi<float, LR_TEAM, false><<<(unsigned)h_blocks[0], LR_TEAM * WAVE, h_lds[0], st>>>(Hf[0], it);
-      if (h_blocks[1]) k_lrdmc_ham_multi<float, 1, false><<<(unsigned)h_blocks[1], WAVE, h_lds[1], st>>>(Hf[1], it);
-      if (h_blocks[2]) k_lrdmc_ham_multi<float, LR_TEAM, true><<<(unsigned)h_blocks[2], LR_TEAM * WAVE, h_lds[2], st>>>(Hf[2], it);
-      if (h_blocks[3]) k_lrdmc_ham_multi<float, 1, true><<<(unsigned)h_blocks[3], WAVE, h_lds[3], st>>>(Hf[3], it);
+      const int rc = lr_multi_elements<float>(Mf, hsys, it, st);
+      if (rc != JQMC_OK) return rc;
       k_lrdmc_move_multi<float><<<(unsigned)blocks, WAVE, lds_move, st>>>(Mf, it);
       lr_multi_jfield<float>(Mf, hsys, it, st);
     } else {
-      if (h_blocks[0]) k_lrdmc_ham_multi<double, LR_TEAM, false><<<(unsigned)h_blocks[0], LR_TEAM * WAVE, h_lds[0], st>>>(Hd[0], it);
-      if (h_blocks[1]) k_lrdmc_ham_multi<double, 1, false><<<(unsigned)h_blocks[1], WAVE, h_lds[1], st>>>(Hd[1], it);
-      if (h_blocks[2]) k_lrdmc_ham_multi<double, LR_TEAM, true><<<(unsigned)h_blocks[2], LR_TEAM * WAVE, h_lds[2], st>>>(Hd[2], it);
-      if (h_blocks[3]) k_lrdmc_ham_multi<double, 1, true><<<(unsigned)h_blocks[3], WAVE, h_lds[3], st>>>(Hd[3], it);
+      const int rc = lr_multi_elements<double>(Md, hsys, it, st);
+      if (rc != JQMC_OK) return rc;
       k_lrdmc_move_multi<double><<<(unsigned)blocks, WAVE, lds_move, st>>>(Md, it);
       lr_multi_jfield<double>(Md, hsys, it, st);
     }

@@ -42,6 +42,29 @@ struct RealTabs {
 constexpr int SHR_PMAX = 4, SHR_AMAX = 6;
 constexpr int SHR_P = 4, SHR_SC = SHR_P + 2 * SHR_PMAX, SHREC = 20;
 
+// AO pieces of the flattened local energy: the shells, those of more than EL_CH AOs cut into runs of at
+// most EL_CH, grouped in order into chunks of at most EL_CH AOs.  A record is read at a wave-uniform
+// index by scalar loads; T is the arithmetic type of the AO values.
+constexpr int EL_CH = 12;                   // AOs per chunk
+constexpr int PIECE_P = 4, PIECE_A = 10;    // primitives and AO scales in the record
+// info of a record: primitives | degree << 4 | PIECE_ANY | AOs << 16.  PIECE_ANY: not the canonical Cartesian
+// AOs of a degree <= 3 as unit monomials with at most PIECE_P primitives; taken from the per-AO and
+// primitive tables.
+constexpr int PIECE_ANY = 1 << 8;
+// The record holds what every piece needs, so that the table of a molecule stays in the scalar cache; the
+// rest is in PieceMore.
+template <typename T>
+struct alignas(32) PieceRec {
+  double c[3];         // centre
+  int info, a0;        // see above; first AO
+  T zc[2 * PIECE_P];   // FP64: (-exponent log2 e, coefficient); FP32: (exponent, coefficient)
+};
+template <typename T>
+struct PieceMore {
+  T sc[PIECE_A];       // AO scales (not PIECE_ANY)
+  int p0, p1;          // its primitives in the primitive tables
+};
+
 struct Sys {
   int n_nuc, n_ao, n_prim, n_up, n_dn, n_el, n_orb, n_unp;
   int orb_is_mo, j1_type, j2_type, j3_on, j3_sym, precision;
@@ -61,6 +84,17 @@ struct Sys {
   const int* ao_sh;          // (n_ao) shell of each AO
   const int* ao_meta;        // (n_ao) shell | nx << 16 | ny << 20 | nz << 24 | AO_UNIT_TERM
   const double* shrec;       // (n_shell, SHREC) shell records (below)
+  int n_chunk, el_ks, mo_same;  // chunks; k-steps of four orbitals (0: h rows from memory); C_up equals C_dn
+  const PieceRec<double>* pc64;
+  const PieceMore<double>* pm64;
+  const PieceRec<float>* pc32;  // mixed precision only
+  const PieceMore<float>* pm32;
+  const int* el_chunks;      // (n_chunk, 4) first piece, end piece, first AO, number of AOs
+  const double* el_scale;    // (n_chunk, EL_CH) AO scales, zero-padded
+  // MO coefficients packed as matrix-core operands (n_chunk, el_ks, 64): lane j + 16 k of step q holds
+  // C[4 q + k][first AO + j], zero outside; el_k*: times the AO scale (kinetic), el_c*: for the points
+  // (times the scale in the FP64 form)
+  const double *el_kup, *el_kdn, *el_cup, *el_cdn;
   RealTabs<double> td;
   RealTabs<float> tf;        // valid when precision is mixed
   const int* ecp_nt;         // (n_nuc)
@@ -85,6 +119,30 @@ __host__ __device__ __forceinline__ const RealTabs<double>& tabs<double>(const S
 template <>
 __host__ __device__ __forceinline__ const RealTabs<float>& tabs<float>(const Sys& s) {
   return s.tf;
+}
+
+// The same through a system in the constant address space.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) RealTabs<T>& tabs_c(
+    const __attribute__((address_space(4))) Sys& s) {
+  if constexpr (sizeof(T) == sizeof(double))
+    return s.td;
+  else
+    return s.tf;
+}
+template <typename T>
+__device__ __forceinline__ const PieceRec<T>* pieces(const __attribute__((address_space(4))) Sys& s) {
+  if constexpr (sizeof(T) == sizeof(double))
+    return s.pc64;
+  else
+    return s.pc32;
+}
+template <typename T>
+__device__ __forceinline__ const PieceMore<T>* pieces_more(const __attribute__((address_space(4))) Sys& s) {
+  if constexpr (sizeof(T) == sizeof(double))
+    return s.pm64;
+  else
+    return s.pm32;
 }
 
 // Walker state pointers (mirror of jqmc_walkers in include/jqmc_hip.h).  The AO and J3-field

@@ -1,7 +1,8 @@
-// Local energy with the points in the lanes (the default E_L kernel).
+// Local energy of single walkers by teams of waves: the FP64 guard of the mixed form (the flattened
+// launches of jqmc_elp.hip evaluate whole walker sets).
 //
-// compute_local_energy_fast (hamiltonians.py:225-290) per walker, one wavefront per walker, in
-// phases whose lanes own the items that are independent:
+// compute_local_energy_fast (hamiltonians.py:225-290) per walker, in phases whose lanes own the items
+// that are independent:
 //
 //   1. positions, G^-1 and the rotated quadrature mesh into LDS;
 //   2. q_e = [M | Lambda_u] G^-1[:, e] (up) or M' G^-1[e, :]^T (dn) for every electron (lanes own
@@ -185,16 +186,13 @@ __device__ __forceinline__ void el_load_walker(const Sys& s, const double* __res
   if (s.ecp_on && s.nv > 0) rotate_mesh(s, L.RT, L.gk, i, tm.N);
 }
 
-// Orbitals of a spin block whose C column a lane holds in registers in the determinant fields; systems
-// with more take the kWide form.
+// Orbitals of a spin block whose C column a lane holds in registers in the determinant fields.
 constexpr int EL_C_REGS = 16;
 
 // 2-3. q_e = [M | Lambda_u] G^-1[:, e] (up) or M' G^-1[e, :]^T (dn) of every electron into Qr, then the
 // determinant fields h_e = C^T q_e into the rows Hw[e][:] (FP64), every sum over the orbitals k in
-// order.  Qw: the walker's pair rows.  kWide (n_orb > EL_C_REGS): the sums of 16 electrons stay in
-// registers while the lane's AO column of C streams past 8 orbitals at a time, instead of the
-// column's orbitals beyond the first 16 being read again for every electron.
-template <int NW, bool kWide = false>
+// order.  Qw: the walker's pair rows.
+template <int NW>
 __device__ __forceinline__ void el_det_fields_rows(const Sys& s, const El2Lds& L, const double* __restrict__ Qw,
                                                    double* Qr, double* Hw, const Team<NW>& tm) {
   const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, na = s.n_ao, no = s.n_orb;
@@ -212,42 +210,6 @@ __device__ __forceinline__ void el_det_fields_rows(const Sys& s, const El2Lds& L
   }
   tm.sync();
 
-  if constexpr (kWide) {
-    constexpr int KW = 8, EC = 16;
-    for (int a = tm.tid; a < na; a += tm.N) {
-      if (!s.orb_is_mo) {
-        for (int e = 0; e < ne; ++e) Hw[(int64_t)e * na + a] = Qr[e * no + a];
-        continue;
-      }
-      for (int blk = 0; blk < 2; ++blk) {
-        const double* C = blk == 0 ? s.td.mo_up : s.td.mo_dn;
-        const int e0 = blk == 0 ? 0 : nu, e1 = blk == 0 ? nu : ne;
-        for (int eb = e0; eb < e1; eb += EC) {
-          double acc[EC];
-#pragma unroll
-          for (int i = 0; i < EC; ++i) acc[i] = 0.0;
-          for (int kb = 0; kb < no; kb += KW) {
-            double c[KW];
-#pragma unroll
-            for (int k = 0; k < KW; ++k) c[k] = kb + k < no ? C[(int64_t)(kb + k) * na + a] : 0.0;
-#pragma unroll
-            for (int i = 0; i < EC; ++i) {
-              if (eb + i >= e1) continue;
-              const double* q = Qr + (eb + i) * no + kb;
-#pragma unroll
-              for (int k = 0; k < KW; ++k)
-                if (kb + k < no) acc[i] += c[k] * q[k];
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < EC; ++i)
-            if (eb + i < e1) Hw[(int64_t)(eb + i) * na + a] = acc[i];
-        }
-      }
-    }
-    tm.sync();
-    return;
-  }
   // the lane's AO column of C held in registers for the first KC orbitals, up block with C_up, dn
   // block with C_dn
   constexpr int KC = EL_C_REGS;
@@ -279,13 +241,13 @@ __device__ __forceinline__ void el_det_fields_rows(const Sys& s, const El2Lds& L
 
 // The q rows in LDS when they fit (el2_q_in_lds), else in the workspace rows Qg; each branch keeps
 // its pointer's address space, so that the q loads compile to LDS or global instructions.
-template <int NW, bool kWide = false>
+template <int NW>
 __device__ __forceinline__ void el_det_fields(const Sys& s, const El2Lds& L, const double* __restrict__ Qw, double* Qg,
                                               double* Hw, const Team<NW>& tm) {
   if (el2_q_in_lds(s))
-    el_det_fields_rows<NW, kWide>(s, L, Qw, L.Q, Hw, tm);
+    el_det_fields_rows(s, L, Qw, L.Q, Hw, tm);
   else
-    el_det_fields_rows<NW, kWide>(s, L, Qw, Qg, Hw, tm);
+    el_det_fields_rows(s, L, Qw, Qg, Hw, tm);
 }
 
 // 4. the continuum kinetic energy T_e (wavefunction.py:1141-1207) with the lanes owning electrons:
@@ -744,71 +706,14 @@ struct ElGuard {
   double e_ref, width;
 };
 
-template <typename T, int WPB>
-__global__ void __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(3))) k_local_energy_pts(Sys s, int64_t W, WalkT<T> wk,
-                                                               const double* __restrict__ RTall, double* e_L,
-                                                               double* kin_out, double* v_out, double* t_elec,
-                                                               double* __restrict__ hws, ElGuard guard,
-                                                               int64_t lds_per_wave) {
-  extern __shared__ double smem[];
-  const int wave = wave_id(), lane = lane_id();
-  const int64_t w = (int64_t)blockIdx.x * WPB + wave;
-  if (w >= W) return;
-  El2Lds L(reinterpret_cast<char*>(smem) + wave * lds_per_wave, s);
-  const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, na = s.n_ao, no = s.n_orb;
-  double kinetic, pot;
-  el_pts_walker<T, T>(s, wk.r_up + w * 3 * nu, wk.r_dn + w * 3 * nd, wk.Ginv + w * nu * nu, wk.pair + w * ne * no,
-                      s.j3_on ? wk.jfield + w * ne * na : nullptr, RTall ? RTall + 9 * w : nullptr,
-                      hws + w * (int64_t)ne * na, hws + W * (int64_t)ne * na + w * (int64_t)ne * no, L,
-                      wave_team(lane), t_elec ? t_elec + w * ne : nullptr, kinetic, pot);
-  if (lane == 0) {
-    const double e = kinetic + pot;
-    e_L[w] = e;
-    if (kin_out) kin_out[w] = kinetic;
-    if (v_out) v_out[w] = pot;
-    if (guard.list && !(fabs(e - guard.e_ref) <= guard.width)) guard.list[atomicAdd(guard.n, 1)] = (int)w;
-  }
-}
-
-// The same local energy with a team of NW waves per walker (one walker per block): the team deals
-// the walker's shells, J2 partners and points to its waves and adds their partial sums in wave order
-// (Team<NW>), so e_L is a fixed function of NW that differs from the one-wave result in the last
-// bits.  Chosen by the JQMC_TUNE_EL_WAVES_PER_WALKER knob.
-template <typename T, int NW>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3))) k_local_energy_team(Sys s, int64_t W, WalkT<T> wk,
-    const double* __restrict__ RTall, double* e_L, double* kin_out, double* v_out, double* t_elec,
-    double* __restrict__ hws, ElGuard guard) {
-  extern __shared__ double smem[];
-  const int64_t w = blockIdx.x;
-  if (w >= W) return;  // uniform across the block
-  El2Lds L(reinterpret_cast<char*>(smem), s, NW);
-  const Team<NW> tm{(int)threadIdx.x, wave_id(), lane_id(), L.red};
-  const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, na = s.n_ao, no = s.n_orb;
-  double kinetic, pot;
-  el_pts_walker<T, T>(s, wk.r_up + w * 3 * nu, wk.r_dn + w * 3 * nd, wk.Ginv + w * nu * nu, wk.pair + w * ne * no,
-                      s.j3_on ? wk.jfield + w * ne * na : nullptr, RTall ? RTall + 9 * w : nullptr,
-                      hws + w * (int64_t)ne * na, hws + W * (int64_t)ne * na + w * (int64_t)ne * no, L,
-                      tm, t_elec ? t_elec + w * ne : nullptr, kinetic, pot);
-  if (threadIdx.x == 0) {
-    const double e = kinetic + pot;
-    e_L[w] = e;
-    if (kin_out) kin_out[w] = kinetic;
-    if (v_out) v_out[w] = pot;
-    if (guard.list && !(fabs(e - guard.e_ref) <= guard.width)) guard.list[atomicAdd(guard.n, 1)] = (int)w;
-  }
-}
-
-}  // namespace jqmc
-
-namespace jqmc {
-
 // FP64 scratch of one guard slot: AO rows, J3 fields, orbital and pair rows, the Gauss-Jordan
-// matrices M and I (I ends as G^-1) and the products U = A J3 (one row per electron).
+// matrices M and I (I ends as G^-1), the products U = A J3 and the determinant field and q rows (one
+// row per electron).
 struct GuardRec {
-  double *A, *g, *orb, *pair, *M, *I, *U;
+  double *A, *g, *orb, *pair, *M, *I, *U, *H, *Q;
   __host__ __device__ static int64_t doubles(const Sys& s) {
     const int64_t ne = s.n_el, na = s.n_ao, no = s.n_orb, nu = s.n_up;
-    return 3 * ne * na + 2 * ne * no + 2 * nu * nu;
+    return 4 * ne * na + 3 * ne * no + 2 * nu * nu;
   }
   __host__ __device__ GuardRec(double* base, const Sys& s) {
     const int64_t ne = s.n_el, na = s.n_ao, no = s.n_orb, nu = s.n_up;
@@ -819,6 +724,8 @@ struct GuardRec {
     M = pair + ne * no;
     I = M + nu * nu;
     U = I + nu * nu;
+    H = U + ne * na;
+    Q = H + ne * na;
   }
 };
 
@@ -832,7 +739,7 @@ __global__ void k_zero_int(int* p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0;
 }
 
-// The walkers listed by k_local_energy_pts<float> recomputed entirely in FP64 from their positions:
+// The walkers listed by k_el_final<float> recomputed entirely in FP64 from their positions:
 // AO values at the electrons, orbital and pair rows, G and G^-1 (wave_gauss_jordan), the J3 fields
 // (jastrow_factor.py:4121-4135) from the products A J3 and A J3^T, then el_pts_walker<double, double>;
 // e_L (and the optional parts) of those walkers are overwritten.  The GT / 64 waves of a block share
@@ -844,7 +751,6 @@ template <int GT>
 __global__ void __launch_bounds__(GT) k_local_energy_guard(Sys s, int64_t W, WalkT<float> wk,
                                                                     const double* __restrict__ RTall, double* e_L,
                                                                     double* kin_out, double* v_out, double* t_elec,
-                                                                    double* __restrict__ hws,
                                                                     const int* __restrict__ list,
                                                                     const int* __restrict__ count,
                                                                     double* __restrict__ scratch, int64_t rec_doubles) {
@@ -946,7 +852,7 @@ __global__ void __launch_bounds__(GT) k_local_energy_guard(Sys s, int64_t W, Wal
     __syncthreads();
     double kin, pot;
     el_pts_walker<double, double>(s, ru, rd, R.I, R.pair, s.j3_on ? R.g : nullptr, RTall ? RTall + 9 * w : nullptr,
-                                  hws + w * (int64_t)ne * na, hws + W * (int64_t)ne * na + w * (int64_t)ne * no, L, tm,
+                                  R.H, R.Q, L, tm,
                                   t_elec ? t_elec + w * ne : nullptr, kin, pot);
     if (t == 0) {
       e_L[w] = kin + pot;

@@ -1,11 +1,11 @@
 // gfx950 kernels of the LRDMC (lattice-regularised diffusion Monte Carlo) path.  One projection of
 // every walker is a sequence of launches:
 //
-//   k_lrdmc_ham[_team|_multi]  lattice Hamiltonian elements at the current configuration (one
-//                  wavefront, or a team of waves, per walker); also the measurement of V_diag /
-//                  V_nondiag at a given rotation
-//   k_lrdmc_move[_multi]  weight update, choice of one off-diagonal move and its rank-1 state
-//                  update, one wavefront per walker
+//   k_el_prep, k_el_kinetic, k_el_points (jqmc_elp.hip)  every element of the lattice Hamiltonian at the
+//                  current configuration: T_e, the lattice neighbours and the ECP quadrature points
+//   k_lrdmc_move[_multi]  one wavefront per walker: the diagonal and off-diagonal sums, weight update,
+//                  choice of one off-diagonal move and its rank-1 state update (k_lrdmc_measure: the sums
+//                  alone, at a given rotation)
 //   k_sweep_jfield_mfma<T, true>  J3 fields of the other electrons of every moved walker, batched
 //                  over walkers on the matrix cores (the sweep's J3 product kernel with a direct
 //                  epilogue: every field row takes its increment)
@@ -19,8 +19,7 @@
 // the weights, the Hamiltonian sums, G and G^-1 are FP64 in both forms.
 #pragma once
 
-#include "jqmc_el.hip"
-#include "jqmc_sweep_batched.hip"
+#include "jqmc_elp.hip"
 
 namespace jqmc {
 
@@ -29,75 +28,84 @@ constexpr int LR_FIXED_STEPS = 0;  // GFMC_n: n_steps projections, w <- w b_x
 constexpr int LR_FIXED_TAU = 1;    // GFMC_t: projections until tau is used, w <- w exp(-dtau e_L)
 constexpr int LR_MEASURE = 2;      // V_diag / V_nondiag at the given rotation, no move
 
-// ---- one projection in two launches: the Hamiltonian of every walker, then its move
+// Buffers of the flattened local energy in a workspace (per walker; val: ld_val doubles per walker).
+struct ElBuf {
+  double *Q, *H, *te, *jc, *jold, *vpot, *val;
+  int *elist, *necp;
+  int64_t ld_val;
+};
+// h rows are stored only for systems with more MOs than the register form takes; AO orbitals: h = q.
+__host__ __device__ inline bool el_h_rows(const Sys& s) { return s.orb_is_mo && s.el_ks == 0; }
+__host__ __device__ inline int64_t el_buf_doubles(const Sys& s, int64_t ld_val) {
+  const int64_t ne = s.n_el;
+  return ne * s.n_orb + (el_h_rows(s) ? ne * s.n_ao : 0) + 3 * ne + 1 + ld_val + (ne + 2) / 2;
+}
+inline ElBuf el_buf(const Sys& s, int64_t W, int64_t ld_val, double* p) {
+  const int64_t ne = s.n_el;
+  ElBuf B;
+  B.Q = p;
+  p += W * ne * s.n_orb;
+  B.H = el_h_rows(s) ? p : B.Q;
+  if (el_h_rows(s)) p += W * ne * s.n_ao;
+  B.te = p;
+  p += W * ne;
+  B.jc = p;
+  p += W * ne;
+  B.jold = p;
+  p += W * ne;
+  B.vpot = p;
+  p += W;
+  B.val = p;
+  p += W * ld_val;
+  B.ld_val = ld_val;
+  B.elist = reinterpret_cast<int*>(p);
+  B.necp = B.elist + W * ne;
+  return B;
+}
+// Non-local sums per walker of an E_L call: one per listed electron and 64 points.
+__host__ __device__ inline int el_parts(const Sys& s) { return s.nv > WAVE ? (s.nv + WAVE - 1) / WAVE : 1; }
 
-// Per-walker state of a projection call between its launches, in the workspace after the field
-// rows: the candidate lists, the rotation, the diagonal / off-diagonal sums, the time left, the
-// projection count, the AO change of the last move and its electron (the J3 field launch's input),
-// the candidate count and the electrons with projected ECP terms.
+// Per-walker state of a projection call between its launches, in the workspace: the local-energy
+// buffers (val: the candidate elements), the rotation, the time left, the projection count, the AO
+// change of the last move and its electron (the J3 field launch's input).
 struct LrState {
-  double* cand;    // (W, n_cmax)
+  ElBuf eb;
   double* RT;      // (W, 9)
-  double* diag;    // (W)
-  double* nondiag; // (W)
   double* tau;     // (W)
   int64_t* nproj;  // (W)
   double* dA;      // (W, n_ao) values of the cache type T (T* cast)
-  int* ncand;      // (W)
-  int* elist;      // (W, N)
   int* mv;         // (W) electron moved by the last move launch, -1 when none
   int* act;        // (2) walkers with time left after the projections it, it + 2, ... (it & 1) (GFMC_t)
-  int n_cmax;
 };
 
-// Doubles of the field rows, the q rows when they do not fit LDS and the state above, per walker.
 __host__ __device__ inline int64_t lr_cmax(const Sys& s) { return 6 * (int64_t)s.n_el + (int64_t)s.n_el * (s.nv > 0 ? s.nv : 0); }
 __host__ __device__ inline int64_t lr_ws_doubles(const Sys& s) {
-  return (int64_t)s.n_el * s.n_ao + (el2_q_in_lds(s) ? 0 : (int64_t)s.n_el * s.n_orb) + lr_cmax(s) + 9 + 4 +
-         s.n_ao + (2 + (int64_t)s.n_el + 1) / 2;
+  return el_buf_doubles(s, lr_cmax(s)) + 9 + 2 + s.n_ao + 1;
 }
 inline int64_t lr_ws_bytes(const Sys& s, int64_t W) { return W * lr_ws_doubles(s) * (int64_t)sizeof(double) + 16; }
 
 inline LrState lr_state(const Sys& s, int64_t W, double* base) {
   LrState S;
-  double* p = base + W * ((int64_t)s.n_el * s.n_ao + (el2_q_in_lds(s) ? 0 : (int64_t)s.n_el * s.n_orb));
-  S.n_cmax = (int)lr_cmax(s);
-  S.cand = p;
-  p += W * S.n_cmax;
+  S.eb = el_buf(s, W, lr_cmax(s), base);
+  double* p = base + W * el_buf_doubles(s, lr_cmax(s));
   S.RT = p;
   p += 9 * W;
-  S.diag = p;
-  p += W;
-  S.nondiag = p;
-  p += W;
   S.tau = p;
   p += W;
   S.nproj = reinterpret_cast<int64_t*>(p);
   p += W;
   S.dA = p;
   p += W * (int64_t)s.n_ao;
-  S.ncand = reinterpret_cast<int*>(p);
-  S.elist = S.ncand + W;
-  S.mv = S.elist + W * (int64_t)s.n_el;
+  S.mv = reinterpret_cast<int*>(p);
   S.act = reinterpret_cast<int*>(base + W * lr_ws_doubles(s));
   return S;
 }
 
-// LDS of one walker of the Hamiltonian launch (a team of nw waves): the local-energy block and the
-// candidate list.
+// Size limit of a system: one walker's local-energy block of the guard's team form and its candidates.
 template <typename T>
-struct LrHamLds {
-  El2Lds E;
-  double *rr, *RT, *cand;
-  uintptr_t end;
-  __host__ __device__ LrHamLds(char* base, const Sys& s, int nw = 1) : E(base, s, nw) {
-    rr = E.rr;
-    RT = E.RT;
-    Carve c{base + (E.end - reinterpret_cast<uintptr_t>(base))};
-    cand = c.take<double>(lr_cmax(s) > 0 ? lr_cmax(s) : 1);
-    end = reinterpret_cast<uintptr_t>(c.p);
-  }
-};
+inline int64_t lr_ham_lds_bytes(const Sys& s) {
+  return el2_lds_bytes(s) + 8 * (lr_cmax(s) > 0 ? lr_cmax(s) : 1);
+}
 
 // LDS of one wavefront of the move launch.
 template <typename T>
@@ -125,10 +133,6 @@ struct LrMoveLds {
 };
 
 template <typename T>
-inline int64_t lr_ham_lds_bytes(const Sys& s, int nw = 1) {
-  return (int64_t)LrHamLds<T>(0, s, nw).end;
-}
-template <typename T>
 inline int64_t lr_move_lds_bytes(const Sys& s) {
   return (int64_t)LrMoveLds<T>(0, s).end;
 }
@@ -144,92 +148,35 @@ struct LrArgs {
   double* V_nondiag;  // (W) out, may be null
   double* tau_left;   // (W) out, may be null
   int64_t* n_proj;    // (W) out, may be null
-  double* hws;        // workspace of lr_ws_bytes(s, W) bytes: field rows, then the state
-  LrState st;         // lr_state() of that workspace
+  LrState st;         // lr_state() of the caller's workspace of lr_ws_bytes(s, W) bytes
 };
 
-// Diagonal and off-diagonal sums of the lattice-regularised Hamiltonian at the current
-// configuration (_body_step_core, jqmc_gfmc.py:4807-5045; _compute_V_elements_n, 5360-5628), with the
-// phases of the local energy: determinant fields, continuum kinetic energies T_e (lanes own
-// electrons), the per-electron ECP data, then every candidate point with the lanes owning points --
-// the 6 lattice moves r_e + s_k, s = a [+x, -x, +y, -y, +z, -z] R^T (wavefunction.py:1779-1860) of
-// every electron and the nv quadrature points of the electrons whose nearest nucleus carries
-// projected ECP terms.  Leaves in L.cand the candidate list of the move choice: min(element, 0) of
-// the lattice moves of every electron (up block first), then the fixed-node ECP elements of those
-// electrons' quadrature points in electron order (L.E.elist); *n_cand is its length.  Hw / Qg: the
-// walker's field rows and workspace q rows (used when the q rows do not fit LDS).
-template <typename T, int NW, bool kWide>
-__device__ void lattice_hamiltonian(const Sys& s, const LrHamLds<T>& L, const double* Qw, double* Qg, double* Hw,
-                                    const T* gw, double alat, int dlt, const Team<NW>& tm, double& diag,
-                                    double& nondiag, int& n_cand) {
-  const int ne = s.n_el, lane = tm.lane;
-  const int n_lat = 6 * ne;
-  const bool nonlocal = s.ecp_on && s.nv > 0;
-  const double kfac = -1.0 / (2.0 * (alat * alat));
-  const El2Lds& E = L.E;
-  if (nonlocal) rotate_mesh(s, L.RT, E.gk, tm.tid, tm.N);
-  el_det_fields<NW, kWide>(s, E, Qw, Qg, Hw, tm);
-  el_kinetic<T>(s, E, Hw, gw, tm, nullptr);
-  const int n_ecp = el_ecp_electrons(s, E, tm, true);
-  tm.sync();
-  const int nv = nonlocal ? s.nv : 0;
-  const int P = n_lat + n_ecp * nv;
-  double sp_fn[2] = {0.0, 0.0};  // ECP: sum max(V, 0), sum fixed-node elements
-  for (int base = tm.wid * WAVE; base < P; base += tm.N) {
-    const int idx = base + lane;
-    const bool valid = idx < P;
-    const int id = valid ? idx : 0;
-    const bool lat = id < n_lat;
-    int e;
-    double px, py, pz, pwt = 0.0;
-    if (lat) {
-      e = id / 6;
-      const int q = id - 6 * e, axis = q >> 1;
-      const double sa = (q & 1) ? -alat : alat;
-      px = L.rr[3 * e] + sa * L.RT[3 * axis];
-      py = L.rr[3 * e + 1] + sa * L.RT[3 * axis + 1];
-      pz = L.rr[3 * e + 2] + sa * L.RT[3 * axis + 2];
-    } else {
-      const int r = id - n_lat, ie = r / nv, k = r - ie * nv;
-      e = E.elist[ie];
-      el_ecp_point(s, E, e, k, px, py, pz, pwt);
-    }
-    double det, dj;
-    el_point<T, T>(s, E, e, px, py, pz, Hw, gw, det, dj);
-    const double jr = exp(dj);
-    if (valid) {
-      if (lat) {
-        L.cand[id] = kfac * (det * jr);
-      } else {
-        // t-move: V = w_P Psi(r')/Psi(r); DLA t-move: V = w_P det ratio and the Jastrow ratio multiplies
-        // the fixed-node part only (jqmc_gfmc.py:4956-5021)
-        const double V = dlt ? pwt * det : pwt * (det * jr);
-        double fn = fmin(V, 0.0);
-        if (dlt) fn = fn * jr;
-        sp_fn[0] += fmax(V, 0.0);
-        sp_fn[1] += fn;
-        L.cand[id] = fn;
-      }
-    }
-  }
-  tm.sync();
-
-  // ---- per electron: sign-flip flag, regularised electron-ion diagonal (jqmc_gfmc.py:4833-4939)
-  const double quarter = 1.0 / (4.0 * (alat * alat));
-  double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, sp_fn[0], sp_fn[1]};  // sum opt, SP, FN, ECP local, el-el, ECP SP, ECP FN
-  for (int e = tm.tid; e < ne; e += tm.N) {
+// Diagonal and off-diagonal sums of the lattice-regularised Hamiltonian of walker w by one wavefront
+// (_body_step_core, jqmc_gfmc.py:4807-5045; _compute_V_elements_n, 5360-5628) from the elements that
+// k_el_points left in val: the six lattice moves of every electron (up block first), then the ECP
+// elements of the listed electrons' quadrature points; *n_cand is their number.  A negative element is
+// an off-diagonal (fixed-node) one, a positive one adds to the diagonal.
+template <typename T>
+__device__ void lr_reduce(const Sys& s, const WalkT<T>& wk, const LrArgs& A, int64_t w, int lane, double& diag,
+                          double& nondiag, int& n_cand) {
+  const ElBuf& B = A.st.eb;
+  const int nu = s.n_up, nd = s.n_dn, ne = s.n_el;
+  const double* cand = B.val + w * B.ld_val;
+  const double alat = A.alat, quarter = 1.0 / (4.0 * (alat * alat));
+  double acc[3] = {0.0, 0.0, 0.0};  // regularised electron-ion terms, positive and negative elements
+  for (int e = lane; e < ne; e += WAVE) {
+    // sign-flip flag, regularised electron-ion diagonal (jqmc_gfmc.py:4833-4939)
     bool flag = false;
-    double nd = 0.0;
+    double nd6 = 0.0;
     for (int k = 0; k < 6; ++k) {
-      const double x = L.cand[6 * e + k];
+      const double x = cand[6 * e + k];
       flag |= x >= 0.0;
-      nd += x + quarter;
+      nd6 += x + quarter;
       acc[1] += fmax(x, 0.0);
-      const double fn = fmin(x, 0.0);
-      acc[2] += fn;
-      L.cand[6 * e + k] = fn;
+      acc[2] += fmin(x, 0.0);
     }
-    const double ex = L.rr[3 * e], ey = L.rr[3 * e + 1], ez = L.rr[3 * e + 2];
+    const double* r = e < nu ? wk.r_up + (w * nu + e) * 3 : wk.r_dn + (w * nd + (e - nu)) * 3;
+    const double ex = r[0], ey = r[1], ez = r[2];
     double v_ei = 0.0, v_fl = 0.0;
     for (int n = 0; n < s.n_nuc; ++n) {
       const double dx = ex - s.nuc_pos[3 * n], dy = ey - s.nuc_pos[3 * n + 1], dz = ez - s.nuc_pos[3 * n + 2];
@@ -237,31 +184,18 @@ __device__ void lattice_hamiltonian(const Sys& s, const LrHamLds<T>& L, const do
       v_ei += -s.nuc_charge[n] / d;
       v_fl += -s.nuc_charge[n] / fmax(d, alat);
     }
-    const double zv = (v_ei + E.te[e]) - nd;
+    const double zv = (v_ei + B.te[w * ne + e]) - nd6;
     const double ei = s.ecp_on ? v_ei : v_fl;
     acc[0] += flag ? fmax(zv, ei) : zv;
   }
-  if (s.ecp_on) {
-    // ECP local part (coulomb_potential.py:1144-1246), lanes over electron-nucleus pairs
-    for (int t = tm.tid; t < ne * s.n_nuc; t += tm.N) {
-      const int e = t / s.n_nuc, n = t - e * s.n_nuc;
-      const double dx = L.rr[3 * e] - s.nuc_pos[3 * n], dy = L.rr[3 * e + 1] - s.nuc_pos[3 * n + 1],
-                   dz = L.rr[3 * e + 2] - s.nuc_pos[3 * n + 2];
-      acc[3] += ecp_local_pair(s, n, sqrt(dx * dx + dy * dy + dz * dz));
-    }
+  n_cand = 6 * ne + B.necp[w] * (s.nv > 0 ? s.nv : 0);
+  for (int k = 6 * ne + lane; k < n_cand; k += WAVE) {
+    acc[1] += fmax(cand[k], 0.0);
+    acc[2] += fmin(cand[k], 0.0);
   }
-  acc[4] = el_el_partial(s, L.rr, tm.tid, tm.N);
-  tm.template sum_k<7>(acc);
-  diag = 3.0 / (2.0 * (alat * alat)) * ne + ((acc[4] + s.ion_ion) + acc[0]);
+  wave_sum_k<3>(acc);
+  diag = 3.0 / (2.0 * (alat * alat)) * ne + ((B.vpot[w] + s.ion_ion) + acc[0]) + acc[1];
   nondiag = acc[2];
-  n_cand = P;
-  if (s.ecp_on) {
-    diag = ((diag + acc[3]) + acc[1]) + acc[5];
-    nondiag += acc[6];
-  } else {
-    diag += acc[1];
-  }
-  tm.sync();
 }
 
 // k = first index with cumsum(cand / psum)[k] >= u (searchsorted, jqmc_gfmc.py:5057-5062), the
@@ -270,7 +204,7 @@ __device__ int choose_candidate(const double* cand, int n, double psum, double u
   double carry = 0.0;
   for (int base = 0; base < n; base += WAVE) {
     const int p = base + lane;
-    double x = p < n ? cand[p] / psum : 0.0;
+    double x = p < n ? fmin(cand[p], 0.0) / psum : 0.0;
 #pragma unroll
     for (int off = 1; off < WAVE; off <<= 1) {
       const double y = __shfl_up(x, off, WAVE);
@@ -381,72 +315,7 @@ __device__ void lrdmc_apply_move(const Sys& s, const LDS& L, T* Aw, double* Pw, 
 }
 
 // Projection `it` of a call (GFMC_n _projection_n, jqmc_gfmc.py:4738-5358; GFMC_t _projection_t_core,
-// 724-1107), part 1, one wavefront per walker: the rotation of projection step0 + it (from the LRDMC
-// Philox stream, sub-streams 0-1, when random_mesh), then the lattice-regularised Hamiltonian; the
-// candidate list, sums and rotation go to the state for the move launch.  LR_MEASURE writes V_diag /
-// V_nondiag at the given rotations instead.  Walkers whose time is used up (GFMC_t) sit out.
-template <typename T, int NW, bool kWide>
-__device__ __forceinline__ void lr_ham_walker(const Sys& s, const WalkT<T>& wk, const LrArgs& A, int64_t W, int64_t w, int it,
-                              const LrHamLds<T>& L, const Team<NW>& tm) {
-  const int i = tm.tid;
-  const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, na = s.n_ao, no = s.n_orb;
-  const LrState& S = A.st;
-  const bool measure = A.mode == LR_MEASURE;
-  if (!measure) {
-    if (it >= A.n_steps) return;
-    if (A.mode == LR_FIXED_TAU && w == 0 && i == 0) S.act[it & 1] = 0;  // counted by this round's moves
-    if (it == 0) {
-      if (i == 0) {
-        S.tau[w] = A.tau;
-        S.nproj[w] = 0;
-      }
-    } else if (A.mode == LR_FIXED_TAU && !(S.tau[w] > 0.0)) {
-      return;
-    }
-  }
-  for (int k = i; k < 3 * nu; k += tm.N) L.rr[k] = wk.r_up[w * 3 * nu + k];
-  for (int k = i; k < 3 * nd; k += tm.N) L.rr[3 * nu + k] = wk.r_dn[w * 3 * nd + k];
-  for (int k = i; k < nu * nu; k += tm.N) L.E.Gi[k] = wk.Ginv[w * nu * nu + k];
-  if (measure) {
-    if (i < 9) L.RT[i] = A.RT ? A.RT[9 * w + i] : ((i % 4) == 0 ? 1.0 : 0.0);
-  } else if (A.random_mesh) {
-    double Rm[9];
-    rotation_RT(A.seed, (uint32_t)w, (uint64_t)(A.step0 + it), STREAM_LRDMC, Rm);
-    if (i == 0)
-      for (int k = 0; k < 9; ++k) L.RT[k] = Rm[k];
-  } else if (i < 9) {
-    L.RT[i] = (i % 4) == 0 ? 1.0 : 0.0;
-  }
-  tm.sync();
-  double* Hw = A.hws + w * (int64_t)ne * na;
-  double* Qg = A.hws + W * (int64_t)ne * na + w * (int64_t)ne * no;  // q rows when they do not fit LDS
-  const T* gw = s.j3_on ? wk.jfield + w * ne * na : nullptr;
-  double diag, nondiag;
-  int n_cand;
-  lattice_hamiltonian<T, NW, kWide>(s, L, wk.pair + w * ne * no, Qg, Hw, gw, A.alat, A.dlt, tm, diag, nondiag, n_cand);
-  if (measure) {
-    if (i == 0) {
-      A.V_diag[w] = diag;
-      A.V_nondiag[w] = nondiag;
-    }
-    return;
-  }
-  double* cw = S.cand + w * S.n_cmax;
-  for (int k = i; k < n_cand; k += tm.N) cw[k] = L.cand[k];
-  const int n_ecp = s.nv > 0 ? (n_cand - 6 * ne) / s.nv : 0;
-  for (int k = i; k < n_ecp; k += tm.N) S.elist[w * ne + k] = L.E.elist[k];
-  if (i < 9) {
-    S.RT[9 * w + i] = L.RT[i];
-    if (A.RT) A.RT[9 * w + i] = L.RT[i];
-  }
-  if (i == 0) {
-    S.diag[w] = diag;
-    S.nondiag[w] = nondiag;
-    S.ncand[w] = n_cand;
-  }
-}
-
-// Part 2: the weight update (GFMC_n: w <- w b_x; GFMC_t: dtau = min(tau_left, ln(1 - xi) / sum offdiag),
+// 724-1107) after its elements: the sums, the weight update (GFMC_n: w <- w b_x; GFMC_t: dtau = min(tau_left, ln(1 - xi) / sum offdiag),
 // w <- w exp(-dtau e_L)), the move chosen by cumulative probabilities (move and waiting-time uniforms
 // from sub-stream 2) and the single-electron update of r, caches, G and G^-1; the call's outputs of
 // the walker are rewritten after each of its projections.
@@ -459,8 +328,9 @@ __device__ void lr_move_walker(const Sys& s, const WalkT<T>& wk, const LrArgs& A
   if (it >= A.n_steps) return;
   double tau_left = S.tau[w];
   if (A.mode == LR_FIXED_TAU && !(tau_left > 0.0)) return;
-  const double diag = S.diag[w], nondiag = S.nondiag[w];
-  const int n_cand = S.ncand[w];
+  double diag, nondiag;
+  int n_cand;
+  lr_reduce<T>(s, wk, A, w, lane, diag, nondiag, n_cand);
   double wgt = A.w ? A.w[w] : 1.0;
   const U4 d2 = draw_words(A.seed, (uint32_t)w, (uint64_t)(A.step0 + it), STREAM_LRDMC, 2);
   const double u = uniform01(d2.x, d2.y);
@@ -481,7 +351,7 @@ __device__ void lr_move_walker(const Sys& s, const WalkT<T>& wk, const LrArgs& A
     move = tau_left > 0.0;
   }
   if (move) {
-    const int k = choose_candidate(S.cand + w * S.n_cmax, n_cand, nondiag, u, lane);
+    const int k = choose_candidate(S.eb.val + w * S.eb.ld_val, n_cand, nondiag, u, lane);
     for (int q = lane; q < 3 * nu; q += WAVE) L.rr[q] = wk.r_up[w * 3 * nu + q];
     for (int q = lane; q < 3 * nd; q += WAVE) L.rr[3 * nu + q] = wk.r_dn[w * 3 * nd + q];
     for (int q = lane; q < nu * nu; q += WAVE) L.Gi[q] = wk.Ginv[w * nu * nu + q];
@@ -498,7 +368,7 @@ __device__ void lr_move_walker(const Sys& s, const WalkT<T>& wk, const LrArgs& A
       nz = L.rr[3 * e + 2] + sa * L.RT[3 * axis + 2];
     } else {
       const int p = k - 6 * ne;
-      e = S.elist[w * ne + p / s.nv];
+      e = S.eb.elist[w * ne + p / s.nv] & 255;
       rotate_mesh(s, L.RT, L.gk, lane);
       const EcpElec E = ecp_electron(s, L.rr, e, L.Vt, lane);
       wave_sync();
@@ -526,36 +396,7 @@ __device__ void lr_move_walker(const Sys& s, const WalkT<T>& wk, const LrArgs& A
   }
 }
 
-// One wavefront per walker, wpb walkers per block.  kWide: the determinant fields of systems with
-// more than EL_C_REGS orbitals (lr_wide).
-template <typename T, bool kWide>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_lrdmc_ham(Sys s, int64_t W, WalkT<T> wk, LrArgs A, int it, int wpb,
-                                                   int64_t lds_per_wave) {
-  extern __shared__ double smem[];
-  const int wave = wave_id(), lane = lane_id();
-  const int64_t w = (int64_t)blockIdx.x * wpb + wave;
-  if (w >= W) return;
-  LrHamLds<T> L(reinterpret_cast<char*>(smem) + wave * lds_per_wave, s);
-  lr_ham_walker<T, 1, kWide>(s, wk, A, W, w, it, L, wave_team(lane));
-}
-
-// The Hamiltonian part with LR_TEAM waves per walker (one walker per block): for walker counts
-// that leave the one-wave launch with few waves per SIMD, the walker's shells and candidate points
-// are shared by the team.
-constexpr int LR_TEAM = 4;
-
-// Systems whose Hamiltonian launch takes the kWide determinant fields.
-inline bool lr_wide(const Sys& s) { return s.orb_is_mo && s.n_orb > EL_C_REGS; }
-template <typename T, bool kWide>
-__global__ void __launch_bounds__(LR_TEAM * 64) k_lrdmc_ham_team(Sys s, int64_t W, WalkT<T> wk, LrArgs A, int it) {
-  extern __shared__ double smem[];
-  const int64_t w = blockIdx.x;
-  if (w >= W) return;  // uniform across the block
-  LrHamLds<T> L(reinterpret_cast<char*>(smem), s, LR_TEAM);
-  const Team<LR_TEAM> tm{(int)threadIdx.x, wave_id(), lane_id(), L.E.red};
-  lr_ham_walker<T, LR_TEAM, kWide>(s, wk, A, W, w, it, L, tm);
-}
-
+// One wavefront per walker, wpb walkers per block.
 template <typename T>
 __global__ void __launch_bounds__(256) k_lrdmc_move(Sys s, int64_t W, WalkT<T> wk, LrArgs A, int it, int wpb,
                                                     int64_t lds_per_wave) {
@@ -567,18 +408,30 @@ __global__ void __launch_bounds__(256) k_lrdmc_move(Sys s, int64_t W, WalkT<T> w
   lr_move_walker<T>(s, wk, A, w, it, L, lane);
 }
 
+// V_diag and V_nondiag at the given rotations, one wavefront per walker.
+template <typename T>
+__global__ void __launch_bounds__(256) k_lrdmc_measure(Sys s, int64_t W, WalkT<T> wk, LrArgs A) {
+  const int64_t w = (int64_t)blockIdx.x * 4 + wave_id();
+  if (w >= W) return;
+  double diag, nondiag;
+  int n_cand;
+  lr_reduce<T>(s, wk, A, w, lane_id(), diag, nondiag, n_cand);
+  if (lane_id() == 0) {
+    A.V_diag[w] = diag;
+    A.V_nondiag[w] = nondiag;
+  }
+}
+
 // Several systems of uneven size in one launch: block b belongs to the system k with
-// block_start[k] <= b < block_start[k + 1] and carries one of its walkers (in the Hamiltonian launch
-// with a team of NW waves, all systems of the launch alike); every system has its own device
-// Hamiltonian, walker arrays and arguments (weights, draws, outputs, workspace).
+// block_start[k] <= b < block_start[k + 1] and carries one of its walkers; every system has its own
+// device Hamiltonian, walker arrays and arguments (weights, draws, outputs, workspace).
 struct LrSystem {
   const Sys* sys;
   int64_t W;
-  int64_t lds_ham, lds_move;
   int64_t block_start;
 };
 
-constexpr int LR_MAX_SYSTEMS = 8;
+constexpr int LR_MAX_SYSTEMS = EL_MAX_JOBS;
 
 // Launch table passed by value in the kernel arguments.
 template <typename T>
@@ -594,20 +447,6 @@ __device__ __forceinline__ int lr_multi_system(const LrMulti<T>& M, int64_t b) {
   int k = 0;
   while (k + 1 < M.n_sys && M.sys[k + 1].block_start <= b) ++k;
   return k;
-}
-
-template <typename T, int NW, bool kWide>
-__global__ void __launch_bounds__(NW * 64) k_lrdmc_ham_multi(LrMulti<T> M, int it) {
-  extern __shared__ double smem[];
-  const int64_t b = blockIdx.x;
-  const int k = lr_multi_system(M, b);
-  const LrSystem& Tk = M.sys[k];
-  const int64_t w = b - Tk.block_start;
-  if (w >= Tk.W) return;  // uniform across the block
-  const Sys& s = *Tk.sys;
-  LrHamLds<T> L(reinterpret_cast<char*>(smem), s, NW);
-  const Team<NW> tm{(int)threadIdx.x, wave_id(), lane_id(), L.E.red};
-  lr_ham_walker<T, NW, kWide>(s, M.wk[k], M.args[k], Tk.W, w, it, L, tm);
 }
 
 template <typename T>
