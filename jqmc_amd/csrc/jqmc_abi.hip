@@ -261,6 +261,17 @@ inline int64_t cache_bytes(const Sys& s) {
 
 // ---------------------------------------------------------------- launchers over T
 
+// G = j1 + S1 J3^T + S2 J3 for the W n_el rows of the prefix sums S1, S2 (k_init_jfield_mfma).
+int launch_jfield_gemm(const Sys& s, int64_t W, const double* S1, const double* S2, const double* j1, double* G,
+                       hipStream_t st) {
+  const int64_t n_rt = (W * s.n_el + JG_TILE - 1) / JG_TILE;
+  const int n_ct = (s.n_ao + JG_TILE - 1) / JG_TILE;
+  const int64_t blocks = (n_rt + 7) / 8 * 8 * n_ct;
+  if (blocks > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+  k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, W * s.n_el, S1, S2, j1, G, n_ct, n_rt);
+  return JQMC_OK;
+}
+
 template <typename T>
 int launch_init(const Sys& s, int64_t W, const jqmc_walkers* wk, void* workspace, hipStream_t st) {
   WalkT<T> k = to_walk<T>(wk);
@@ -279,11 +290,8 @@ int launch_init(const Sys& s, int64_t W, const jqmc_walkers* wk, void* workspace
     T* S2 = S1 + W * s.n_el * s.n_ao;
     k_init_jsums<T><<<grid_for(W * s.n_ao, B), B, 0, st>>>(s, W, k, S1, S2);
     if constexpr (std::is_same<T, double>::value) {
-      const int64_t n_rt = (W * s.n_el + JG_TILE - 1) / JG_TILE;
-      const int n_ct = (s.n_ao + JG_TILE - 1) / JG_TILE;
-      const int64_t blocks = (n_rt + 7) / 8 * 8 * n_ct;
-      if (blocks > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
-      k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, W * s.n_el, S1, S2, k.jfield, n_ct, n_rt);
+      const int rc = launch_jfield_gemm(s, W, S1, S2, s.td.j3v, k.jfield, st);
+      if (rc != JQMC_OK) return rc;
     } else {
       // the mixed form keeps its FP32 sums in AO order: its Markov chains are functions of their rounding
       k_init_jfield<T><<<grid_for(W * s.n_el * s.n_ao, B), B, 0, st>>>(s, W, k, S1, S2);
@@ -537,6 +545,105 @@ int launch_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* w
     }
   }
   HIP_TRY(hipGetLastError());
+  return JQMC_OK;
+}
+
+// The walkers w0 ... of a state.
+WalkT<double> walk_from(const Sys& s, WalkT<double> k, int64_t w0) {
+  const int64_t ne = s.n_el, na = s.n_ao, no = s.n_orb, nu = s.n_up;
+  k.r_up += w0 * 3 * nu;
+  if (k.r_dn) k.r_dn += w0 * 3 * s.n_dn;
+  k.ao += w0 * ne * na;
+  k.pair += w0 * ne * no;
+  if (k.jfield) k.jfield += w0 * ne * na;
+  k.Ginv += w0 * nu * nu;
+  return k;
+}
+
+int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, const double* RT, const FrOut& out,
+                  double* base, hipStream_t st) {
+  const Sys& s = sys->s;
+  const FrBuf B(s, W, base);
+  const int64_t M = W * s.n_el, tiles = W * ((s.n_up + 15) / 16 + (s.n_dn + 15) / 16);
+  const unsigned rows = (unsigned)((tiles + 3) / 4), blocks = (unsigned)((M + EL_KIN_ROWS - 1) / EL_KIN_ROWS);
+  ElJobs<double> P{};
+  P.n = 1;
+  ElJob<double>& E = P.job[0];
+  E.sys = sys->d_sys;
+  E.wk = wk;
+  E.W = W;
+  E.Q = B.q;
+  E.H = B.h;
+  E.jold = B.jold;
+  E.vpot = B.vpot;
+  E.elist = B.elist;
+  E.necp = B.necp;
+  E.q_blocks = rows;
+  k_el_prep<double><<<rows + (unsigned)((W + 3) / 4), 256, 0, st>>>(P);
+  if (s.orb_is_mo) k_el_hrows<double><<<rows, 256, 0, st>>>(E);
+  FrJob J{};
+  J.sys = sys->d_sys;
+  J.wk = wk;
+  J.W = W;
+  J.RT = RT;
+  J.Q = B.q;
+  J.H = B.h;
+  J.jold = B.jold;
+  J.vpot = B.vpot;
+  J.elist = B.elist;
+  J.necp = B.necp;
+  J.te = B.te;
+  J.jc = B.jc;
+  J.el = B.el;
+  J.wv = B.wv;
+  J.gbar = B.gbar;
+  J.qbar = B.qbar;
+  J.phib = B.phib;
+  J.t = B.t;
+  J.RA = B.RA;
+  J.RL = B.RL;
+  J.part = B.part;
+  J.re = B.re;
+  J.pt = B.pt;
+  constexpr size_t tile = EL_KIN_ROWS * EL_LD * sizeof(double);
+  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
+  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fr_orbital),
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(FR_WAVES * 3 * tile));
+  HIP_TRY(allowed);
+  k_fr_kinetic<<<blocks, FR_WAVES * WAVE, FR_WAVES * 2 * tile, st>>>(J);
+  if (s.ecp_on && s.nv > 0) {
+    const int per = std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)), groups = (4 * s.n_el + per - 1) / per;
+    const int64_t n = ((W + 3) / 4 * groups + 3) / 4;
+    if (n > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+    k_fr_points<<<(unsigned)n, 256, 0, st>>>(J, groups);
+  }
+  k_fr_adjoint<<<blocks, FR_WAVES * WAVE, FR_WAVES * 2 * tile, st>>>(J);
+  if (s.orb_is_mo) k_fr_qbar<<<rows, 256, 0, st>>>(J);
+  // the AO-value adjoints: the J3 part into the rows of gbar, C^T phibar (AO orbitals: phibar) onto it
+  J.a0 = s.j3_on ? B.gbar : (s.orb_is_mo ? B.wv : B.phib);
+  if (s.j3_on) {
+    WalkT<double> g = wk;
+    g.ao = B.gbar;
+    double* before = s.orb_is_mo ? B.wv : B.t;  // rows that are done with, or not in use yet
+    k_init_jsums<double><<<grid_for(W * s.n_ao, 256), 256, 0, st>>>(s, W, g, before, B.x);
+    const int rc = launch_jfield_gemm(s, W, before, B.x, nullptr, B.gbar, st);
+    if (rc != JQMC_OK) return rc;
+    if (!s.orb_is_mo) {
+      J.phib = B.gbar;
+      J.phib_add = 1;
+    }
+  }
+  k_fr_pairing<<<(unsigned)W, 256, 2 * sizeof(double) * s.n_up * s.n_up, st>>>(J);
+  if (s.orb_is_mo) {
+    E.Q = B.phib;
+    E.H = s.j3_on ? B.gbar : B.wv;
+    if (s.j3_on)
+      k_el_hrows<double, true><<<rows, 256, 0, st>>>(E);
+    else
+      k_el_hrows<double><<<rows, 256, 0, st>>>(E);
+  }
+  k_fr_orbital<<<blocks, FR_WAVES * WAVE, FR_WAVES * 3 * tile, st>>>(J);
+  k_fr_out<<<(unsigned)W, 256, 0, st>>>(J, out);
   return JQMC_OK;
 }
 
@@ -1246,7 +1353,7 @@ int jqmc_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk,
 int jqmc_position_grads_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes) {
   if (!sys || !bytes) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (W < 0) return fail(JQMC_ERR_SHAPE, "W < 0");
-  *bytes = W * FrWs::per_walker(sys->s) * (int64_t)sizeof(double);
+  *bytes = FrBuf(sys->s, std::min(W, FR_CHUNK), nullptr).doubles * (int64_t)sizeof(double);
   return JQMC_OK;
 }
 
@@ -1264,13 +1371,18 @@ int jqmc_position_grads(const jqmc_system* sys, int64_t W, const jqmc_walkers* w
   jqmc_position_grads_workspace_bytes(sys, W, &need);
   if (!workspace || workspace_bytes < need)
     return fail(JQMC_ERR_WORKSPACE, "workspace of %lld bytes required", (long long)need);
-  const int64_t per_wave = forces_lds_bytes(s);
-  if (per_wave > kMaxLdsPerBlock) return fail(JQMC_ERR_UNSUPPORTED, "system too large for the forces LDS budget");
-  const int wpb = walkers_per_block(per_wave);
+  if (forces_lds_bytes(s) > kMaxLdsPerBlock)
+    return fail(JQMC_ERR_UNSUPPORTED, "system too large for the forces LDS budget");
   hipStream_t st = (hipStream_t)stream;
-  k_forces<<<grid_for(W, wpb), wpb * WAVE, wpb * per_wave, st>>>(
-      s, W, to_walk<double>(wk), RT, static_cast<double*>(workspace), e_L, dE_dr, dE_dR, dlnpsi_dr, dlnpsi_dR,
-      force_HF, force_PP, swct ? 1 : 0, wpb, per_wave);
+  const int64_t ne = s.n_el, nn = s.n_nuc;
+  auto at = [](double* p, int64_t n) { return p ? p + n : nullptr; };
+  for (int64_t w0 = 0; w0 < W; w0 += FR_CHUNK) {
+    const FrOut out{at(e_L, w0), at(dE_dr, 3 * ne * w0), at(dE_dR, 3 * nn * w0), at(dlnpsi_dr, 3 * ne * w0),
+                    at(dlnpsi_dR, 3 * nn * w0), at(force_HF, 3 * nn * w0), at(force_PP, 3 * nn * w0), swct ? 1 : 0};
+    rc = launch_forces(sys, std::min(W - w0, FR_CHUNK), walk_from(s, to_walk<double>(wk), w0), RT ? RT + 9 * w0 : nullptr,
+                       out, static_cast<double*>(workspace), st);
+    if (rc != JQMC_OK) return rc;
+  }
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }

@@ -308,8 +308,8 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
 }
 
 // h rows of systems whose orbital count exceeds the register form (more than 64 MOs): H = Q C on the
-// matrix cores, wave (w, row tile).
-template <typename T>
+// matrix cores, wave (w, row tile); kAdd: onto the rows that H holds.
+template <typename T, bool kAdd = false>
 __global__ void __launch_bounds__(256) k_el_hrows(ElJob<T> J) {
   CSys& s = csys(J.sys);
   const int wave = wave_id(), lane = lane_id(), il = lane & 15, ih = lane >> 4;
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(256) k_el_hrows(ElJob<T> J) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int r = e0 + JfMfma<double>::row(q, ih);
-      if (r < n_sp && c < na) Hw[(int64_t)r * na + c] = acc[q];
+      if (r < n_sp && c < na) Hw[(int64_t)r * na + c] = kAdd ? Hw[(int64_t)r * na + c] + acc[q] : acc[q];
     }
   }
 }

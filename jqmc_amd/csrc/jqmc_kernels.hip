@@ -776,10 +776,9 @@ __global__ void __launch_bounds__(WPB * 64) k_vmc_sweep(Sys s, int64_t W, WalkT<
 
 // ============================================================ single-electron point ratios
 
-// Points evaluated together per pass of the AO loop of electron_points_ratio: the LDS radial table
-// holds up to PTS_CHUNK; the forces kernel uses EL_PTS_CHUNK (fewer live registers).
+// Points evaluated together per pass of the AO loop of electron_points_ratio (the LDS radial table holds as
+// many per shell).
 constexpr int PTS_CHUNK = 6;
-constexpr int EL_PTS_CHUNK = 4;
 
 // Determinant field of electron e into h (LDS, n_ao): q_e = [M | Lambda_u] G^-1[:, e] (up) or
 // M' G^-1[e, :]^T (dn) into q, then h_e = C^T q_e, in FP64; the single-electron determinant ratio at
@@ -819,10 +818,10 @@ __device__ inline void det_field(const Sys& s, const double* Gi, double* q, doub
 // (_compute_ratio_Jastrow_part_rank1_update, jastrow_factor.py:2696-2960).  Lanes own AOs for the
 // basis sums and own (other electron | nucleus) pairs for the J1/J2 sums; PTS_CHUNK points per
 // pass, one butterfly per chunk.  Basis sums in T, Jastrow pair sums and the results in FP64.
-template <typename T, int PC = PTS_CHUNK>
+template <typename T>
 __device__ void electron_points_ratio(const Sys& s, const double* rr, int e, const double* h, const T* Ae, const T* ge,
                                       const double* pts, int n, double* det_out, double* dj_out, T* rad, int lane) {
-  static_assert(PC <= PTS_CHUNK, "radial table holds PTS_CHUNK points per shell");
+  constexpr int PC = PTS_CHUNK;
   const int na = s.n_ao, nsh = s.n_shell;
   const RealTabs<T>& R = tabs<T>(s);
   const int n_j2 = s.j2_type ? s.n_el : 0;

@@ -400,7 +400,7 @@ struct JfMfma<float> {
 };
 
 // J3 fields of every electron of every walker from the prefix sums of k_init_jsums as one FP64 GEMM on
-// the matrix cores: rows = the M = W n_el electrons, G[m, a] = j1[a] + sum_b S1[m, b] J3T[b, a] +
+// the matrix cores: rows = the M = W n_el electrons, G[m, a] = j1[a] (NULL: 0) + sum_b S1[m, b] J3T[b, a] +
 // sum_b S2[m, b] J3[b, a] (jastrow_factor.py:4121-4135); a symmetric J3 takes one product with S1 + S2.
 // Bound by the FP64 matrix rate (4 n_ao^2 flops per electron): 64 x 64 output tiles, 16-deep slices of
 // both operands through LDS with the next slice in registers, four waves of 2 x 2 MFMA tiles each.
@@ -412,7 +412,8 @@ constexpr int JG_A_LD = JG_KC + 1;    // doubles per LDS row of S: 34 banks apar
 constexpr int JG_B_LD = JG_TILE + 8;  // the four 16-lane groups read rows 16 banks apart
 
 __global__ void __launch_bounds__(256) k_init_jfield_mfma(Sys s, int64_t M, const double* __restrict__ S1,
-                                                          const double* __restrict__ S2, double* __restrict__ G,
+                                                          const double* __restrict__ S2,
+                                                          const double* __restrict__ j1, double* __restrict__ G,
                                                           int n_ct, int64_t n_rt) {
   using MF = JfMfma<double>;
   __shared__ double a_s[JG_TILE][JG_A_LD];
@@ -479,13 +480,13 @@ __global__ void __launch_bounds__(256) k_init_jfield_mfma(Sys s, int64_t M, cons
   for (int y = 0; y < 2; ++y) {
     const int a = a0 + wc + 16 * y + il;
     if (a >= na) continue;
-    const double j1 = s.td.j3v[a];
+    const double ja = j1 ? j1[a] : 0.0;
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int64_t m = m0 + wr + 16 * x + MF::row(q, ih);
-        if (m < M) G[m * na + a] = j1 + acc[x][y][q];
+        if (m < M) G[m * na + a] = ja + acc[x][y][q];
       }
   }
 }
