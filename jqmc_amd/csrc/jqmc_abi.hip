@@ -1801,7 +1801,7 @@ int jqmc_sr_colstats(const double* O, int64_t S, int64_t P, int64_t ld, const do
                      void* stream) {
   if (!O || !wn || !mean || !var) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (S <= 0 || P <= 0 || ld < P) return fail(JQMC_ERR_SHAPE, "need S > 0, P > 0, ld >= P");
-  k_sr_colstats<<<grid_for(P, 256), 256, 0, (hipStream_t)stream>>>(O, S, P, ld, wn, mean, var);
+  k_sr_colstats<<<grid_for(P, SRC_COLS), SRC_WAVES * 64, 0, (hipStream_t)stream>>>(O, S, P, ld, wn, mean, var);
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }
@@ -1810,7 +1810,7 @@ int jqmc_sr_project(const double* O, int64_t S, int64_t P, int64_t ld, const dou
                     const double* cs, const double* x, double* out, void* stream) {
   if (!O || !mean || !rs || !cs || !x || !out) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (S <= 0 || P <= 0 || ld < P) return fail(JQMC_ERR_SHAPE, "need S > 0, P > 0, ld >= P");
-  k_sr_project<<<grid_for(P, 256), 256, 0, (hipStream_t)stream>>>(O, S, P, ld, mean, rs, cs, x, out);
+  k_sr_project<<<grid_for(P, SRC_COLS), SRC_WAVES * 64, 0, (hipStream_t)stream>>>(O, S, P, ld, mean, rs, cs, x, out);
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }
