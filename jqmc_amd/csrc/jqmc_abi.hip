@@ -1724,31 +1724,29 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
   const int ne = s.n_el, na = s.n_ao, no = s.n_orb, nu = s.n_up, nd = s.n_dn;
   double* Z = static_cast<double*>(workspace);
   T* S1 = reinterpret_cast<T*>(Z + W * nu * no);
-  T* S2 = S1 + W * ne * na;
-  constexpr int64_t kChunk = 32768;  // walkers per launch along grid z
-  if (lay.lam >= 0) {
-    k_ginv_phi<T><<<grid_for(W * nu * no, 256), 256, 0, st>>>(s, W, k, Z);
-    if (nd > 0) {
-      for (int64_t w0 = 0; w0 < W; w0 += kChunk) {
-        const int64_t nw = (W - w0) < kChunk ? (W - w0) : kChunk;
-        dim3 grid(grid_for(no, RO_TILE), grid_for(no, RO_TILE), (unsigned)nw);
-        k_rank_outer<double, double><<<grid, 256, 0, st>>>(nd, no, no, Z + w0 * nu * no, (int64_t)nu * no, no,
-                                                      k.orb + w0 * ne * no + (int64_t)nu * no, (int64_t)ne * no, no,
-                                                      O + w0 * ld, ld, no + (nu - nd), lay.lam);
-      }
+  // out (M x N per walker) = L^T R on the matrix cores
+  auto outer = [&](int K, int M, int N, auto* L, int64_t l_ld, int64_t l_rs, int64_t l_cs, auto* R, int64_t r_ld,
+                   int64_t r_rs, double* out, int64_t out_ld, int64_t out_rs, int64_t out_off) {
+    constexpr int64_t kChunk = 1 << 20;  // walkers per launch (at most 2^31 blocks)
+    const int64_t n_mt = (M + RO_ROWS - 1) / RO_ROWS;
+    for (int64_t w0 = 0; w0 < W; w0 += kChunk) {
+      const int64_t nw = std::min(W - w0, kChunk);
+      k_rank_outer<<<(unsigned)((nw + 7) / 8 * 8 * n_mt), 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs,
+                                                                       R + w0 * r_ld, r_ld, r_rs, out + w0 * out_ld,
+                                                                       out_ld, out_rs, out_off);
     }
+  };
+  if (lay.lam >= 0) {
+    outer(nu, nu, no, k.Ginv, (int64_t)nu * nu, 1, nu, k.orb, (int64_t)ne * no, no, Z, (int64_t)nu * no, no, 0);
+    if (nd > 0)
+      outer(nd, no, no, Z, (int64_t)nu * no, no, 1, k.orb + (int64_t)nu * no, (int64_t)ne * no, no, O, ld,
+            no + (nu - nd), lay.lam);
   }
   if (lay.j3 >= 0) {
-    k_init_jsums<T><<<grid_for(W * na, 256), 256, 0, st>>>(s, W, k, S1, S2);
-    for (int64_t w0 = 0; w0 < W; w0 += kChunk) {
-      const int64_t nw = (W - w0) < kChunk ? (W - w0) : kChunk;
-      dim3 grid(grid_for(na, RO_TILE), grid_for(na, RO_TILE), (unsigned)nw);
-      k_rank_outer<T, T><<<grid, 256, 0, st>>>(ne, na, na, k.ao + w0 * ne * na, (int64_t)ne * na, na,
-                                               S1 + w0 * ne * na, (int64_t)ne * na, na, O + w0 * ld, ld, na + 1,
-                                               lay.j3);
-    }
+    k_init_jsums<T><<<grid_for(W * na, 256), 256, 0, st>>>(s, W, k, S1, nullptr);
+    outer(ne, na, na, k.ao, (int64_t)ne * na, na, 1, S1, (int64_t)ne * na, na, O, ld, na + 1, lay.j3);
   }
-  k_dlnpsi_small<T><<<grid_for(W, 4), 4 * WAVE, 0, st>>>(s, W, k, Z, lay, O, ld, 4);
+  k_dlnpsi_small<T><<<(unsigned)W, 256, 0, st>>>(s, W, k, Z, lay, O, ld);
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }
@@ -1771,7 +1769,7 @@ int jqmc_param_layout(const jqmc_system* sys, int32_t blocks, int64_t* offsets, 
 int jqmc_dln_psi_dparams_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes) {
   if (!sys || !bytes) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   const Sys& s = sys->s;
-  *bytes = W * (int64_t)s.n_up * s.n_orb * (int64_t)sizeof(double) + 2 * W * (int64_t)s.n_el * s.n_ao * cache_bytes(s);
+  *bytes = W * (int64_t)s.n_up * s.n_orb * (int64_t)sizeof(double) + W * (int64_t)s.n_el * s.n_ao * cache_bytes(s);
   return JQMC_OK;
 }
 

@@ -311,21 +311,25 @@ __global__ void k_init_jsums(Sys s, int64_t W, const WalkT<T> wk, T* __restrict_
   const int64_t w = idx / s.n_ao;
   const int a = (int)(idx - w * s.n_ao);
   const int nu = s.n_up, ne = s.n_el, na = s.n_ao;
-  const T* A = wk.ao + w * ne * na;
+  const T* __restrict__ A = wk.ao + w * ne * na;
   double tot_up = 0.0, tot_dn = 0.0;
+#pragma unroll 8
   for (int e = 0; e < nu; ++e) tot_up += (double)A[e * na + a];
+#pragma unroll 8
   for (int e = nu; e < ne; ++e) tot_dn += (double)A[e * na + a];
   double before = 0.0;
+#pragma unroll 4
   for (int e = 0; e < nu; ++e) {
     const double ae = A[e * na + a];
-    S2[(w * ne + e) * na + a] = (T)before;
+    if (S2) S2[(w * ne + e) * na + a] = (T)before;
     S1[(w * ne + e) * na + a] = (T)((tot_up - before - ae) + tot_dn);
     before += ae;
   }
   before = 0.0;
+#pragma unroll 4
   for (int e = nu; e < ne; ++e) {
     const double ae = A[e * na + a];
-    S2[(w * ne + e) * na + a] = (T)(before + tot_up);
+    if (S2) S2[(w * ne + e) * na + a] = (T)(before + tot_up);
     S1[(w * ne + e) * na + a] = (T)(tot_dn - before - ae);
     before += ae;
   }
