@@ -349,7 +349,7 @@ int launch_sweep_batched(const jqmc_system* sys, int64_t W, const jqmc_walkers* 
                          double epsilon_AS, uint64_t seed, int64_t move0, const int64_t* move_ctr, void* workspace,
                          hipStream_t st) {
   const Sys& s = sys->s;
-  if (grid_for(W, JF_WALKERS) > 65535u) return fail(JQMC_ERR_SHAPE, "too many walkers for one batched sweep");
+  if (W > 65535 * (int64_t)32) return fail(JQMC_ERR_SHAPE, "too many walkers for one batched sweep");
   const int64_t per_wave = prop_lds_bytes<T>(s);
   if (per_wave > kMaxLdsPerBlock) return fail(JQMC_ERR_UNSUPPORTED, "system too large for the sweep LDS budget");
   const int wpb = tuned_wpb(per_wave, sys->tune_sweep_wpb);
@@ -360,10 +360,7 @@ int launch_sweep_batched(const jqmc_system* sys, int64_t W, const jqmc_walkers* 
   for (int m = 0; m < n_moves; ++m) {
     k_sweep_propose<T><<<grid_for(W, wpb), wpb * WAVE, lds, st>>>(sys->s, W, k, ws, m, Dt, epsilon_AS, seed,
                                                                   move0, move_ctr, wpb, per_wave);
-    if (s.j3_on) {
-      const dim3 jg(grid_for(s.n_ao, JF_ROWS), grid_for(W, JF_WALKERS));
-      k_sweep_jfield_mfma<T><<<jg, 256, 0, st>>>(sys->s, W, k, ws);
-    }
+    if (s.j3_on) launch_jfield_move<T, false>(sys->s, W, k, ws, st);
   }
   const int64_t n_flush = std::max<int64_t>(s.j3_on ? W * s.n_el * s.n_ao : 0, W);
   k_sweep_flush<T><<<grid_for(n_flush, 256), 256, 0, st>>>(W, k, ws, s.n_el, s.n_ao, s.n_up);
@@ -756,10 +753,7 @@ int launch_lrdmc(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, cons
       k_lrdmc_measure<T><<<grid_for(W, 4), 256, 0, st>>>(s, W, k, A);
     } else {
       k_lrdmc_move<T><<<grid_for(W, wpb_m), wpb_m * WAVE, wpb_m * per_move, st>>>(s, W, k, A, it, wpb_m, per_move);
-      if (s.j3_on) {
-        const dim3 jg(grid_for(s.n_ao, JF_ROWS), grid_for(W, JF_WALKERS));
-        k_sweep_jfield_mfma<T, true><<<jg, 256, 0, st>>>(s, W, k, lr_jfield_ws<T>(A.st));
-      }
+      if (s.j3_on) launch_jfield_move<T, true>(s, W, k, lr_jfield_ws<T>(A.st), st);
     }
     if (A.mode == LR_FIXED_TAU && (it % LR_POLL == LR_POLL - 1 || it == rounds - 1)) {
       HIP_TRY(hipGetLastError());
@@ -795,8 +789,7 @@ void lr_multi_jfield(const LrMulti<T>& M, const Sys* const* hsys, int it, hipStr
     const Sys& s = *hsys[slot];
     const int64_t W = M.sys[slot].W;
     if (!s.j3_on || W == 0 || it >= M.args[slot].n_steps) continue;
-    const dim3 jg(grid_for(s.n_ao, JF_ROWS), grid_for(W, JF_WALKERS));
-    k_sweep_jfield_mfma<T, true><<<jg, 256, 0, st>>>(s, W, M.wk[slot], lr_jfield_ws<T>(M.args[slot].st));
+    launch_jfield_move<T, true>(s, W, M.wk[slot], lr_jfield_ws<T>(M.args[slot].st), st);
   }
 }
 

@@ -10,10 +10,9 @@
 //                     ratios, AS factor, acceptance; on accept the walker state (position, AO /
 //                     orbital / pair rows, G, G^-1) is updated in place and dA is left in the
 //                     workspace with the moved electron's index
-//     k_sweep_jfield_mfma  [T1 | T2] = [J3 | J3^T] x dA on the matrix cores, one block per 64 AO
-//                     rows x 32 walkers (16 x 64 tiles of J3 staged in LDS, the next tile prefetched
-//                     into registers), then the J3 field increments of jastrow_factor.py:4121-4135
-//                     on those rows
+//     k_sweep_jfield_mfma  [T1 | T2] = [J3 | J3^T] x dA of the walkers that accepted on the matrix
+//                     cores, a wave per 16 of them and 16 AOs, then the J3 field increments of
+//                     jastrow_factor.py:4121-4135 on those
 //   k_sweep_flush     spin-block offsets added to every field row; R_AS stored
 //
 // The draws, proposal and acceptance are those of k_vmc_sweep (jqmc_mcmc.py:4316-4531) on the
@@ -368,13 +367,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   }
 }
 
-constexpr int JF_WALKERS = 32;  // walkers per block of k_sweep_jfield_mfma
-constexpr int JF_ROWS = 64;     // AO rows per tile
-constexpr int JF_KC = 16;       // AO columns per staged J3 tile
-// Row strides of the LDS tiles, padded so that the four 16-lane groups of a wave, which read four
-// consecutive tile rows, start 16 banks apart (64 banks of 4 bytes): 72 and 40 doubles.
-constexpr int JF_ROWS_LDS = JF_ROWS + 8;
-constexpr int JF_WALKERS_LDS = JF_WALKERS + 8;
+constexpr int JF_SEG = 64;      // walkers whose movers one block collects
+constexpr int JF_KC = 16;       // AO columns per step
+constexpr int JF_LD = 17;       // words per LDS row of the staged changes: no conflict over 16 rows
 
 // Matrix-core step of the J3 field products: D(16 x 16) += A(16 x 4) B(4 x 16) with A(i, k) from lane
 // i + 16 k and B(k, j) from lane j + 16 k; row(q, ih) is the tile row that element q of lane
@@ -491,204 +486,185 @@ __global__ void __launch_bounds__(256) k_init_jfield_mfma(Sys s, int64_t M, cons
   }
 }
 
-// [T1 | T2] = [J3 dA | J3^T dA] on AO rows a0..a0+63 (a0 = 64 blockIdx.x) for the 32 walkers
-// blockIdx.y of the block that accepted, then the field increments on those rows: an up move of
+// [T1 | T2] = [J3 dA | J3^T dA] of the walkers that accepted, then their field increments: an up move of
 // e gives t1 to up f < e and t2 to every other electron; a dn move gives t1 to every up electron
 // and to dn f < e, t2 to dn f > e.  The part shared by a spin block goes to its offset, the mover's
 // own row is compensated, and the side of the mover's block with fewer electrons takes the
 // individual correction (none for a symmetric J3).  With kDirect (the LRDMC move, whose fields are
 // read by the next Hamiltonian launch), every row f != e of a moved walker takes its increment
-// instead: t1 for f < e, t2 for f > e, no offsets.  The products run on the matrix cores as
-// D(walker, a) = sum_b dA(walker, b) J(b, a): A(i, k) = dA of walker 16 t + i at AO
-// b0 + k (LDS da_s), B(k, j) = J3^T or J3 at (b0 + k, AO a0 + 16 wave + j) (LDS jt_s / jj_s).  Wave w
-// owns the 16 AOs a0 + 16 w .. + 15 of all 32 walkers (two 16-walker tiles, T1 and T2 each), so in
-// the epilogue 16 consecutive lanes touch 16 consecutive AOs of one walker's row.
+// instead: t1 for f < e, t2 for f > e, no offsets.
+//
+// The four waves of a block share 64 walkers and 16 AOs: wave t takes the movers 16 t .. 16 t + 15 of the 64
+// (in order; a wave without any leaves at once) as the rows of D(mover, a) = sum_b dA(mover, b) J(b, a).
+// A(i, k) = dA of mover i at AO b0 + k through the wave's own LDS tile, B(k, j) = J3^T or J3 at (b0 + k, AO
+// a0 + j) straight from L2, both with the next sixteen b on their way during the current ones: no barrier, so
+// that the products of some waves overlap the row updates of others, and many small blocks, so that small
+// walker counts fill the chip.  The sums run over b in order in fours.  The AO tiles of a segment are eight
+// blocks apart (one XCD): the lines that two tiles share meet in its L2.
+// Bound by the row updates at large walker counts (104 bytes per AO and accepted move of benzene, 340 MB of
+// 16384 walkers, at scattered rows) and by latency at small ones.  Blocks of 32 walkers x 64 AOs with barriers
+// took 32.7 us for 1024 benzene walkers, 175 us for 16384, 38.5 us for 2048 of 4 x H2O in FP32 and 9.3 us for
+// 256 of H2O; this 20.8, 173, 27.7 and 7.7 us.  Two AO tiles a wave: 31.4, 174 and 36.0 us, 32 movers a wave
+// 171 us for 16384.
 template <typename T, bool kDirect = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_sweep_jfield_mfma(Sys s, int64_t W, WalkT<T> wk, SweepWs<T> ws) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_sweep_jfield_mfma(Sys s, int64_t W,
+                                                                                                   WalkT<T> wk,
+                                                                                                   SweepWs<T> ws) {
   using M = JfMfma<T>;
   typedef typename M::v4 v4;
-  const RealTabs<T>& R = tabs<T>(s);
-  __shared__ __align__(16) T jt_s[JF_KC][JF_ROWS_LDS];
-  __shared__ __align__(16) T jj_s[JF_KC][JF_ROWS_LDS];
-  __shared__ __align__(16) T da_s[JF_KC][JF_WALKERS_LDS];
-  __shared__ int mv_s[JF_WALKERS];
-  __shared__ int any_s;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int a0 = (int)blockIdx.x * JF_ROWS;
-  const int64_t w0 = (int64_t)blockIdx.y * JF_WALKERS;
+  __shared__ T da_sh[4][2][JF_KC * JF_LD];
+  __shared__ int mv_sh[4][JF_SEG], at_sh[4][JF_SEG];
+  const int lane = threadIdx.x & 63, wave = wave_id(), il = lane & 15, ih = lane >> 4;
   const int nu = s.n_up, ne = s.n_el, na = s.n_ao;
-  if (t == 0) any_s = 0;
-  __syncthreads();
-  if (t < JF_WALKERS) {
-    const int64_t w = w0 + t;
-    const int e = w < W ? ws.mv[w] : -1;
-    mv_s[t] = e;
-    if (e >= 0) atomicOr(&any_s, 1);
-  }
-  __syncthreads();
-  if (!any_s) return;  // uniform across the block
-  const bool sym = s.j3_sym != 0;
-  const T* __restrict__ JT = R.j3T;
-  const T* __restrict__ JJ = R.j3;
-  const T* __restrict__ DA = ws.dA;
-  T pjt[4], pjj[4], pda[2];
-  auto fetch = [&](int b0) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = t + 256 * r;
-      const int bb = k / JF_ROWS, aa = k - bb * JF_ROWS;
-      const int b = b0 + bb, a = a0 + aa;
-      const bool ok = b < na && a < na;
-      pjt[r] = ok ? JT[(int64_t)b * na + a] : (T)0;
-      pjj[r] = (ok && !sym) ? JJ[(int64_t)b * na + a] : (T)0;
+  const int n_ct = (na + 15) / 16;
+  const int64_t blk = blockIdx.x, w0 = (blk / (8 * n_ct) * 8 + blk % 8) * JF_SEG;
+  const int a0 = (int)((blk / 8) % n_ct) * 16;
+  if (w0 >= W) return;
+  const int e_l = w0 + lane < W ? ws.mv[w0 + lane] : -1;
+  const uint64_t movers = __ballot(e_l >= 0);
+  const int n = __popcll(movers) - 16 * wave;  // movers of this wave and the later ones
+  if (n <= 0) return;
+  int* mv_s = mv_sh[wave];
+  int* at_s = at_sh[wave];
+  if (e_l >= 0) {
+    const int r = __popcll(movers & ((1ull << lane) - 1ull)) - 16 * wave;
+    if (r >= 0) {
+      mv_s[r] = e_l;
+      at_s[r] = lane;
     }
+  }
+  wave_sync();
+  const T* __restrict__ JT = tabs<T>(s).j3T;
+  const T* __restrict__ JJ = tabs<T>(s).j3;
+  // staged change: columns (lane & 3) + 4 r of mover lane / 4 (past the last mover: zeros)
+  const int sr = lane >> 2, sk = lane & 3;
+  const bool s_on = sr < n;
+  const T* __restrict__ DA = ws.dA + (w0 + at_s[s_on ? sr : 0]) * na;
+  const int a = a0 + il < na ? a0 + il : na - 1;  // columns past the end are not used
+  T pa[4], pt[4], pj[4], ct[4], cj[4];
+  auto fetch = [&](int b0) {  // without branches: AOs past the end repeat the last one
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int k = t + 256 * r;
-      const int ww = k / JF_KC, bb = k - ww * JF_KC;
-      const int b = b0 + bb;
-      pda[r] = (mv_s[ww] >= 0 && b < na) ? DA[(w0 + ww) * na + b] : (T)0;
+    for (int q = 0; q < 4; ++q) {
+      const int ba = b0 + sk + 4 * q < na ? b0 + sk + 4 * q : na - 1;
+      const int b = b0 + 4 * q + ih < na ? b0 + 4 * q + ih : na - 1;
+      pa[q] = DA[ba];
+      pt[q] = JT[(int64_t)b * na + a];
+      pj[q] = JJ[(int64_t)b * na + a];
     }
   };
-  v4 acc1[2], acc2[2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x) acc1[x] = acc2[x] = v4{0, 0, 0, 0};
-  const int il = lane & 15, ih = lane >> 4;
+  v4 acc1 = {0, 0, 0, 0}, acc2 = {0, 0, 0, 0};
   fetch(0);
-  for (int b0 = 0; b0 < na; b0 += JF_KC) {
+  for (int b0 = 0, st = 0; b0 < na; b0 += JF_KC, st ^= 1) {
+    T* da = da_sh[wave][st];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = t + 256 * r;
-      const int bb = k / JF_ROWS, aa = k - bb * JF_ROWS;
-      jt_s[bb][aa] = pjt[r];
-      jj_s[bb][aa] = pjj[r];
+    for (int q = 0; q < 4; ++q) {
+      da[(sk + 4 * q) * JF_LD + sr] = s_on && b0 + sk + 4 * q < na ? pa[q] : (T)0;  // zero against repeated rows of J
+      ct[q] = pt[q];
+      cj[q] = pj[q];
     }
+    if (b0 + JF_KC < na) fetch(b0 + JF_KC);
+    asm volatile("" ::: "memory");  // one wave's LDS accesses are taken in order
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int k = t + 256 * r;
-      const int ww = k / JF_KC, bb = k - ww * JF_KC;
-      da_s[bb][ww] = pda[r];
+    for (int q = 0; q < 4; ++q) {
+      const T fa = da[(4 * q + ih) * JF_LD + il];
+      acc1 = M::mma(fa, ct[q], acc1);
+      acc2 = M::mma(fa, cj[q], acc2);
     }
-    __syncthreads();
-    if (b0 + JF_KC < na) fetch(b0 + JF_KC);  // next stage in flight during this one
-#pragma unroll
-    for (int kk = 0; kk < JF_KC; kk += 4) {
-      const int kl = kk + ih;
-      const T fj = jt_s[kl][16 * wave + il];
-      const T fjj = sym ? fj : jj_s[kl][16 * wave + il];
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const T fa = da_s[kl][16 * x + il];
-        acc1[x] = M::mma(fa, fj, acc1[x]);
-        acc2[x] = M::mma(fa, fjj, acc2[x]);
-      }
-    }
-    __syncthreads();
   }
-  // epilogue: pair (x, q) of this lane is walker 16 x + row(q, ih) of the block and AO a0 + 16 wave + il
-  const int a = a0 + 16 * wave + il;
-  const bool aok = a < na;
+  if (a0 + il >= na) return;  // no cross-lane work follows
+  // epilogue: element q of this lane is mover row(q, ih) of the wave
+  int ee[4];
+  int64_t ww[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = M::row(q, ih);
+    ee[q] = r < n ? mv_s[r] : -1;
+    ww[q] = w0 + at_s[r < n ? r : 0];
+  }
   if constexpr (kDirect) {
-    if (!aok) return;  // no barrier follows
-    int ee[8];
-    T t1[8], t2[8];
-    T* col[8];
+    // four rows of the four walkers per pass, all 16 loads in flight together
+    for (int f0 = 0; f0 < ne; f0 += 4) {
+      T v[4][4];
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      const int x = p >> 2, q = p & 3, r = 16 * x + M::row(q, ih);
-      ee[p] = mv_s[r];
-      t1[p] = acc1[x][q];
-      t2[p] = acc2[x][q];
-      col[p] = ee[p] >= 0 ? wk.jfield + (w0 + r) * ne * na + a : wk.jfield;
-    }
-    // two rows of the 8 walkers per pass, all 16 loads in flight together
-    for (int f0 = 0; f0 < ne; f0 += 2) {
-      T v[2][8];
+      for (int h = 0; h < 4; ++h)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int p = 0; p < 8; ++p) {
+        for (int q = 0; q < 4; ++q) {
           const int f = f0 + h;
-          v[h][p] = (f < ne && ee[p] >= 0 && f != ee[p]) ? col[p][(int64_t)f * na] : (T)0;
+          v[h][q] = (f < ne && ee[q] >= 0 && f != ee[q]) ? wk.jfield[(ww[q] * ne + f) * na + a] : (T)0;
         }
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 4; ++h)
 #pragma unroll
-        for (int p = 0; p < 8; ++p) {
+        for (int q = 0; q < 4; ++q) {
           const int f = f0 + h;
-          if (f < ne && ee[p] >= 0 && f != ee[p]) col[p][(int64_t)f * na] = v[h][p] + (f < ee[p] ? t1[p] : t2[p]);
+          if (f < ne && ee[q] >= 0 && f != ee[q])
+            wk.jfield[(ww[q] * ne + f) * na + a] = v[h][q] + (f < ee[q] ? acc1[q] : acc2[q]);
         }
     }
     return;
   }
-  int ee[8], cs[8], cn[8];
-  bool upm[8], lw[8];
-  T d8[8], t1[8], t2[8];
+  const bool sym = s.j3_sym != 0;
+  int cs[4], cn[4];
+  bool upm[4], lw[4];
+  T d4[4];
 #pragma unroll
-  for (int p = 0; p < 8; ++p) {
-    const int x = p >> 2, q = p & 3;
-    const int e = mv_s[16 * x + M::row(q, ih)];
-    ee[p] = e;
-    upm[p] = e < nu;
-    const int f0 = upm[p] ? 0 : nu, f1 = upm[p] ? nu : ne;
-    lw[p] = sym || (e - f0) <= (f1 - 1 - e);
-    cs[p] = 0;
-    cn[p] = 0;
+  for (int q = 0; q < 4; ++q) {
+    const int e = ee[q];
+    upm[q] = e < nu;
+    const int f0 = upm[q] ? 0 : nu, f1 = upm[q] ? nu : ne;
+    lw[q] = sym || (e - f0) <= (f1 - 1 - e);
+    cs[q] = 0;
+    cn[q] = 0;
     if (e >= 0 && !sym) {
-      cs[p] = lw[p] ? f0 : e + 1;
-      cn[p] = (lw[p] ? e : f1) - cs[p];
+      cs[q] = lw[q] ? f0 : e + 1;
+      cn[q] = (lw[q] ? e : f1) - cs[q];
     }
-    t1[p] = acc1[x][q];
-    t2[p] = acc2[x][q];
-    d8[p] = lw[p] ? t1[p] - t2[p] : t2[p] - t1[p];
+    d4[q] = lw[q] ? acc1[q] - acc2[q] : acc2[q] - acc1[q];
   }
   {
-    T go[8], ou[8], od[8];
+    T go[4], ou[4], od[4];
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      const int64_t w = w0 + 16 * (p >> 2) + M::row(p & 3, ih);
-      const bool on = ee[p] >= 0 && aok;
-      const int64_t row = w * ne * na + (int64_t)(ee[p] > 0 ? ee[p] : 0) * na;
-      go[p] = on ? wk.jfield[row + a] : (T)0;
-      ou[p] = on ? ws.Oup[w * na + a] : (T)0;
-      od[p] = on ? ws.Odn[w * na + a] : (T)0;
+    for (int q = 0; q < 4; ++q) {
+      const bool on = ee[q] >= 0;
+      go[q] = on ? wk.jfield[(ww[q] * ne + ee[q]) * na + a] : (T)0;
+      ou[q] = on ? ws.Oup[ww[q] * na + a] : (T)0;
+      od[q] = on ? ws.Odn[ww[q] * na + a] : (T)0;
     }
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      if (ee[p] < 0 || !aok) continue;
-      const int64_t w = w0 + 16 * (p >> 2) + M::row(p & 3, ih);
-      const int64_t row = w * ne * na + (int64_t)ee[p] * na;
-      const T own = lw[p] ? t2[p] : t1[p];
-      wk.jfield[row + a] = go[p] - own;
-      ws.Oup[w * na + a] = ou[p] + (upm[p] ? own : t1[p]);
-      ws.Odn[w * na + a] = od[p] + (upm[p] ? t2[p] : own);
+    for (int q = 0; q < 4; ++q) {
+      if (ee[q] < 0) continue;
+      const T own = lw[q] ? acc2[q] : acc1[q];
+      wk.jfield[(ww[q] * ne + ee[q]) * na + a] = go[q] - own;
+      ws.Oup[ww[q] * na + a] = ou[q] + (upm[q] ? own : acc1[q]);
+      ws.Odn[ww[q] * na + a] = od[q] + (upm[q] ? acc2[q] : own);
     }
   }
-  // individual corrections: rows cs .. cs + cn - 1 of each walker get d, two rows per pass with
-  // all their loads in flight together
+  // individual corrections: rows cs .. cs + cn - 1 of each walker get d, four rows per pass with all their
+  // loads in flight together
   int nmax = 0;
 #pragma unroll
-  for (int p = 0; p < 8; ++p) nmax = cn[p] > nmax ? cn[p] : nmax;
-  for (int r = 0; r < nmax; r += 2) {
-    T v[2][8];
+  for (int q = 0; q < 4; ++q) nmax = cn[q] > nmax ? cn[q] : nmax;
+  for (int r = 0; r < nmax; r += 4) {
+    T v[4][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 4; ++h)
 #pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        const bool on = r + h < cn[p] && aok;
-        const int64_t w = w0 + 16 * (p >> 2) + M::row(p & 3, ih);
-        v[h][p] = on ? wk.jfield[w * ne * na + (int64_t)(cs[p] + r + h) * na + a] : (T)0;
-      }
+      for (int q = 0; q < 4; ++q)
+        v[h][q] = r + h < cn[q] ? wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a] : (T)0;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 4; ++h)
 #pragma unroll
-      for (int p = 0; p < 8; ++p) {
-        if (r + h < cn[p] && aok) {
-          const int64_t w = w0 + 16 * (p >> 2) + M::row(p & 3, ih);
-          wk.jfield[w * ne * na + (int64_t)(cs[p] + r + h) * na + a] = v[h][p] + d8[p];
-        }
-      }
+      for (int q = 0; q < 4; ++q)
+        if (r + h < cn[q]) wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a] = v[h][q] + d4[q];
   }
+}
+
+// The J3 field update of one move.
+template <typename T, bool kDirect>
+inline void launch_jfield_move(const Sys& s, int64_t W, const WalkT<T>& wk, const SweepWs<T>& ws, hipStream_t st) {
+  const int64_t segs = (W + JF_SEG - 1) / JF_SEG, n_ct = (s.n_ao + 15) / 16;
+  k_sweep_jfield_mfma<T, kDirect><<<(unsigned)((segs + 7) / 8 * 8 * n_ct), 256, 0, st>>>(s, W, wk, ws);
 }
 
 // Offsets into every field row and the AS factor into the walker state (one thread per element).
