@@ -442,6 +442,39 @@ __device__ __forceinline__ void shell_values(const Sys& s, int sh, double x, dou
   for (int a = a0; a < a1; ++a) out[a] = R.ao_scale[a] * nr * ao_poly_meta<T>(s, a, s.ao_meta[a], dx, dy, dz);
 }
 
+// The same from the shell's record, bit for bit: one level of loads instead of three that depend on each other,
+// the chains of the exponentials together (primitives past the last have coefficient 0).
+__device__ __forceinline__ void shell_record_values(const Sys& s, int sh, double x, double y, double z, double* out) {
+  const double* r = s.shrec + (int64_t)sh * SHREC;
+  const int info = (int)r[3];
+  if (!(info & (1 << 8))) {
+    shell_values<double>(s, sh, x, y, z, out);
+    return;
+  }
+  const double dx = x - r[0], dy = y - r[1], dz = z - r[2];
+  const double r2 = fmin(dx * dx + dy * dy + dz * dz, 1.0e300);  // finite against a padded exponent of zero
+  double nr = 0;
+#pragma unroll
+  for (int q = 0; q < SHR_PMAX; ++q) nr += r[SHR_P + 2 * q + 1] * exp_nonpos(-r[SHR_P + 2 * q] * r2);
+  const int l = (info >> 4) & 15;
+  const double* sc = r + SHR_SC;
+  double* v = out + (info >> 9);
+  if (l == 0) {
+    v[0] = sc[0] * nr;
+  } else if (l == 1) {
+    v[0] = sc[0] * nr * dx;
+    v[1] = sc[1] * nr * dy;
+    v[2] = sc[2] * nr * dz;
+  } else {
+    v[0] = sc[0] * nr * (dx * dx);
+    v[1] = sc[1] * nr * (dx * dy);
+    v[2] = sc[2] * nr * (dx * dz);
+    v[3] = sc[3] * nr * (dy * dy);
+    v[4] = sc[4] * nr * (dy * dz);
+    v[5] = sc[5] * nr * (dz * dz);
+  }
+}
+
 // Value, gradient and Laplacian of every AO of shell sh at (x, y, z) into v, g (3 per AO) and l:
 // the radial moments NR, ZNR, Z^2NR once per shell, the polynomial algebra of ao_vgl per AO.
 template <typename T>

@@ -48,7 +48,7 @@ __device__ inline void wave_matvec_T(const TC* __restrict__ CT, const TX* x, int
     const int kk = kb + k;
     TY acc = 0;
     if (kk < no) {
-#pragma unroll 4
+#pragma unroll 8
       for (int a = grp; a < na; a += G) acc += (TY)CT[(int64_t)a * no + kk] * (TY)x[a];
     }
     for (int off = lg; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off, WAVE);
@@ -419,6 +419,20 @@ inline int64_t sweep_lds_bytes(const Sys& s) {
 
 __device__ __forceinline__ double step_factor(double Z, double d) { return 1.0 / (Z * Z) * (1.0 + Z * Z * d) / (1.0 + d); }
 
+// nearest_nucleus by one wavefront, a nucleus per lane: the smallest distance, the first of equal ones (and the
+// first nucleus if no distance is a number).
+__device__ __forceinline__ int nearest_nucleus_wave(const Sys& s, double x, double y, double z, int lane) {
+  if (s.n_nuc > WAVE) return nearest_nucleus(s, x, y, z);
+  double d = __builtin_inf();
+  if (lane < s.n_nuc) {
+    const double dx = s.nuc_pos[3 * lane] - x, dy = s.nuc_pos[3 * lane + 1] - y, dz = s.nuc_pos[3 * lane + 2] - z;
+    d = sqrt(dx * dx + dy * dy + dz * dz);
+  }
+  const double m = wave_min(d);
+  const uint64_t at = __ballot(lane < s.n_nuc && d == m);
+  return at ? __ffsll((unsigned long long)at) - 1 : 0;
+}
+
 // Attaccalite-Sorella factor of (G, G^-1) after a candidate rank-1 change held in LDS:
 // mode 0 = current matrices, 1 = row idx += vv (up move), 2 = column idx += vv (dn move);
 // the candidate inverse is G^-1 - xx yy^T / ratio (determinant.py:1223-1260).
@@ -435,6 +449,7 @@ __device__ inline double sweep_as_factor(const LdsT& L, int nu, int lane, int mo
   double smin = 1.0e300;
   for (int p = lane; p < nu; p += WAVE) {
     double rs = 0.0, cs = 0.0;
+#pragma unroll 8
     for (int q = 0; q < nu; ++q) {
       double gr = L.Gm[p * nu + q], gc = L.Gm[q * nu + p];
       if (mode == 1) {
