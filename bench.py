@@ -77,15 +77,6 @@ def kernel_work(pack, W, n_moves, accepted, n_ecp_el=None):
     return sweep, el
 
 
-# HBM bytes per dispatch measured with rocprofv3 FETCH_SIZE / WRITE_SIZE (each scaled by what the
-# counter reads for a plain 1 GiB device copy: x2.00 and x1.00) for the default configuration.
-MEASURED_TRAFFIC = {
-    ("benzene_ecp", 16384, "sweep"): (24.2e9, "profiles/vmc_step_benzene_ecp_w16384_fp64.md"),
-    ("benzene_ecp", 16384, "k_local_energy_pts"): (4.70e9, "profiles/vmc_step_benzene_ecp_w16384_fp64.md"),
-    ("benzene_ecp", 16384, "k_local_energy_team<double, 2>"): (4.46e9, "profiles/vmc_step_benzene_ecp_w16384_fp64.md"),
-}
-
-
 def cpu_model() -> str:
     try:
         with open("/proc/cpuinfo") as f:
@@ -549,8 +540,7 @@ def main(argv=None):
     tuning = None
     if not args.no_autotune:
         # launch shapes for this system and walker count (set-up, outside the timed region; the
-        # walkers-per-block knobs change no result bit, a team of waves per walker changes e_L in
-        # the last bits)
+        # knobs change no result bit)
         from jqmc_amd.autotune import autotune
 
         tuning = autotune(ws, n_moves=n_moves)
@@ -617,23 +607,18 @@ def main(argv=None):
 
     n_ecp_el = ecp_electrons(pack, ws.r_up.cpu().numpy(), ws.r_dn.cpu().numpy())
     sweep_w, el_w = kernel_work(pack, W, n_moves, accepted, n_ecp_el)
-    # the roofline kernel: the single kernel with the largest time per step, the local energy
-    # (k_local_energy_pts, or k_local_energy_team when the autotuner picked a team of waves per
-    # walker; one launch per step; the sweep is 62 launches of four kernels)
-    team = tuning["best"].get("el_waves_per_walker", 1) if tuning and "best" in tuning else 1
-    name = f"k_local_energy_team<double, {team}>" if team > 1 else "k_local_energy_pts"
+    # the roofline row: the local energy, four launches per step, most of it in k_el_points (the sweep is
+    # 62 launches of four kernels)
+    name = "local energy (k_el_prep, k_el_kinetic, k_el_points, k_el_final)"
     ms, work = el_ms, el_w
     intensity = work["flops"] / work["bytes"]
-    traffic = MEASURED_TRAFFIC.get((args.workload, W, name))
     achieved = work["flops"] / (ms / 1e3) / 1e12
     roof = {"kernel": name, "bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS,
-            "note": "FP64 vector ALU kernel (no matrix instruction) far above the machine balance "
+            "note": "FP64 vector ALU kernels (the determinant fields on the matrix cores) far above the machine balance "
                     f"({intensity:.0f} flop/B of compulsory traffic); peak = MI355X FP64 vector 78.6 TFLOP/s; "
                     "exp/sqrt/div count one op each"}
-    roof["traffic"] = traffic[0] if traffic else None
-    if traffic:
-        roof["traffic_source"] = traffic[1]
+    roof["traffic"] = None
     roof["avg_ms"] = ms
     roof["algorithmic"] = {"flops": work["flops"], "bytes": work["bytes"], "flop_per_byte": intensity,
                            "flops_per_walker": work["flops"] / W,
@@ -643,11 +628,6 @@ def main(argv=None):
                             "avg_ms": sweep_ms, "TFLOP_per_s": sweep_w["flops"] / (sweep_ms / 1e3) / 1e12,
                             "GB_per_s": sweep_w["bytes"] / (sweep_ms / 1e3) / 1e9,
                             "note": "J3 field products on the FP64 matrix cores, proposals on the vector ALUs"}
-    sweep_traffic = MEASURED_TRAFFIC.get((args.workload, W, "sweep"))
-    if sweep_traffic:
-        roof["other_kernel"]["traffic"] = sweep_traffic[0]
-        roof["other_kernel"]["traffic_source"] = sweep_traffic[1]
-
     extra = {}
     if not args.no_extras:
         extra = extras(system, ham, args, W, n_moves, e_steps)

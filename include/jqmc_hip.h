@@ -151,12 +151,11 @@ int jqmc_system_destroy(jqmc_system* sys);
 
 /*
  * Launch-shape knobs of a system, set by the autotuner (jqmc_amd/autotune.py) or by hand; value 0
- * restores the library's default.  The walkers-per-block knobs change no result bit: they choose how
- * many walkers share a block in the E_L kernel and the move-synchronous proposal kernel (1, 2 or 4,
- * capped by the LDS budget).  JQMC_TUNE_EL_WAVES_PER_WALKER (1, 2 or 4; one walker per block when
- * above 1 and its LDS fits) gives the E_L kernel a team of waves per walker, whose partial sums are
- * added in wave order: e_L then differs from the one-wave result in the last bits, as a fixed
- * function of the value.  No counterpart in the reference (XLA picks its own launch shapes).
+ * restores the library's default.  The walkers-per-block knob of the move-synchronous proposal kernel
+ * (1, 2 or 4, capped by the LDS budget) changes no result bit.  The two knobs of the E_L kernel (walkers
+ * per block 1, 2 or 4; waves per walker 1, 2 or 4) are taken and returned as before and no longer change
+ * anything: the local energy runs over electrons and points of all walkers, not over walkers.  No
+ * counterpart in the reference (XLA picks its own launch shapes).
  */
 #define JQMC_TUNE_EL_WALKERS_PER_BLOCK 2
 #define JQMC_TUNE_SWEEP_WALKERS_PER_BLOCK 3
@@ -256,10 +255,9 @@ int jqmc_rotation_matrices(int64_t W, uint64_t seed, int64_t step, int32_t strea
  * wavefunction.py:1141-1207) + bare Coulomb (coulomb_potential.py:2252-2281) + ECP local
  * (1144-1246) + ECP non-local with NN=1 and the rotated nv-point mesh (1477-1712).
  * Outputs (W): e_L, kinetic, v_total (may be NULL); t_elec (W, N) per-electron kinetic
- * (may be NULL).  workspace: jqmc_local_energy_workspace_bytes() bytes (the FP64 determinant
- * field rows h_e of every electron, W x N x n_ao doubles, the W x N x n_orb q_e rows when
- * N x n_orb doubles exceed 16 KiB, and in the mixed form the list and FP64 scratch of the guard,
- * jqmc_system_set_mixed_guard).
+ * (may be NULL).  workspace: jqmc_local_energy_workspace_bytes() bytes (the W x N x n_orb q_e rows, with
+ * more than 64 MOs also the h_e rows W x N x n_ao, a few doubles per electron, and in the mixed form the
+ * list and FP64 scratch of the guard, jqmc_system_set_mixed_guard).
  */
 int jqmc_local_energy_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes);
 int jqmc_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const double* RT, double* e_L,

@@ -1,11 +1,11 @@
 """Launch-shape autotuner for a system on this GPU.
 
-The walkers per block of the E_L and move-synchronous proposal kernels, and the waves per walker of
-the E_L kernel, are chosen per system by timing every candidate on the caller's walker count, on
-scratch walkers built at the caller's positions, so the caller's chain does not move.  The
-walkers-per-block knobs (jqmc_system_set_tuning) change no result bit; a team of two waves per walker
-changes e_L in the last bits, as a fixed function of the choice (tests/test_gpu_autotune.py checks
-both).  The reference has no counterpart (XLA picks its own launch shapes).
+The walkers per block of the move-synchronous proposal kernel are chosen per system by timing every
+candidate on the caller's walker count, on scratch walkers built at the caller's positions, so the
+caller's chain does not move.  The two knobs of the E_L kernel are timed and set along with it; the
+local energy runs over the electrons and points of all walkers and does not depend on them.  No knob
+(jqmc_system_set_tuning) changes a result bit (tests/test_gpu_autotune.py checks).  The reference
+has no counterpart (XLA picks its own launch shapes).
 """
 
 from __future__ import annotations

@@ -84,7 +84,6 @@ struct Team {
 };
 
 // The one-wavefront team of lane `lane`.
-__device__ __forceinline__ Team<1> wave_team(int lane) { return Team<1>{lane, 0, lane, nullptr}; }
 
 // The q_e rows of all electrons stay in LDS when they take at most EL2_Q_LDS bytes, otherwise they
 // go to the workspace after the h_e rows (large AO-orbital geminals).
@@ -93,7 +92,7 @@ __host__ __device__ inline bool el2_q_in_lds(const Sys& s) {
   return (int64_t)s.n_el * s.n_orb * (int64_t)sizeof(double) <= EL2_Q_LDS;
 }
 
-// LDS of one walker of k_local_energy_pts (one wavefront; nw > 1: a team of nw wavefronts, which
+// LDS of one walker of the guard's local energy (one wavefront; nw > 1: a team of nw wavefronts, which
 // also needs the reduction words red and the per-wave kinetic partials kred).
 struct El2Lds {
   double *rr, *Gi, *RT, *gk, *Q, *en, *Vt, *jold, *te, *jc, *red, *kred;
