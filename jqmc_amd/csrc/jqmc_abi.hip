@@ -428,7 +428,8 @@ ElJob<T> el_job(const Sys* d_sys, const Sys& s, int64_t W, const WalkT<T>& wk, c
   return J;
 }
 
-// Waves of a k_el_kinetic block: four, or two where four would not leave room for two blocks per CU.
+// Waves of a k_el_kinetic block: four, or two where four would not leave room for two blocks per CU (with the
+// limit at 64 KiB the 56-electron chain took 360 us, with 80 KiB 252; the uneven LRDMC batch 622 and 323 us).
 constexpr int64_t kMaxKineticLds = 80 * 1024;
 template <typename T>
 int el_kin_waves(const Sys& s) {
