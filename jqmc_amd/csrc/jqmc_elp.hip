@@ -60,9 +60,20 @@ __device__ __forceinline__ void fma_step(double* p, const double* f, double c) {
         : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "s"(c));
 }
 
-// e[i] = 2^(z[i] x) for z[i] <= 0 <= x < 1e300: the integer part k of t = z x, the remainder f = z x - k
-// by one fma (|f| <= 1/2, no rounding of the product) and the degree-11 Chebyshev interpolant of 2^f
-// (relative error 2e-17 with its rounded coefficients); large arguments underflow to 0 in ldexp.
+// The largest argument x given to exp2_prods: beyond it every 2^(z x) of a basis (z x below -1075) is 0.
+constexpr double EXP2_XMAX = 1.0e20;
+
+// k = (int)t with the saturation of the hardware conversion (in C++ a t outside the range is undefined).
+__device__ __forceinline__ int sat_int(double t) {
+  int k;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(k) : "v"(t));
+  return k;
+}
+
+// e[i] = 2^(z[i] x) for -1e20 <= z[i] <= 0 <= x <= EXP2_XMAX: the integer part k of t = z x, the remainder
+// f = z x - k by one fma (|f| <= 1/2, no rounding of the product) and the degree-11 Chebyshev interpolant of
+// 2^f (relative error 2e-17 with its rounded coefficients).  Past |t| = 2^53 the remainder is the rounding
+// error of the product, at most 2^-53 1e40 here, so that the polynomial stays finite and ldexp gives 0.
 template <int N>
 __device__ __forceinline__ void exp2_prods(const double* z, double x, double* e) {
   double f[N], p[N];
@@ -71,7 +82,7 @@ __device__ __forceinline__ void exp2_prods(const double* z, double x, double* e)
   for (int i = 0; i < N; ++i) {
     const double t = rint(z[i] * x);
     f[i] = fma(z[i], x, -t);
-    k[i] = (int)t;
+    k[i] = sat_int(t);
     p[i] = 4.4558179083360645e-10;
   }
   fma_step<N>(p, f, 7.074194297288521e-09);
@@ -87,9 +98,10 @@ __device__ __forceinline__ void exp2_prods(const double* z, double x, double* e)
 #pragma unroll
   for (int i = 0; i < N; ++i) e[i] = ldexp(fma(p[i], f[i], 1.0), k[i]);
 }
+// The same for any x >= 0.
 __device__ __forceinline__ double exp2_prod(double z, double x) {
   double e;
-  exp2_prods<1>(&z, x, &e);
+  exp2_prods<1>(&z, fmin(x, EXP2_XMAX), &e);
   return e;
 }
 
@@ -811,7 +823,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KQ == 
         }
         continue;
       }
-      if constexpr (std::is_same<T, double>::value) r2 = fmin(r2, 1.0e200);
+      if constexpr (std::is_same<T, double>::value) r2 = fmin(r2, EXP2_XMAX);
       // the field words of an s or p shell before the exponentials (an s shell reads two words too many)
       const double h[3] = {hrow[o], hrow[o + 1], hrow[o + 2]};
       const T g[3] = {grow[o], grow[o + 1], grow[o + 2]};
@@ -1096,7 +1108,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         }
         continue;
       }
-      const double r2 = fmin(r2u, 1.0e200);
+      const double r2 = fmin(r2u, EXP2_XMAX);
       // radial moments sum c e, sum Z c e, sum Z^2 c e (the record holds -Z log2 e)
       double nr = 0.0, znr = 0.0, z2nr = 0.0;
       auto moments = [&](auto Nc) {

@@ -467,7 +467,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
           }
           continue;
         }
-        const double r2 = fmin(r2u, 1.0e200);
+        const double r2 = fmin(r2u, EXP2_XMAX);
         piece_radials<3>(hd, r2, R);
         hd.load(rec + p + 1);
         with_degree((info >> 4) & 15, [&](auto Lc) {
@@ -642,7 +642,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
         }
         continue;
       }
-      const double r2 = fmin(r2u, 1.0e200);
+      const double r2 = fmin(r2u, EXP2_XMAX);
       piece_radials<3>(hd, r2, R);
       hd.load(rec + p + 1);
       with_degree((info >> 4) & 15, [&](auto Lc) {
@@ -882,7 +882,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
             }
             continue;
           }
-          const double nr = piece_radial(hd, fmin(r2, 1.0e200));
+          const double nr = piece_radial(hd, fmin(r2, EXP2_XMAX));
           hd.load(rec + p + 1);
           with_degree((info >> 4) & 15, [&](auto Lc) {
             constexpr int l = decltype(Lc)::value, N = Mono<l>::N;
@@ -973,7 +973,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
             v_s[(o + q) * (WAVE + 1) + lane] = R[0] * y.P;
           }
         } else {
-          piece_radials<2>(hd, fmin(r2, 1.0e200), R);
+          piece_radials<2>(hd, fmin(r2, EXP2_XMAX), R);
           hd.load(rec + p + 1);
           with_degree((info >> 4) & 15, [&](auto Lc) {
             constexpr int l = decltype(Lc)::value, N = Mono<l>::N;
@@ -1273,7 +1273,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         }
         continue;
       }
-      const double r2 = fmin(r2u, 1.0e200);
+      const double r2 = fmin(r2u, EXP2_XMAX);
       piece_radials<4>(hd, r2, R);
       hd.load(rec + p + 1);
       with_degree((info >> 4) & 15, [&](auto Lc) {

@@ -1,0 +1,56 @@
+"""Distances at the ends of the FP64 range through the flattened kernels (local energy, lattice elements, position
+derivatives): a nucleus so far away that every exponential of its shells and of its Jastrow terms underflows
+(their arguments reach 1e121).  Against the oracle at 1e-9 of 1 + |T| + |V| (forces: of the largest element), as
+for the same kernels at ordinary distances."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _far_system(D, **kw):
+    """N2 with a hydrogen at distance D; every electron near N2."""
+    from jqmc_amd import synthetic
+
+    st = synthetic._structure(["N", "N", "H"], [[0.0, 0.0, -1.3], [0.0, 0.0, 1.3], [D, 0.0, 0.0]])
+    system = synthetic._assemble("far", st, {"N": "3s3p", "H": "2s1p1d"}, 1, ecp_elements={"N": 2}, **kw)
+    r_up, r_dn = system.initial_walkers(3, seed=4, sigma=0.8)
+    for r in (r_up, r_dn):
+        far = np.abs(r[..., 0]) > 1e4
+        r[far] = np.random.default_rng(0).normal(size=(int(far.sum()), 3))
+    return system.hamiltonian_data, r_up, r_dn
+
+
+@pytest.mark.parametrize("kw", [{}, {"j1": ("pade", 0.9), "j2": ("exp", 1.1)}], ids=["exp_pade", "pade_exp"])
+@pytest.mark.parametrize("D", [1e20, 1e23, 1e60])
+def test_far_nucleus_matches_oracle(D, kw):
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+    from oracle import coulomb as oc
+    from oracle import forces as of
+    from oracle import gfmc as og
+    from oracle import wf as owf
+
+    ham, r_up, r_dn = _far_system(D, **kw)
+    ws = WalkerState(SystemPack(ham), len(r_up)).init(r_up, r_dn)
+    RT = ws.rotations(3, 0)
+    e, kin, pot, _ = ws.local_energy(RT, with_parts=True)
+    Vd, Vn = ws.lrdmc_local_energy(WalkerState.lrdmc_params(0.25), RT)
+    grads = {k: v.cpu().numpy() for k, v in ws.position_grads(RT).items()}
+    for w in range(len(r_up)):
+        R = RT[w].cpu().numpy()
+        Gi = owf.geminal_inverse(owf.geminal(ham.wavefunction_data.geminal_data, r_up[w], r_dn[w]))
+        tu, td = owf.kinetic_all_elements_fast(ham.wavefunction_data, r_up[w], r_dn[w], Gi)
+        T = float(np.sum(tu) + np.sum(td))
+        V = oc.coulomb_potential_fast(ham.coulomb_potential_data, ham.wavefunction_data, r_up[w], r_dn[w], R, Gi, 1, 6)
+        tol = 1e-9 * (1.0 + abs(T) + abs(V))
+        assert abs(float(kin[w]) - T) <= tol and abs(float(pot[w]) - V) <= tol, (w, float(kin[w]), T, float(pot[w]), V)
+        d, n, _, _ = og.hamiltonian_elements(ham, r_up[w], r_dn[w], Gi, R, 0.25, "tmove")
+        tol = 1e-9 * (1.0 + abs(d) + abs(n))
+        assert abs(float(Vd[w]) - d) <= tol and abs(float(Vn[w]) - n) <= tol, (w, float(Vd[w]), d, float(Vn[w]), n)
+        ref = of.local_energy_position_grads(ham, r_up[w], r_dn[w], R)
+        for k in ("dE_dr", "dE_dR", "dlnpsi_dr", "dlnpsi_dR"):
+            size = max(1.0, float(np.abs(ref[k]).max()))
+            assert float(np.abs(grads[k][w] - ref[k]).max()) <= 1e-9 * size, (w, k)
