@@ -105,15 +105,16 @@ __device__ __forceinline__ double exp2_prod(double z, double x) {
   return e;
 }
 
-// 1 / x for normal x: two Newton steps on the hardware reciprocal.
+// 1 / x for normal x away from the ends of the range: two Newton steps on the hardware reciprocal.
 __device__ __forceinline__ double rcp_nr(double x) {
   double y = __builtin_amdgcn_rcp(x);
   y = fma(y, fma(-x, y, 1.0), y);
   return fma(y, fma(-x, y, 1.0), y);
 }
 
-// sqrt(x) and its reciprocal for x >= 0 (x = 0: taken as 1e-280): one Goldschmidt step on the hardware
-// reciprocal square root, then one residual correction of each.
+// sqrt(x) and its reciprocal for x >= 0 (below 1e-280: taken as that): one Goldschmidt step on the hardware
+// reciprocal square root, then one residual correction of each.  For distances whose reciprocal is not used,
+// or is cut off first.
 __device__ __forceinline__ double sqrt_nr(double x, double& inv) {
   x = fmax(x, 1.0e-280);
   const double y = __builtin_amdgcn_rsq(x);
@@ -125,6 +126,17 @@ __device__ __forceinline__ double sqrt_nr(double x, double& inv) {
   const double i = h + h;
   inv = fma(i, fma(-g, i, 1.0), i);
   return g;
+}
+
+// The same for every x, the reciprocal of 0 infinite: for Coulomb terms, so that the energy of coincident
+// particles is no number of ordinary size.
+__device__ __forceinline__ double sqrt_inv(double x, double& inv) {
+  double r = sqrt_nr(x, inv);
+  if (!(x >= 1.0e-280 && x <= 1.0e300)) {
+    r = sqrt(x);
+    inv = 1.0 / r;
+  }
+  return r;
 }
 
 struct JasPar {
@@ -294,7 +306,8 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
           bd = d;
           best = n;
         }
-        const double di = rcp_nr(d);
+        double di = rcp_nr(d);
+        if (!(d >= 1.0e-140 && d <= 1.0e150)) di = 1.0 / d;  // 0: infinite
         if (!J.lr) pot += -nc[n] * di;
         if (s.ecp_on) pot += ecp_local_nr(s, n, d, di);
         if (JP.j1_type) old += j1_value(JP, s.j1_c[n], s.j1_A[n], d);
@@ -303,7 +316,7 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
         if (f == e) continue;
         const double dx = x - rr[3 * f], dy = y - rr[3 * f + 1], dz = z - rr[3 * f + 2];
         double ri;
-        const double r = sqrt_nr(dx * dx + dy * dy + dz * dz, ri);
+        const double r = sqrt_inv(dx * dx + dy * dy + dz * dz, ri);
         pot += 0.5 * ri;
         if (JP.j2_type) old += j2_value(JP, r);
       }
@@ -662,7 +675,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KQ == 
                  gz = m0 * R[2] + m1 * R[5] + m2 * R[8];
     const double rx = s.nuc_pos[3 * nuc] - ex, ry = s.nuc_pos[3 * nuc + 1] - ey, rz = s.nuc_pos[3 * nuc + 2] - ez;
     double ri, gi;
-    const double rn2 = rx * rx + ry * ry + rz * rz, rn = sqrt_nr(rn2, ri);
+    const double rn2 = rx * rx + ry * ry + rz * rz, rn = sqrt_inv(rn2, ri);
     sqrt_nr(gx * gx + gy * gy + gz * gz, gi);
     px = ex + (rx + rn * gx);
     py = ey + (ry + rn * gy);

@@ -800,8 +800,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     const double g0 = m0 * Rm[0] + m1 * Rm[3] + m2 * Rm[6], g1 = m0 * Rm[1] + m1 * Rm[4] + m2 * Rm[7],
                  g2 = m0 * Rm[2] + m1 * Rm[5] + m2 * Rm[8];
     const double rx = s.nuc_pos[3 * nuc] - ex, ry = s.nuc_pos[3 * nuc + 1] - ey, rz = s.nuc_pos[3 * nuc + 2] - ez;
-    double ri, gni;
-    const double rn2 = rx * rx + ry * ry + rz * rz, rn = sqrt_nr(rn2, ri);
+    double gni;
+    const double rn2 = rx * rx + ry * ry + rz * rz, rn = sqrt(rn2), ri = 1.0 / rn;
     sqrt_nr(g0 * g0 + g1 * g1 + g2 * g2, gni);
     const double px = ex + (rx + rn * g0), py = ey + (ry + rn * g1), pz = ez + (rz + rn * g2);
     const double hx = -rx * ri, hy = -ry * ri, hz = -rz * ri;  // (r_e - R) / |r_e - R|

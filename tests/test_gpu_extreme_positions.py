@@ -54,3 +54,44 @@ def test_far_nucleus_matches_oracle(D, kw):
         for k in ("dE_dr", "dE_dR", "dlnpsi_dr", "dlnpsi_dR"):
             size = max(1.0, float(np.abs(ref[k]).max()))
             assert float(np.abs(grads[k][w] - ref[k]).max()) <= 1e-9 * size, (w, k)
+
+
+@pytest.mark.parametrize("name", ["water_ae", "benzene_ecp"])
+def test_coincident_particles_have_no_finite_energy(name):
+    """An electron pair of opposite spin at one point, an electron on a bare nucleus and one on a nucleus with an
+    effective core potential: the Coulomb terms are infinite (or no number), as plain division gives them, so that
+    a filter on finite energies sees these walkers; 1e-150 bohr apart the repulsion is 1e150.  Their neighbours
+    keep the values that they have alone."""
+    from jqmc_amd import synthetic
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+
+    system = synthetic.WORKLOADS[name](0)
+    ham = system.hamiltonian_data
+    pos = ham.structure_data.positions
+    pack = SystemPack(ham)
+    r_up, r_dn = system.initial_walkers(6, seed=5, sigma=0.8)
+    plain = WalkerState(pack, 6).init(r_up, r_dn)
+    e0 = plain.local_energy(plain.rotations(3, 0))
+    r_dn[1, 0] = r_up[1, 0]
+    r_up[2, 0] = pos[-1]  # hydrogen, without a core potential
+    r_up[3, 0] = pos[0]
+    r_dn[4, 0], r_up[4, 0, 2], r_dn[4, 0, 2] = r_up[4, 0], 1.0e-150, 2.0e-150
+    ws = WalkerState(pack, 6).init(r_up, r_dn)
+    RT = ws.rotations(3, 0)
+    e, kin, pot, _ = ws.local_energy(RT, with_parts=True)
+    inf = float("inf")
+    assert float(pot[1]) == inf and float(e[1]) == inf and np.isfinite(float(kin[1]))
+    assert float(pot[2]) == -inf and float(e[2]) == -inf
+    assert not np.isfinite(float(e[3]))
+    assert abs(float(e[4]) - 1.0e150) <= 1e-9 * 1.0e150
+    assert torch.equal(e[[0, 5]], e0[[0, 5]])
+    Vd, _ = ws.lrdmc_local_energy(WalkerState.lrdmc_params(0.25), RT)
+    assert float(Vd[1]) == inf and abs(float(Vd[4]) - 1.0e150) <= 1e-9 * 1.0e150
+    g = ws.position_grads(RT)
+    assert float(g["e_L"][1]) == inf and float(g["e_L"][2]) == -inf
+    for w in (1, 2, 3):
+        assert not torch.isfinite(g["dE_dr"][w, 0]).any() or not torch.isfinite(g["dE_dr"][w, pack.n_up]).any()
+        assert not torch.isfinite(g["force_HF"][w]).all()
+    if ham.coulomb_potential_data.ecp_flag:  # the quadrature of that electron has no direction: nothing of it is finite
+        assert not torch.isfinite(g["dE_dr"][3]).any()
