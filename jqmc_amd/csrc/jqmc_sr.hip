@@ -45,9 +45,13 @@ struct SrMoments {
   }
 };
 // Union of two sets about its own mean (rounded): the first moments about the rounded means are kept, so that
-// their rounding enters var in second order only, as it does in two passes.
+// their rounding enters var in second order only, as it does in two passes.  A set without weight has no mean:
+// the other's is the common pivot, else the distance to its arbitrary one would cancel in s2.
 __device__ __forceinline__ SrMoments sr_merge(SrMoments a, SrMoments b) {
-  b.shift(a.m - b.m);
+  const double pivot = a.w != 0.0 ? a.m : b.m;
+  a.shift(pivot - a.m);
+  b.shift(pivot - b.m);
+  a.m = pivot;
   a.w += b.w;
   a.s1 += b.s1;
   a.s2 += b.s2;
@@ -106,7 +110,7 @@ __global__ void __launch_bounds__(SRC_WAVES * 64) k_sr_colstats(const double* __
   }
   t.shift(mk - t.m);
   mean[k] = mk;
-  var[k] = t.s2;
+  var[k] = t.s2 < 0.0 ? 0.0 : t.s2;  // the rounding of a constant column
 }
 
 // out_k = cs_k * sum_i (O_ik - mean_k) rs_i x_i for the row-major (S x P) O: theta = X x (and

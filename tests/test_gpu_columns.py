@@ -48,6 +48,32 @@ def test_column_statistics_and_projection(S, P, ld, shift):
     assert (np.abs(out.cpu().numpy() - terms.sum(axis=0)) <= (S + 8) * U * (np.abs(terms).sum(axis=0) + U)).all()
 
 
+@pytest.mark.parametrize("S,zero", [(64, slice(0, 8)), (200, slice(0, 64)), (200, slice(64, 128)), (1030, slice(0, 700)),
+                                    (70, slice(0, 69)), (130, slice(8, 130))])
+def test_column_statistics_with_rows_of_no_weight(S, zero):
+    """Whole groups of rows with weight exactly 0 (walkers that are out), wherever they stand; the bound of the
+    statistics above.  A constant column has no negative variance."""
+    rng = np.random.default_rng(S)
+    P = 70
+    O = rng.normal(size=(S, P)) + 1e7
+    O[:, 3] = -0.1
+    O[:, 4] = 1e5 / 3.0
+    wn = rng.uniform(0.2, 1.0, size=S)
+    wn[zero] = 0.0
+    wn /= wn.sum()
+    X, w = O.astype(np.longdouble), wn.astype(np.longdouble)
+    m_ref = w @ X
+    v_ref = w @ (X - m_ref) ** 2
+    Od, wd = torch.as_tensor(O, device="cuda"), torch.as_tensor(wn, device="cuda")
+    mean = torch.full((P,), np.nan, dtype=torch.float64, device="cuda")
+    var = torch.full_like(mean, np.nan)
+    _lib.call("jqmc_sr_colstats", _ptr(Od), S, P, P, _ptr(wd), _ptr(mean), _ptr(var), stream_handle())
+    m, v = mean.cpu().numpy(), var.cpu().numpy()
+    assert (np.abs(m - m_ref) <= (S + 4) * U * (w @ np.abs(X))).all()
+    assert (np.abs(v - v_ref) <= 4 * (S + 16) * U * (v_ref + U * np.abs(X).max(axis=0) ** 2)).all()
+    assert (v >= 0.0).all()
+
+
 @pytest.mark.parametrize("name,W", [("water_ae", 1), ("water_ae", 17), ("chain10", 9), ("benzene_ecp", 8),
                                     ("water4_jagp", 3)])
 def test_parameter_blocks_are_the_outer_products(name, W):
