@@ -436,7 +436,22 @@ int el_kin_waves(const Sys& s) {
   return el_kin_lds<T>(s.n_orb, s.el_ks, EL_KIN_WAVES) <= kMaxKineticLds ? EL_KIN_WAVES : EL_KIN_WAVES / 2;
 }
 
-// The three launches for the jobs of systems host[k] (jobs and host in the same order).
+// f with the orbital class of a system (Sys::el_ks) as a constant.
+template <typename F>
+void with_kq(int kq, F&& f) {
+  if (kq == 4)
+    f(std::integral_constant<int, 4>{});
+  else if (kq == 8)
+    f(std::integral_constant<int, 8>{});
+  else if (kq == 12)
+    f(std::integral_constant<int, 12>{});
+  else if (kq == 16)
+    f(std::integral_constant<int, 16>{});
+  else
+    f(std::integral_constant<int, 0>{});
+}
+
+// The launches for the jobs of systems host[k] (jobs and host in the same order).
 template <typename T>
 int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
   int64_t n = 0;
@@ -457,52 +472,46 @@ int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
       const int64_t waves = M.job[k].W * ((s.n_up + 15) / 16 + (s.n_dn + 15) / 16);
       k_el_hrows<T><<<(unsigned)((waves + 3) / 4), 256, 0, st>>>(M.job[k]);
     }
+  // the kinetic energies: one launch per orbital class and waves per block present, so that the order of a
+  // system's sums does not depend on the systems that share the call; the points: one per orbital class
   for (int kq : {4, 8, 12, 16, 0}) {
-    ElJobs<T> G{};
-    int64_t nk = 0, np = 0, lds = 0;
-    int nw = EL_KIN_WAVES;
-    for (int k = 0; k < M.n; ++k) {
-      const Sys& s = *host[k];
-      if (s.el_ks != kq) continue;
-      ElJob<T>& J = G.job[G.n++];
-      J = M.job[k];
-      J.kin0 = nk;
-      nk += (J.W * s.n_el + EL_KIN_ROWS - 1) / EL_KIN_ROWS;
-      nw = std::min(nw, el_kin_waves<T>(s));
-      // points: lattice groups of ten electrons, then per four walkers the groups of listed electrons
-      const bool nonlocal = s.ecp_on && s.nv > 0;
-      const int parts = el_parts(s), per = s.nv > 0 ? std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)) : 1;
-      J.pts0 = np;
-      J.lat_groups = J.lr ? (J.W * s.n_el + EL_SLOTS - 1) / EL_SLOTS : 0;
-      J.ecp_groups = (4 * s.n_el * parts + per - 1) / per;
-      const int64_t ecp = nonlocal ? (J.W + 3) / 4 * J.ecp_groups : 0;
-      np += (J.lat_groups + ecp + 3) / 4;
+    ElJobs<T> P{};
+    int64_t np = 0;
+    for (int nw : {EL_KIN_WAVES / 2, EL_KIN_WAVES}) {
+      ElJobs<T> G{};
+      int64_t nk = 0, lds = 0;
+      for (int k = 0; k < M.n; ++k) {
+        const Sys& s = *host[k];
+        if (s.el_ks != kq || el_kin_waves<T>(s) != nw) continue;
+        ElJob<T>& J = G.job[G.n++];
+        J = M.job[k];
+        J.kin0 = nk;
+        nk += (J.W * s.n_el + EL_KIN_ROWS - 1) / EL_KIN_ROWS;
+        lds = std::max(lds, el_kin_lds<T>(s.n_orb, kq, nw));
+        // points: lattice groups of ten electrons, then per four walkers the groups of listed electrons
+        const bool nonlocal = s.ecp_on && s.nv > 0;
+        const int parts = el_parts(s), per = s.nv > 0 ? std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)) : 1;
+        J.pts0 = np;
+        J.lat_groups = J.lr ? (J.W * s.n_el + EL_SLOTS - 1) / EL_SLOTS : 0;
+        J.ecp_groups = (4 * s.n_el * parts + per - 1) / per;
+        const int64_t ecp = nonlocal ? (J.W + 3) / 4 * J.ecp_groups : 0;
+        np += (J.lat_groups + ecp + 3) / 4;
+        P.job[P.n++] = J;
+      }
+      if (G.n == 0) continue;
+      if (nk > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+      with_kq(kq, [&](auto K) {
+        constexpr int KQ = decltype(K)::value;
+        // more than 64 KiB of dynamic LDS has to be allowed once per kernel
+        static const hipError_t allowed =
+            hipFuncSetAttribute(reinterpret_cast<const void*>(&k_el_kinetic<T, KQ>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxKineticLds);
+        (void)allowed;
+        k_el_kinetic<T, KQ><<<(unsigned)nk, nw * WAVE, lds, st>>>(G);
+      });
     }
-    if (G.n == 0) continue;
-    if (std::max(nk, np) > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
-    for (int k = 0; k < M.n; ++k)
-      if (host[k]->el_ks == kq) lds = std::max(lds, el_kin_lds<T>(host[k]->n_orb, kq, nw));
-    const unsigned bk = (unsigned)nk, bp = (unsigned)np;
-    auto run = [&](auto K) {
-      constexpr int KQ = decltype(K)::value;
-      // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-      static const hipError_t allowed =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(&k_el_kinetic<T, KQ>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxKineticLds);
-      (void)allowed;
-      k_el_kinetic<T, KQ><<<bk, nw * WAVE, lds, st>>>(G);
-      if (bp) k_el_points<T, KQ><<<bp, 256, 0, st>>>(G);
-    };
-    if (kq == 4)
-      run(std::integral_constant<int, 4>{});
-    else if (kq == 8)
-      run(std::integral_constant<int, 8>{});
-    else if (kq == 12)
-      run(std::integral_constant<int, 12>{});
-    else if (kq == 16)
-      run(std::integral_constant<int, 16>{});
-    else
-      run(std::integral_constant<int, 0>{});
+    if (np > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+    if (np) with_kq(kq, [&](auto K) { k_el_points<T, decltype(K)::value><<<(unsigned)np, 256, 0, st>>>(P); });
   }
   return JQMC_OK;
 }

@@ -93,3 +93,33 @@ def test_lattice_elements_match_oracle(name, mos, nv, W):
         d, n, _, _ = og.hamiltonian_elements(ham, r_up[w], r_dn[w], Gi, RT[w].cpu().numpy(), 0.25, move, Nv=nv)
         tol = 1e-9 * (1.0 + abs(d) + abs(n))
         assert abs(float(Vd[w]) - d) <= tol and abs(float(Vn[w]) - n) <= tol, (move, float(Vd[w]), d, float(Vn[w]), n)
+
+
+def test_batch_companions_change_no_bit():
+    """A system of 50 orbitals (four waves per block of the kinetic kernel) has the same bits alone and in one call
+    with a system of 60 orbitals (two waves) of the same orbital class, and with one of another class."""
+    import torch
+
+    from jqmc_amd import synthetic
+    from jqmc_amd._api import WalkerState, lrdmc_projection_multi
+    from jqmc_amd._pack import SystemPack
+
+    base = synthetic.chain_ecp(30, 1)
+    packs = [SystemPack(_with_mos(base, n, True)) for n in (50, 60, 18)]
+    prm = WalkerState.lrdmc_params(0.3, n_steps=2)
+
+    def run(n_systems):
+        states = []
+        for k, W in zip(range(n_systems), (5, 3, 2)):
+            states.append(WalkerState(packs[k], W).init(*base.initial_walkers(W, seed=21 + k)))
+        outs = lrdmc_projection_multi(states, [prm] * n_systems, 17, [100] * n_systems)
+        torch.cuda.synchronize()
+        return states[0], outs[0]
+
+    s1, o1 = run(1)
+    for n in (2, 3):
+        s, o = run(n)
+        for key in ("V_diag", "V_nondiag", "w_L", "RT"):
+            assert torch.equal(o[key], o1[key]), (n, key)
+        for key in ("r_up", "r_dn", "Ginv", "jfield"):
+            assert torch.equal(getattr(s, key), getattr(s1, key)), (n, key)
