@@ -500,20 +500,31 @@ int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
       }
       if (G.n == 0) continue;
       if (nk > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
-      with_kq(kq, [&](auto K) {
-        constexpr int KQ = decltype(K)::value;
-        // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-        static const hipError_t allowed =
-            hipFuncSetAttribute(reinterpret_cast<const void*>(&k_el_kinetic<T, KQ>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxKineticLds);
-        (void)allowed;
-        k_el_kinetic<T, KQ><<<(unsigned)nk, nw * WAVE, lds, st>>>(G);
-      });
+      with_kq(kq, [&](auto K) { k_el_kinetic<T, decltype(K)::value><<<(unsigned)nk, nw * WAVE, lds, st>>>(G); });
     }
     if (np > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
     if (np) with_kq(kq, [&](auto K) { k_el_points<T, decltype(K)::value><<<(unsigned)np, 256, 0, st>>>(P); });
   }
   return JQMC_OK;
+}
+
+constexpr size_t FR_TILE_BYTES = EL_KIN_ROWS * EL_LD * sizeof(double);
+
+// Allows the kernels that take more than 64 KiB of dynamic LDS to do so on the current device, the system's:
+// a permission holds for one kernel on one device.
+hipError_t allow_large_lds(const Sys& s) {
+  auto allow = [](auto* kernel, int64_t bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)bytes);
+  };
+  hipError_t rc = hipSuccess;
+  with_kq(s.el_ks, [&](auto K) {
+    constexpr int KQ = decltype(K)::value;
+    rc = s.precision == JQMC_PRECISION_MIXED_FP32 ? allow(&k_el_kinetic<float, KQ>, kMaxKineticLds)
+                                                  : allow(&k_el_kinetic<double, KQ>, kMaxKineticLds);
+  });
+  if (rc == hipSuccess) rc = allow(&k_fr_orbital, FR_WAVES * 3 * FR_TILE_BYTES);
+  return rc;
 }
 
 template <typename T>
@@ -612,11 +623,7 @@ int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, co
   J.part = B.part;
   J.re = B.re;
   J.pt = B.pt;
-  constexpr size_t tile = EL_KIN_ROWS * EL_LD * sizeof(double);
-  // more than 64 KiB of dynamic LDS has to be allowed once per kernel
-  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fr_orbital),
-                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(FR_WAVES * 3 * tile));
-  HIP_TRY(allowed);
+  constexpr size_t tile = FR_TILE_BYTES;
   k_fr_kinetic<<<blocks, FR_WAVES * WAVE, FR_WAVES * 2 * tile, st>>>(J);
   if (s.ecp_on && s.nv > 0) {
     const int per = std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)), groups = (4 * s.n_el + per - 1) / per;
@@ -1112,6 +1119,10 @@ int jqmc_system_create(const jqmc_system_desc* d, jqmc_system** out) {
     UPLOAD(d->mesh_weights, (size_t)d->nv, s.mesh_w);
   }
   UPLOAD(&s, 1, sys->d_sys);
+  if (const hipError_t rc = allow_large_lds(s); rc != hipSuccess) {
+    jqmc_system_destroy(sys);
+    return fail(JQMC_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(rc));
+  }
   {
     void* h = nullptr;
     HIP_TRY(hipHostMalloc(&h, LR_MAX_SYSTEMS * sizeof(int), hipHostMallocDefault));
