@@ -255,6 +255,11 @@ WalkT<T> to_walk(const jqmc_walkers* w) {
 
 inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
+// Grid of n blocks whose kernel takes its index from wide_block() (and leaves at indices past its work).
+inline dim3 wide_grid(int64_t n) {
+  return n <= WIDE_ROW ? dim3((unsigned)n) : dim3((unsigned)WIDE_ROW, (unsigned)((n + WIDE_ROW - 1) / WIDE_ROW));
+}
+
 inline int64_t cache_bytes(const Sys& s) {
   return s.precision == JQMC_PRECISION_MIXED_FP32 ? (int64_t)sizeof(float) : (int64_t)sizeof(double);
 }
@@ -267,7 +272,7 @@ int launch_jfield_gemm(const Sys& s, int64_t W, const double* S1, const double* 
   const int64_t n_rt = (W * s.n_el + JG_TILE - 1) / JG_TILE;
   const int n_ct = (s.n_ao + JG_TILE - 1) / JG_TILE;
   const int64_t blocks = (n_rt + 7) / 8 * 8 * n_ct;
-  if (blocks > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+  if (blocks > MAX_BLOCKS) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
   k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, W * s.n_el, S1, S2, j1, G, n_ct, n_rt);
   return JQMC_OK;
 }
@@ -463,9 +468,8 @@ int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
     J.q_blocks = (J.W * tiles + 3) / 4;
     n += J.q_blocks + (J.W + 3) / 4;
   }
-  if (n > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
   if (n == 0) return JQMC_OK;
-  k_el_prep<T><<<(unsigned)n, 256, 0, st>>>(M);
+  k_el_prep<T><<<wide_grid(n), 256, 0, st>>>(M);
   for (int k = 0; k < M.n; ++k)
     if (el_h_rows(*host[k])) {
       const Sys& s = *host[k];
@@ -499,10 +503,10 @@ int launch_el(ElJobs<T>& M, const Sys* const* host, hipStream_t st) {
         P.job[P.n++] = J;
       }
       if (G.n == 0) continue;
-      if (nk > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+      if (nk > MAX_BLOCKS) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
       with_kq(kq, [&](auto K) { k_el_kinetic<T, decltype(K)::value><<<(unsigned)nk, nw * WAVE, lds, st>>>(G); });
     }
-    if (np > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+    if (np > MAX_BLOCKS) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
     if (np) with_kq(kq, [&](auto K) { k_el_points<T, decltype(K)::value><<<(unsigned)np, 256, 0, st>>>(P); });
   }
   return JQMC_OK;
@@ -628,7 +632,7 @@ int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, co
   if (s.ecp_on && s.nv > 0) {
     const int per = std::min(EL_SLOTS, WAVE / std::min(s.nv, WAVE)), groups = (4 * s.n_el + per - 1) / per;
     const int64_t n = ((W + 3) / 4 * groups + 3) / 4;
-    if (n > 0x7FFFFFFFll) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
+    if (n > MAX_BLOCKS) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
     k_fr_points<<<(unsigned)n, 256, 0, st>>>(J, groups);
   }
   k_fr_adjoint<<<blocks, FR_WAVES * WAVE, FR_WAVES * 2 * tile, st>>>(J);
@@ -1741,8 +1745,7 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
   // out (M x N per walker) = L^T R on the matrix cores
   auto outer = [&](int K, int M, int N, auto* L, int64_t l_ld, int64_t l_rs, int64_t l_cs, auto* R, int64_t r_ld,
                    int64_t r_rs, double* out, int64_t out_ld, int64_t out_rs, int64_t out_off) {
-    constexpr int64_t kChunk = 1 << 20;  // walkers per launch (at most 2^31 blocks)
-    const int64_t n_mt = (M + RO_ROWS - 1) / RO_ROWS;
+    const int64_t n_mt = (M + RO_ROWS - 1) / RO_ROWS, kChunk = MAX_BLOCKS / n_mt / 8 * 8;  // walkers per launch
     for (int64_t w0 = 0; w0 < W; w0 += kChunk) {
       const int64_t nw = std::min(W - w0, kChunk);
       k_rank_outer<<<(unsigned)((nw + 7) / 8 * 8 * n_mt), 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs,
@@ -1760,7 +1763,7 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
     k_init_jsums<T><<<grid_for(W * na, 256), 256, 0, st>>>(s, W, k, S1, nullptr);
     outer(ne, na, na, k.ao, (int64_t)ne * na, na, 1, S1, (int64_t)ne * na, na, O, ld, na + 1, lay.j3);
   }
-  k_dlnpsi_small<T><<<(unsigned)W, 256, 0, st>>>(s, W, k, Z, lay, O, ld);
+  k_dlnpsi_small<T><<<wide_grid(W), 256, 0, st>>>(s, W, k, Z, lay, O, ld);
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }

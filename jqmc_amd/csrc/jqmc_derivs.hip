@@ -97,7 +97,8 @@ __global__ void __launch_bounds__(256) k_dlnpsi_small(Sys s, int64_t W, WalkT<T>
                                                       ParamLayout lay, double* __restrict__ out, int64_t out_ld) {
   __shared__ double part[4][2];
   const int wave = wave_id(), lane = lane_id(), tid = threadIdx.x;
-  const int64_t w = blockIdx.x;
+  const int64_t w = wide_block();
+  if (w >= W) return;  // uniform across the block
   const int ne = s.n_el, na = s.n_ao, no = s.n_orb, nu = s.n_up, nd = s.n_dn;
   double* ow = out + w * out_ld;
   double acc[2] = {0.0, 0.0};

@@ -175,6 +175,11 @@ __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 // instead of the same computation repeated in 64 lanes.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); }
 
+// Blocks of 256 threads that one launch takes along x (the runtime refuses 2^32 work-items), and the block index
+// of a grid that goes on along y past a row of WIDE_ROW blocks (wide_grid on the host).
+constexpr int64_t MAX_BLOCKS = (1ll << 24) - 1, WIDE_ROW = 1ll << 23;
+__device__ __forceinline__ int64_t wide_block() { return (int64_t)blockIdx.y * WIDE_ROW + blockIdx.x; }
+
 // Makes this wavefront's earlier LDS and global writes visible to all of its lanes:
 // release/acquire fences at workgroup scope (outstanding memory operations complete,
 // no compiler reordering across the point) around the wavefront barrier.  Only lanes

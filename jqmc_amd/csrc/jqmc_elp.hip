@@ -224,11 +224,12 @@ __device__ __forceinline__ double ecp_local_nr(CSys& s, int n, double d, double 
 template <typename T>
 __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
   __shared__ double rr_s[4][3 * 128];  // n_up <= 64, so at most 128 electrons
+  const int64_t bid = wide_block();
   int kj = 0;
-  while (kj + 1 < M.n && M.job[kj + 1].prep0 <= (int64_t)blockIdx.x) ++kj;
+  while (kj + 1 < M.n && M.job[kj + 1].prep0 <= bid) ++kj;
   const ElJob<T>& J = M.job[kj];
   CSys& s = csys(J.sys);
-  const int64_t blk = (int64_t)blockIdx.x - J.prep0;
+  const int64_t blk = bid - J.prep0;
   const int wave = wave_id(), lane = lane_id();
   const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, no = s.n_orb;
   if (blk < J.q_blocks) {

@@ -75,5 +75,23 @@ def large_lds(host):
     return out
 
 
+def many_walkers(host):
+    """H2 with the most walkers that the set-up takes in one launch: set-up, local energy, one projection and the
+    parameter derivatives."""
+    from jqmc_amd import synthetic
+
+    st = synthetic._structure(["H", "H"], [[0.0, 0.0, 0.0], [0.0, 0.0, 1.4]])
+    pack = host.pack(synthetic._assemble("h2", st, {"H": "1s"}, 1, use_j3=False).hamiltonian_data)
+    W = (1 << 25) - 8
+    p = ctypes.byref(host.walkers())
+    out = host.launches("jqmc_walkers_init", pack.handle, W, p, FAKE, 1 << 60, None)
+    out += host.local_energy(pack, W)
+    prm = host.lib.LrdmcParams(mode=0, n_steps=1, alat=0.3, E_scf=0.0, tau=0.0, non_local_move=0, random_mesh=1)
+    out += host.launches("jqmc_lrdmc_projection", pack.handle, W, p, ctypes.byref(prm), 1, 0, FAKE, FAKE, FAKE, FAKE,
+                         FAKE, FAKE, FAKE, 1 << 60, None)
+    out += host.launches("jqmc_dln_psi_dparams", pack.handle, W, p, 15, FAKE, 1 << 10, FAKE, 1 << 60, None)
+    return out
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[2]](Host(sys.argv[1]))))

@@ -123,3 +123,24 @@ def test_batch_companions_change_no_bit():
             assert torch.equal(o[key], o1[key]), (n, key)
         for key in ("r_up", "r_dn", "Ginv", "jfield"):
             assert torch.equal(getattr(s, key), getattr(s1, key)), (n, key)
+
+
+def test_more_walkers_than_a_row_of_blocks():
+    """12 million walkers of H2: the grids of k_el_prep and k_dlnpsi_small go on along y.  Every walker has the bits
+    that it has in a small set."""
+    import torch
+
+    from jqmc_amd import synthetic
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+
+    st = synthetic._structure(["H", "H"], [[0.0, 0.0, 0.0], [0.0, 0.0, 1.4]])
+    system = synthetic._assemble("h2", st, {"H": "1s"}, 1, use_j3=False)
+    pack, n, rep = SystemPack(system.hamiltonian_data), 1000, 12000
+    r_up, r_dn = (torch.as_tensor(r, device="cuda") for r in system.initial_walkers(n, seed=2))
+    small = WalkerState(pack, n).init(r_up, r_dn)
+    large = WalkerState(pack, n * rep).init(r_up.repeat(rep, 1, 1), r_dn.repeat(rep, 1, 1))
+    assert torch.equal(large.local_energy().view(rep, n), small.local_energy().expand(rep, n))
+    O, ref = large.dln_psi_dparams(), small.dln_psi_dparams()
+    for k in ref:
+        assert torch.equal(O[k].view(rep, n, -1), ref[k].view(1, n, -1).expand(rep, n, ref[k][0].numel())), k
