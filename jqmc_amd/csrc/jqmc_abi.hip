@@ -1735,6 +1735,9 @@ ParamLayout param_layout(const Sys& s, int32_t blocks) {
   return L;
 }
 
+// Waves per walker of k_dlnpsi_small.
+inline int dln_waves(const Sys& s) { return s.n_el > 16 || s.n_ao > 64 ? 4 : 1; }
+
 template <typename T>
 int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLayout& lay, double* O, int64_t ld,
                   void* workspace, hipStream_t st) {
@@ -1745,12 +1748,23 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
   // out (M x N per walker) = L^T R on the matrix cores
   auto outer = [&](int K, int M, int N, auto* L, int64_t l_ld, int64_t l_rs, int64_t l_cs, auto* R, int64_t r_ld,
                    int64_t r_rs, double* out, int64_t out_ld, int64_t out_rs, int64_t out_off) {
-    const int64_t n_mt = (M + RO_ROWS - 1) / RO_ROWS, kChunk = MAX_BLOCKS / n_mt / 8 * 8;  // walkers per launch
+    const bool narrow = N <= RO_NARROW;
+    const int cols = narrow ? (N > 16 ? 32 : 16) : N;
+    const int64_t n_mt = (M + RO_ROWS - 1) / RO_ROWS * ((N + cols - 1) / cols);
+    const int64_t kChunk = MAX_BLOCKS / n_mt / 8 * 8;  // walkers per launch
     for (int64_t w0 = 0; w0 < W; w0 += kChunk) {
       const int64_t nw = std::min(W - w0, kChunk);
-      k_rank_outer<<<(unsigned)((nw + 7) / 8 * 8 * n_mt), 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs,
-                                                                       R + w0 * r_ld, r_ld, r_rs, out + w0 * out_ld,
-                                                                       out_ld, out_rs, out_off);
+      const unsigned tiles = (unsigned)((nw * n_mt + 3) / 4);
+      if (cols == 16)
+        k_rank_narrow<1><<<tiles, 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs, R + w0 * r_ld, r_ld,
+                                                r_rs, out + w0 * out_ld, out_ld, out_rs, out_off);
+      else if (narrow)
+        k_rank_narrow<2><<<tiles, 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs, R + w0 * r_ld, r_ld,
+                                                r_rs, out + w0 * out_ld, out_ld, out_rs, out_off);
+      else
+        k_rank_outer<<<(unsigned)((nw + 7) / 8 * 8 * n_mt), 256, 0, st>>>(K, M, N, nw, L + w0 * l_ld, l_ld, l_rs, l_cs,
+                                                                         R + w0 * r_ld, r_ld, r_rs,
+                                                                         out + w0 * out_ld, out_ld, out_rs, out_off);
     }
   };
   if (lay.lam >= 0) {
@@ -1763,7 +1777,7 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
     k_init_jsums<T><<<grid_for(W * na, 256), 256, 0, st>>>(s, W, k, S1, nullptr);
     outer(ne, na, na, k.ao, (int64_t)ne * na, na, 1, S1, (int64_t)ne * na, na, O, ld, na + 1, lay.j3);
   }
-  k_dlnpsi_small<T><<<wide_grid(W), 256, 0, st>>>(s, W, k, Z, lay, O, ld);
+  k_dlnpsi_small<T><<<wide_grid(W), dln_waves(s) * WAVE, 0, st>>>(s, W, k, Z, lay, O, ld);
   HIP_TRY(hipGetLastError());
   return JQMC_OK;
 }

@@ -78,8 +78,6 @@ def test_column_statistics_with_rows_of_no_weight(S, zero):
                                     ("water4_jagp", 3)])
 def test_parameter_blocks_are_the_outer_products(name, W):
     from jqmc_amd import synthetic
-    from jqmc_amd._api import WalkerState
-    from jqmc_amd._pack import SystemPack
 
     if name == "chain10":
         system = synthetic.chain_ecp(10, 1)
@@ -87,6 +85,24 @@ def test_parameter_blocks_are_the_outer_products(name, W):
         system = synthetic.water4_ecp(0, jagp=True)
     else:
         system = synthetic.WORKLOADS[name](0)
+    _check_parameter_blocks(system, W)
+
+
+@pytest.mark.parametrize("jagp", [False, True])
+@pytest.mark.parametrize("n_ao,W", [(16, 3), (17, 5), (32, 2), (33, 7), (112, 3), (113, 3)])
+def test_parameter_blocks_around_the_narrow_tiles(n_ao, W, jagp):
+    """AO counts around the 16- and 32-column tiles of the narrow form and its largest size; an open shell."""
+    from jqmc_amd import synthetic
+
+    st = synthetic._structure(["N"], [[0.0, 0.0, 0.0]])
+    _check_parameter_blocks(synthetic._assemble("n", st, {"N": f"{n_ao}s"}, 1, jagp=jagp, lam_rank=12), W)
+
+
+def _check_parameter_blocks(system, W):
+    """The J3 and Lambda_p blocks against outer products of the cached rows."""
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+
     r_up, r_dn = system.initial_walkers(W, seed=21)
     ws = WalkerState(SystemPack(system.hamiltonian_data), W).init(r_up, r_dn)
     O = {k: v.reshape(W, -1) for k, v in ws.dln_psi_dparams().items()}

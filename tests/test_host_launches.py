@@ -43,5 +43,5 @@ def test_what_the_set_up_takes_is_taken_by_the_other_calls(shim):
     """A launch of 2^32 work-items or more along one dimension is refused: no call of a walker set that the set-up
     takes runs into that."""
     rec = _scenario(shim, "many_walkers")
-    assert {"k_init_rows", "k_el_prep", "k_lrdmc_move", "k_dlnpsi_small", "k_rank_outer"} <= {r[0] for r in rec}
+    assert {"k_init_rows", "k_el_prep", "k_lrdmc_move", "k_dlnpsi_small", "k_rank_narrow"} <= {r[0] for r in rec}
     assert not [r for r in rec if r[-1]]
