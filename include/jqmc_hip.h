@@ -308,7 +308,7 @@ int jqmc_counter_add(int64_t* ctr, int64_t inc, void* stream);
  * Outputs: e_L (W), dE_dr and dlnpsi_dr (W, N, 3), dE_dR, dlnpsi_dR, force_HF, force_PP
  * (W, n_nuc, 3); any may be NULL.  Plain FP64 systems only (JQMC_ERR_UNSUPPORTED otherwise).
  * workspace: jqmc_position_grads_workspace_bytes() bytes, contents need not be initialised; it grows with W up
- * to 4096 walkers, more are taken 4096 at a time.
+ * to 131072 electrons, more are taken in equal parts of at most as many.
  */
 int jqmc_position_grads_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes);
 int jqmc_position_grads(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const double* RT, int32_t swct,

@@ -651,7 +651,7 @@ int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, co
       J.phib_add = 1;
     }
   }
-  k_fr_pairing<<<(unsigned)W, 256, 2 * sizeof(double) * s.n_up * s.n_up, st>>>(J);
+  k_fr_pairing<<<(unsigned)W, fr_pairing_waves(s) * WAVE, 2 * sizeof(double) * s.n_up * s.n_up, st>>>(J);
   if (s.orb_is_mo) {
     E.Q = B.phib;
     E.H = s.j3_on ? B.gbar : B.wv;
@@ -661,7 +661,7 @@ int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, co
       k_el_hrows<double><<<rows, 256, 0, st>>>(E);
   }
   k_fr_orbital<<<blocks, FR_WAVES * WAVE, FR_WAVES * 3 * tile, st>>>(J);
-  k_fr_out<<<(unsigned)W, 256, 0, st>>>(J, out);
+  k_fr_out<<<(unsigned)W, fr_out_waves(s) * WAVE, 0, st>>>(J, out);
   return JQMC_OK;
 }
 
@@ -1371,7 +1371,7 @@ int jqmc_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk,
 int jqmc_position_grads_workspace_bytes(const jqmc_system* sys, int64_t W, int64_t* bytes) {
   if (!sys || !bytes) return fail(JQMC_ERR_INVALID_ARGUMENT, "NULL argument");
   if (W < 0) return fail(JQMC_ERR_SHAPE, "W < 0");
-  *bytes = FrBuf(sys->s, std::min(W, FR_CHUNK), nullptr).doubles * (int64_t)sizeof(double);
+  *bytes = FrBuf(sys->s, std::min(W, FR_ELECTRONS / sys->s.n_el), nullptr).doubles * (int64_t)sizeof(double);
   return JQMC_OK;
 }
 
@@ -1394,10 +1394,11 @@ int jqmc_position_grads(const jqmc_system* sys, int64_t W, const jqmc_walkers* w
   hipStream_t st = (hipStream_t)stream;
   const int64_t ne = s.n_el, nn = s.n_nuc;
   auto at = [](double* p, int64_t n) { return p ? p + n : nullptr; };
-  for (int64_t w0 = 0; w0 < W; w0 += FR_CHUNK) {
+  const int64_t chunk = fr_chunk(s, W);
+  for (int64_t w0 = 0; w0 < W; w0 += chunk) {
     const FrOut out{at(e_L, w0), at(dE_dr, 3 * ne * w0), at(dE_dR, 3 * nn * w0), at(dlnpsi_dr, 3 * ne * w0),
                     at(dlnpsi_dR, 3 * nn * w0), at(force_HF, 3 * nn * w0), at(force_PP, 3 * nn * w0), swct ? 1 : 0};
-    rc = launch_forces(sys, std::min(W - w0, FR_CHUNK), walk_from(s, to_walk<double>(wk), w0), RT ? RT + 9 * w0 : nullptr,
+    rc = launch_forces(sys, std::min(W - w0, chunk), walk_from(s, to_walk<double>(wk), w0), RT ? RT + 9 * w0 : nullptr,
                        out, static_cast<double*>(workspace), st);
     if (rc != JQMC_OK) return rc;
   }

@@ -153,9 +153,14 @@ struct FrBuf {
   }
 };
 
-// Walkers a call takes at a time, so that its workspace stays bounded (benzene: 1.1 GB): large enough that every
-// launch fills the chip (a walker has at least one wave of work in each of them).
-constexpr int64_t FR_CHUNK = 4096;
+// Walkers that a call of W takes at a time, so that its workspace stays bounded (benzene: 1.3 GB): at most 2^17
+// electrons, 2048 blocks of the launches over electrons, in parts of equal size.  32768 walkers of N (7 electrons)
+// took 1286 us in parts of 4096 walkers and 797 so, H2 1122 and 459 us (with the waves of k_fr_out below).
+constexpr int64_t FR_ELECTRONS = 1 << 17;
+inline int64_t fr_chunk(const Sys& s, int64_t W) {
+  const int64_t most = FR_ELECTRONS / s.n_el, parts = (W + most - 1) / most;
+  return parts > 0 ? (W + parts - 1) / parts : 0;
+}
 
 // Size bound of the systems taken, in bytes: one walker's vectors of every pass within the LDS of a CU.
 inline int64_t forces_lds_bytes(const Sys& s) {
@@ -1068,12 +1073,13 @@ __global__ void __launch_bounds__(256) k_fr_qbar(FrJob J) {
   }
 }
 
-// One block per walker, its four waves on the 16 x 16 tiles of each product in turn; Gbar and one
+// One block per walker, its waves (fr_pairing_waves) on the 16 x 16 tiles of each product in turn; Gbar and one
 // intermediate (n_up^2 each) in LDS.
+inline int fr_pairing_waves(const Sys& s) { return std::min(FR_WAVES, (s.n_up + 15) / 16 * ((s.n_orb + 15) / 16)); }
 __global__ void __launch_bounds__(256) k_fr_pairing(FrJob J) {
   extern __shared__ double smem[];
   CSys& s = csys(J.sys);
-  const int wave = wave_id(), lane = lane_id(), il = lane & 15, ih = lane >> 4;
+  const int wave = wave_id(), lane = lane_id(), il = lane & 15, ih = lane >> 4, nw = blockDim.x / WAVE;
   const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, no = s.n_orb, un = s.n_unp;
   const int64_t w = blockIdx.x;
   const double* Gi = J.wk.Ginv + w * nu * nu;
@@ -1086,7 +1092,7 @@ __global__ void __launch_bounds__(256) k_fr_pairing(FrJob J) {
   // st(r, c, sum_k fa(r, k) fb(k, c)) over an m x n product of depth d
   auto product = [&](int m, int n, int d, auto fa, auto fb, auto st) {
     const int ct = (n + 15) / 16, tiles = (m + 15) / 16 * ct;
-    for (int x = wave; x < tiles; x += 4) {
+    for (int x = wave; x < tiles; x += nw) {
       const int r0 = x / ct * 16, c0 = (x - x / ct * ct) * 16, r = r0 + il, c = c0 + il;
       const auto acc = mfma_rows(
           d, ih, [&](int k) { return (k < d && r < m) ? fa(r, k) : 0.0; },
@@ -1364,15 +1370,18 @@ struct FrOut {
   int swct;
 };
 
-// One block per walker, lanes = electrons; its four waves share the partners, points and nuclei.
+// One block per walker, lanes = electrons; its waves (fr_out_waves) share the partners, points and nuclei.  Three
+// waves fit a SIMD, so that waves without a partner of their own cost a round: the whole call for 2048 walkers of
+// H2 (2 electrons) 98 us with four waves in this kernel and k_fr_pairing, 89 with one.
+inline int fr_out_waves(const Sys& s) { return std::min(FR_WAVES, (std::max(s.n_el, s.n_nuc) + 3) / 4); }
 __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
   __shared__ double p_sh[FR_WAVES][3][WAVE];
   CSys& s = csys(J.sys);
-  const int wave = wave_id(), lane = lane_id();
+  const int wave = wave_id(), lane = lane_id(), nw = blockDim.x / WAVE;
   const int nu = s.n_up, nd = s.n_dn, ne = s.n_el, nn = s.n_nuc, nv = s.nv;
   const int64_t w = blockIdx.x, M = J.W * ne;
   double* sums = J.part + w * 12 * nn;  // per nucleus: dE/dR, -dln|Psi|/dR, warped parts of both
-  for (int k = threadIdx.x; k < 12 * nn; k += 256) sums[k] = 0.0;
+  for (int k = threadIdx.x; k < 12 * nn; k += blockDim.x) sums[k] = 0.0;
   const CPtr<double> ru = cview(J.wk.r_up) + w * 3 * nu;
   const CPtr<double> rd = cview(J.wk.r_dn) + w * 3 * nd;
   const CPtr<double> el = cview(J.el) + w * ne;
@@ -1400,7 +1409,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
       en[1] += S;
     }
     // e-e pairs: e's own terms and those of its partners together (each is odd in r_e - r_f)
-    for (int f = wave; f < ne; f += FR_WAVES) {
+    for (int f = wave; f < ne; f += nw) {
       const CPtr<double> q = f < nu ? ru + 3 * f : rd + 3 * (f - nu);
       const double ux = ex - q[0], uy = ey - q[1], uz = ez - q[2];
       const double d2 = ux * ux + uy * uy + uz * uz;
@@ -1423,7 +1432,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
     }
     // the other electrons' quadrature points move with r_e through J2
     if (JP.j2_type)
-      for (int j = wave; j < n_ecp; j += FR_WAVES) {
+      for (int j = wave; j < n_ecp; j += nw) {
         const int x = cview(J.elist)[w * ne + j] & 255;
         const CPtr<double> q = cview(J.pt) + (w * ne + j) * (int64_t)nv * 4;
         for (int k = 0; k < nv; ++k) {
@@ -1437,7 +1446,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
         }
       }
     // nuclei
-    for (int n = wave; n < nn; n += FR_WAVES) {
+    for (int n = wave; n < nn; n += nw) {
       const double ux = ex - np[3 * n], uy = ey - np[3 * n + 1], uz = ez - np[3 * n + 2];
       const double d2 = ux * ux + uy * uy + uz * uz, d = sqrt(d2);
       double v[3] = {0.0, 0.0, 0.0}, c = s.nuc_charge[n] / (d2 * d);  // -Z / d
@@ -1469,7 +1478,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       re[c] = p_sh[0][c][lane];
-      for (int q = 1; q < FR_WAVES; ++q) re[c] += p_sh[q][c][lane];
+      for (int q = 1; q < nw; ++q) re[c] += p_sh[q][c][lane];
     }
     if (act && wave == 0) {
 #pragma unroll
@@ -1491,7 +1500,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
         dK[2] += c * uz;
       }
     const double Ki = O.swct ? 1.0 / K : 0.0;
-    for (int n = wave; n < nn; n += FR_WAVES) {
+    for (int n = wave; n < nn; n += nw) {
       double x[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
       if (act) {
 #pragma unroll
@@ -1518,7 +1527,7 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
   wave_sum_k<2>(en);
   if (threadIdx.x == 0 && O.e_L) O.e_L[w] = en[0] + (J.vpot[w] + s.ion_ion) + en[1];
   __syncthreads();
-  for (int k = threadIdx.x; k < 3 * nn; k += 256) {
+  for (int k = threadIdx.x; k < 3 * nn; k += blockDim.x) {
     const int n = k / 3, c = k - 3 * n;
     double F = sums[12 * n + c];
     for (int m = 0; m < nn; ++m) {  // ion-ion repulsion

@@ -93,5 +93,16 @@ def many_walkers(host):
     return out
 
 
+def long_forces(host):
+    """Forces of the most water walkers that are taken at once, and of one more: electrons per launch of the
+    kinetic kernel, and the workspaces of both calls."""
+    from jqmc_amd import synthetic
+
+    pack = host.pack(synthetic.water_ae(0).hamiltonian_data)
+    most = (1 << 17) // 10
+    return [[[r[1] for r in host.position_grads(pack, W) if r[0] == "k_fr_kinetic"],
+             host.bytes("jqmc_position_grads_workspace_bytes", pack, W)] for W in (most, most + 1)]
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[2]](Host(sys.argv[1]))))

@@ -45,13 +45,14 @@ def test_position_grads_match_oracle(name, mos, nv, W):
 
 
 def test_long_call_matches_short_calls():
-    """A call of 4096 + 5 walkers is taken in two parts; every walker's results are those of a short call."""
+    """A call of 13112 walkers of 10 electrons (more than 2^17 electrons) is taken in two parts; every walker's
+    results are those of a short call."""
     from jqmc_amd._api import WalkerState
 
-    W = 4101
+    W = 13112
     _, ws, r_up, r_dn = _state("water_ae", None, 6, W)
     out = ws.position_grads(None)
-    for a, b in ((0, 3), (4094, W)):
+    for a, b in ((0, 3), (6550, 6560), (W - 4, W)):
         sub = WalkerState(ws.pack, b - a).init(r_up[a:b], r_dn[a:b])
         ref = sub.position_grads(None)
         for k, v in ref.items():

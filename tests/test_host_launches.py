@@ -45,3 +45,10 @@ def test_what_the_set_up_takes_is_taken_by_the_other_calls(shim):
     rec = _scenario(shim, "many_walkers")
     assert {"k_init_rows", "k_el_prep", "k_lrdmc_move", "k_dlnpsi_small", "k_rank_narrow"} <= {r[0] for r in rec}
     assert not [r for r in rec if r[-1]]
+
+
+def test_forces_are_taken_in_equal_parts(shim):
+    """One walker more than fit a part does not cost a chain of launches of its own, nor a larger workspace."""
+    (one, b1), (two, b2) = _scenario(shim, "long_forces")
+    assert len(one) == 1 and len(two) == 2 and abs(two[0] - two[1]) <= 1
+    assert b2 == b1
