@@ -269,11 +269,16 @@ inline int64_t cache_bytes(const Sys& s) {
 // G = j1 + S1 J3^T + S2 J3 for the W n_el rows of the prefix sums S1, S2 (k_init_jfield_mfma).
 int launch_jfield_gemm(const Sys& s, int64_t W, const double* S1, const double* S2, const double* j1, double* G,
                        hipStream_t st) {
-  const int64_t n_rt = (W * s.n_el + JG_TILE - 1) / JG_TILE;
+  const int64_t M = W * s.n_el, n_rt = (M + JG_TILE - 1) / JG_TILE;
   const int n_ct = (s.n_ao + JG_TILE - 1) / JG_TILE;
+  if (s.n_ao <= JG_TILE && n_rt < JG_FEW) {
+    const int64_t tiles = (M + 15) / 16 * ((s.n_ao + 15) / 16);
+    k_init_jfield_tile<<<(unsigned)((tiles + 3) / 4), 256, 0, st>>>(s, M, S1, S2, j1, G);
+    return JQMC_OK;
+  }
   const int64_t blocks = (n_rt + 7) / 8 * 8 * n_ct;
   if (blocks > MAX_BLOCKS) return fail(JQMC_ERR_SHAPE, "too many walkers for one launch");
-  k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, W * s.n_el, S1, S2, j1, G, n_ct, n_rt);
+  k_init_jfield_mfma<<<(unsigned)blocks, 256, 0, st>>>(s, M, S1, S2, j1, G, n_ct, n_rt);
   return JQMC_OK;
 }
 

@@ -414,7 +414,7 @@ struct JfMfma<float> {
 // The column tiles of a row tile are eight blocks apart, so they run on one XCD and share the rows in
 // its L2.  512 benzene walkers (15360 x 228): 1389 us with one thread per output and n_ao dependent
 // steps, 98 us as this GEMM (33 TFLOP/s).
-constexpr int JG_TILE = 64, JG_KC = 16;
+constexpr int JG_TILE = 64, JG_KC = 16, JG_FEW = 1024;
 constexpr int JG_A_LD = JG_KC + 1;    // doubles per LDS row of S: 34 banks apart, no conflict over 16 rows
 constexpr int JG_B_LD = JG_TILE + 8;  // the four 16-lane groups read rows 16 banks apart
 
@@ -495,6 +495,51 @@ __global__ void __launch_bounds__(256) k_init_jfield_mfma(Sys s, int64_t M, cons
         const int64_t m = m0 + wr + 16 * x + MF::row(q, ih);
         if (m < M) G[m * na + a] = ja + acc[x][y][q];
       }
+  }
+}
+
+// The same bit for bit with a wave per 16 x 16 tile and the operands straight from L2, for small systems (at most
+// JG_TILE AOs) up to JG_FEW row tiles of the form above, whose slices cost a memory latency each.  The whole set-up
+// of N2 (24 AOs): 64 walkers 49 us with that form and 45 so, 2048 walkers 71 and 68, 8192 (1280 row tiles) 151 and
+// 148; 256 walkers of H2 with 50 AOs 39 and 33.  Many AOs take it worse: 16 walkers of 4 x H2O (300) 289 and 316 us.
+__global__ void __launch_bounds__(256) k_init_jfield_tile(Sys s, int64_t M, const double* __restrict__ S1,
+                                                          const double* __restrict__ S2, const double* __restrict__ j1,
+                                                          double* __restrict__ G) {
+  using MF = JfMfma<double>;
+  const int lane = lane_id(), il = lane & 15, ih = lane >> 4, na = s.n_ao, n_ct = (na + 15) / 16;
+  const int64_t id = (int64_t)blockIdx.x * 4 + wave_id(), m0 = id / n_ct * 16;
+  if (m0 >= M) return;
+  const int a0 = (int)(id % n_ct) * 16, a = a0 + il < na ? a0 + il : na - 1;
+  const bool sym = s.j3_sym != 0, row = m0 + il < M;
+  const int64_t m = row ? m0 + il : M - 1;
+  MF::v4 acc = {0, 0, 0, 0};
+  for (int part = 0; part < (sym ? 1 : 2); ++part) {
+    const double* __restrict__ S = (part ? S2 : S1) + m * na;
+    const double* __restrict__ T = S2 + m * na;
+    const double* __restrict__ J = (part ? s.td.j3 : s.td.j3T) + a;
+    for (int b0 = 0; b0 < na; b0 += 16) {
+      double fa[4], ft[4], fb[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int b = b0 + 4 * x + ih < na ? b0 + 4 * x + ih : na - 1;
+        fa[x] = S[b];
+        ft[x] = sym ? T[b] : 0.0;
+        fb[x] = J[(int64_t)b * na];
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const bool ok = b0 + 4 * x + ih < na;
+        if (sym) fa[x] += ft[x];
+        acc = MF::mma(ok && row ? fa[x] : 0.0, ok ? fb[x] : 0.0, acc);
+      }
+    }
+  }
+  if (a0 + il >= na) return;
+  const double ja = j1 ? j1[a] : 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int64_t r = m0 + MF::row(q, ih);
+    if (r < M) G[r * na + a] = ja + acc[q];
   }
 }
 
