@@ -197,9 +197,9 @@ __global__ void k_init_geminal(Sys s, int64_t W, WalkT<T> wk) {
 __device__ inline void wave_gauss_jordan(double* M, double* I, int n, int lane, double& logabs_out, double& sgn_out) {
   double logabs = 0.0, sgn = 1.0;
   for (int k = 0; k < n; ++k) {
-    // pivot search: lane i holds |M[i][k]| for i >= k
+    // pivot search: lane i holds |M[i][k]| for i >= k; row k when no element is a number
     double best = -1.0;
-    int bi = n;
+    int bi = k;
     for (int i = k + lane; i < n; i += WAVE) {
       const double v = fabs(M[i * n + k]);
       if (v > best) {

@@ -95,3 +95,27 @@ def test_coincident_particles_have_no_finite_energy(name):
         assert not torch.isfinite(g["force_HF"][w]).all()
     if ham.coulomb_potential_data.ecp_flag:  # the quadrature of that electron has no direction: nothing of it is finite
         assert not torch.isfinite(g["dE_dr"][3]).any()
+
+
+@pytest.mark.parametrize("name", ["water_ae", "chain10"])
+def test_singular_walkers_leave_their_neighbours_alone(name):
+    """A dn electron where every AO has underflowed makes a column of G zero, and the elimination then meets columns
+    without a number: no row outside the matrix is taken as the pivot, so the walkers of the same block keep their
+    bits."""
+    from jqmc_amd import synthetic
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+
+    system = synthetic.chain_ecp(10, 1) if name == "chain10" else synthetic.water_ae(0)
+    pack = SystemPack(system.hamiltonian_data)
+    r_up, r_dn = system.initial_walkers(8, seed=5)
+    plain = WalkerState(pack, 8).init(r_up, r_dn)
+    e0 = plain.local_energy(plain.rotations(3, 0))
+    r_dn[2, 0] = r_dn[5, 1] = [1.0e4, 0.0, 0.0]
+    ws = WalkerState(pack, 8).init(r_up, r_dn)
+    e = ws.local_energy(ws.rotations(3, 0))
+    keep = [0, 1, 3, 4, 6, 7]
+    for key in ("Ginv", "logabsdet", "sign", "as_factor"):
+        assert torch.equal(getattr(ws, key)[keep], getattr(plain, key)[keep]), key
+    assert torch.equal(e[keep], e0[keep])
+    assert not torch.isfinite(ws.Ginv[2]).all() and not torch.isfinite(ws.Ginv[5]).all()
