@@ -540,6 +540,7 @@ template <typename T>
 int launch_local_energy(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, const double* RT, double* e_L,
                         double* kinetic, double* v_total, double* t_elec, void* workspace, hipStream_t st) {
   const Sys& s = sys->s;
+  // the limit of the guard's team form; it stands for plain FP64 too, so that what is refused does not change
   if (el2_lds_bytes(s) > kMaxLdsPerBlock) return fail(JQMC_ERR_UNSUPPORTED, "system too large for the E_L LDS budget");
   const WalkT<T> k = to_walk<T>(wk);
   const ElWs ws = el_ws(s, W, workspace);
@@ -763,7 +764,7 @@ int launch_lrdmc(const jqmc_system* sys, int64_t W, const jqmc_walkers* wk, cons
                  hipStream_t st) {
   const Sys& s = sys->s;
   const int64_t per_move = lr_move_lds_bytes<T>(s);
-  if (std::max(lr_ham_lds_bytes<T>(s), per_move) > kMaxLdsPerBlock)
+  if (std::max(lr_ham_lds_bytes(s), per_move) > kMaxLdsPerBlock)
     return fail(JQMC_ERR_UNSUPPORTED, "system too large for the LRDMC LDS budget");
   const int wpb_m = walkers_per_block(per_move);
   const WalkT<T> k = to_walk<T>(wk);
@@ -1544,7 +1545,7 @@ int jqmc_lrdmc_projection_multi(int32_t n_sys, const jqmc_system* const* systems
     if (W[k] > 0 && (!workspaces[k] || workspace_bytes[k] < lr_ws_bytes(sys->s, W[k])))
       return fail(JQMC_ERR_WORKSPACE, "workspace %d: %lld bytes required", k, (long long)lr_ws_bytes(sys->s, W[k]));
     const bool mixed = prec == JQMC_PRECISION_MIXED_FP32;
-    const int64_t per_ham = lr_ham_lds_bytes<double>(sys->s);
+    const int64_t per_ham = lr_ham_lds_bytes(sys->s);
     const int64_t per_move = mixed ? lr_move_lds_bytes<float>(sys->s) : lr_move_lds_bytes<double>(sys->s);
     if (std::max(per_ham, per_move) > kMaxLdsPerBlock)
       return fail(JQMC_ERR_UNSUPPORTED, "system %d too large for the LRDMC LDS budget", k);

@@ -1,5 +1,5 @@
-// Local energy of single walkers by teams of waves: the FP64 guard of the mixed form (the flattened
-// launches of jqmc_elp.hip evaluate whole walker sets).
+// Local energy of single walkers in FP64, a block of several waves each: the guard of the mixed form (the
+// flattened launches of jqmc_elp.hip evaluate whole walker sets).
 //
 // compute_local_energy_fast (hamiltonians.py:225-290) per walker, in phases whose lanes own the items
 // that are independent:
@@ -7,8 +7,8 @@
 //   1. positions, G^-1 and the rotated quadrature mesh into LDS;
 //   2. q_e = [M | Lambda_u] G^-1[:, e] (up) or M' G^-1[e, :]^T (dn) for every electron (lanes own
 //      (electron, orbital) pairs) into LDS;
-//   3. the determinant fields h_e = C^T q_e of every electron (lanes own AOs) into the per-walker
-//      workspace rows hws[w][e][:] (FP64);
+//   3. the determinant fields h_e = C^T q_e of every electron (lanes own AOs) into the guard slot's
+//      rows;
 //   4. the continuum kinetic energy T_e (wavefunction.py:1141-1207) with the lanes owning electrons:
 //      the AO value / gradient / Laplacian at r_e shell after shell, the shell and AO tables read at
 //      wave-uniform indices (scalar loads), dotted with h_e and the J3 field g_e, plus the J1 / J2
@@ -18,8 +18,8 @@
 //   6. the non-local ECP (NN = 1, coulomb_potential.py:1477-1712) with the lanes owning the
 //      quadrature points of all listed electrons, 64 at a time: each lane builds its point and
 //      projector weight, the J1 / J2 change, and runs the AO basis shell after shell with uniform
-//      table reads, accumulating a(r') . h_e (determinant ratio, FP64) and a(r') . g_e (in T), whose
-//      difference from c_e is the J3 log-ratio;
+//      table reads, accumulating a(r') . h_e (determinant ratio) and a(r') . g_e, whose difference
+//      from c_e is the J3 log-ratio;
 //   7. bare Coulomb and the local ECP part (coulomb_potential.py:1144-1246, 2252-2281).
 //
 // No lane idles on a per-AO table lookup: the AO tables sit behind a constant-address-space view,
@@ -42,39 +42,29 @@ __device__ __forceinline__ CPtr<U> cview(const U* p) {
   return (CPtr<U>)p;
 }
 
-// The threads that evaluate one walker: NW wavefronts.  NW = 1: one wavefront of a block that may
-// hold several walkers (wave_sync is its barrier); NW > 1: the whole block (__syncthreads).  Loops
-// over independent items start at tid and stride by N; sum() and sum_k() reduce over the team in a
-// fixed order (the butterfly of each wave, then the waves in order through the LDS words red,
-// NW * 8 doubles), so every thread gets the bitwise-identical total.  With NW = 1 every phase below
-// runs the same operations in the same order as a plain one-wavefront loop.
+// The threads that evaluate one walker: the NW > 1 wavefronts of a block.  Loops over independent items start at
+// tid and stride by N; sum() and sum_k() reduce over the team in a fixed order (the butterfly of each wave, then
+// the waves in order through the LDS words red, NW * 8 doubles), so every thread gets the bitwise-identical total.
 template <int NW>
 struct Team {
+  static_assert(NW > 1);
   static constexpr int N = WAVE * NW;
   int tid, wid, lane;
   double* red;
-  __device__ __forceinline__ void sync() const {
-    if constexpr (NW == 1)
-      wave_sync();
-    else
-      __syncthreads();
-  }
   template <int K>
   __device__ __forceinline__ void sum_k(double* v) const {
     wave_sum_k<K>(v);
-    if constexpr (NW > 1) {
-      if (lane == 0)
+    if (lane == 0)
 #pragma unroll
-        for (int k = 0; k < K; ++k) red[wid * 8 + k] = v[k];
-      __syncthreads();
+      for (int k = 0; k < K; ++k) red[wid * 8 + k] = v[k];
+    __syncthreads();
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        double t = red[k];
-        for (int q = 1; q < NW; ++q) t += red[q * 8 + k];
-        v[k] = t;
-      }
-      __syncthreads();
+    for (int k = 0; k < K; ++k) {
+      double t = red[k];
+      for (int q = 1; q < NW; ++q) t += red[q * 8 + k];
+      v[k] = t;
     }
+    __syncthreads();
   }
   __device__ __forceinline__ double sum(double x) const {
     double v[1] = {x};
@@ -83,8 +73,6 @@ struct Team {
   }
 };
 
-// The one-wavefront team of lane `lane`.
-
 // The q_e rows of all electrons stay in LDS when they take at most EL2_Q_LDS bytes, otherwise they
 // go to the workspace after the h_e rows (large AO-orbital geminals).
 constexpr int64_t EL2_Q_LDS = 16 * 1024;
@@ -92,8 +80,8 @@ __host__ __device__ inline bool el2_q_in_lds(const Sys& s) {
   return (int64_t)s.n_el * s.n_orb * (int64_t)sizeof(double) <= EL2_Q_LDS;
 }
 
-// LDS of one walker of the guard's local energy (one wavefront; nw > 1: a team of nw wavefronts, which
-// also needs the reduction words red and the per-wave kinetic partials kred).
+// LDS of one walker of the guard's local energy (nw > 1: with the reduction words red and the per-wave kinetic
+// partials kred of a team of nw wavefronts; nw = 1, the walker alone, is the size limit of el2_lds_bytes).
 struct El2Lds {
   double *rr, *Gi, *RT, *gk, *Q, *en, *Vt, *jold, *te, *jc, *red, *kred;
   int* elist;
@@ -156,22 +144,21 @@ __device__ __forceinline__ void cart_vgl(double dx, double dy, double dz, double
 
 // Value of the monomial or term sum of AO a (meta word m) at (dx, dy, dz), tables read at the
 // wave-uniform index a.
-template <typename U>
-__device__ __forceinline__ U poly_uniform(const Sys& s, int a, int m, U dx, U dy, U dz) {
+__device__ __forceinline__ double poly_uniform(const Sys& s, int a, int m, double dx, double dy, double dz) {
   if (m & AO_UNIT_TERM) return ipow(dx, (m >> 16) & 15) * ipow(dy, (m >> 20) & 15) * ipow(dz, (m >> 24) & 15);
   const CPtr<int> tp = cview(s.ao_tp);
   const CPtr<int> pw = cview(s.term_pow);
-  const CPtr<U> tc = cview(tabs<U>(s).term_coef);
-  U P = 0;
+  const CPtr<double> tc = cview(s.td.term_coef);
+  double P = 0.0;
   const int t1 = tp[a + 1];
   for (int t = tp[a]; t < t1; ++t) P += tc[t] * (ipow(dx, pw[3 * t]) * ipow(dy, pw[3 * t + 1]) * ipow(dz, pw[3 * t + 2]));
   return P;
 }
 
-// ---- the phases, each run by the whole wavefront of one walker
+// ---- the phases, each run by the whole team
 
 // 1. positions, G^-1 and the rotation RTw (NULL: identity) into LDS; the rotated mesh when the system
-// has non-local terms (read after the next wave_sync).
+// has non-local terms (read after the next barrier).
 template <int NW>
 __device__ __forceinline__ void el_load_walker(const Sys& s, const double* __restrict__ r_up,
                                                const double* __restrict__ r_dn, const double* __restrict__ Giw,
@@ -181,7 +168,7 @@ __device__ __forceinline__ void el_load_walker(const Sys& s, const double* __res
   for (int k = i; k < 3 * nd; k += tm.N) L.rr[3 * nu + k] = r_dn[k];
   for (int k = i; k < nu * nu; k += tm.N) L.Gi[k] = Giw[k];
   if (i < 9) L.RT[i] = RTw ? RTw[i] : ((i % 4) == 0 ? 1.0 : 0.0);
-  tm.sync();
+  __syncthreads();
   if (s.ecp_on && s.nv > 0) rotate_mesh(s, L.RT, L.gk, i, tm.N);
 }
 
@@ -207,7 +194,7 @@ __device__ __forceinline__ void el_det_fields_rows(const Sys& s, const El2Lds& L
     }
     Qr[t] = acc;
   }
-  tm.sync();
+  __syncthreads();
 
   // the lane's AO column of C held in registers for the first KC orbitals, up block with C_up, dn
   // block with C_dn
@@ -235,7 +222,7 @@ __device__ __forceinline__ void el_det_fields_rows(const Sys& s, const El2Lds& L
       }
     }
   }
-  tm.sync();
+  __syncthreads();
 }
 
 // The q rows in LDS when they fit (el2_q_in_lds), else in the workspace rows Qg; each branch keeps
@@ -252,13 +239,12 @@ __device__ __forceinline__ void el_det_fields(const Sys& s, const El2Lds& L, con
 // 4. the continuum kinetic energy T_e (wavefunction.py:1141-1207) with the lanes owning electrons:
 // AO value / gradient / Laplacian at r_e shell after shell, dotted with h_e (Hw) and the J3 field
 // g_e (gw, NULL without J3), plus the J1 / J2 gradients and Laplacians.  T_e goes to L.te and to
-// t_elec_w when given; c_e = a(r_e) . g_e (FP64 AO values) to L.jc, the J3 term that the point
-// ratios subtract.  Returns the walker's kinetic energy on every thread.  A team of NW > 1 waves
-// splits the shells (wave w takes shells w, w + NW, ...) and the J2 partners among its waves, all
+// t_elec_w when given; c_e = a(r_e) . g_e to L.jc, the J3 term that the point ratios subtract.
+// Returns the walker's kinetic energy on every thread.  The team splits the shells (wave w takes shells w, w + NW, ...) and the J2 partners among its waves, all
 // waves holding the same electrons in their lanes; the nine partial sums per electron are added in
 // wave order through L.kred, and wave 0 forms T_e.
-template <typename TC, int NW>
-__device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __restrict__ Hw, const TC* gw,
+template <int NW>
+__device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __restrict__ Hw, const double* gw,
                              const Team<NW>& tm, double* t_elec_w) {
   const int lane = tm.lane;
   const int ne = s.n_el, na = s.n_ao, nsh = s.n_shell;
@@ -276,7 +262,7 @@ __device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __rest
     const int ec = act ? e : 0;
     const double ex = L.rr[3 * ec], ey = L.rr[3 * ec + 1], ez = L.rr[3 * ec + 2];
     const double* hrow = Hw + (int64_t)ec * na;
-    const TC* grow = gw ? gw + (int64_t)ec * na : nullptr;
+    const double* grow = gw ? gw + (int64_t)ec * na : nullptr;
     double acc8[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // gJ(3), lapJ, gD(3), lapD'
     double jc = 0.0;
     // per AO: value P, gradient and Laplacian of the angular part, the contributions to the fields
@@ -286,7 +272,7 @@ __device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __rest
                    g2 = f * (nr * Pz - 2.0 * dz * znr * P);
       const double lp = f * (nr * lapP - 4.0 * znr * rdg + (4.0 * r2 * z2nr - 6.0 * znr) * P);
       if (grow) {
-        const double gj = (double)grow[a];
+        const double gj = grow[a];
         acc8[0] += gj * g0;
         acc8[1] += gj * g1;
         acc8[2] += gj * g2;
@@ -417,20 +403,18 @@ __device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __rest
                     acc8[1], acc8[2], acc8[3]);
       }
     }
-    if constexpr (NW > 1) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) L.kred[(tm.wid * 9 + k) * WAVE + lane] = acc8[k];
-      L.kred[(tm.wid * 9 + 8) * WAVE + lane] = jc;
-      __syncthreads();
-      if (tm.wid == 0) {
-        for (int q = 1; q < NW; ++q) {
+    for (int k = 0; k < 8; ++k) L.kred[(tm.wid * 9 + k) * WAVE + lane] = acc8[k];
+    L.kred[(tm.wid * 9 + 8) * WAVE + lane] = jc;
+    __syncthreads();
+    if (tm.wid == 0) {
+      for (int q = 1; q < NW; ++q) {
 #pragma unroll
-          for (int k = 0; k < 8; ++k) acc8[k] += L.kred[(q * 9 + k) * WAVE + lane];
-          jc += L.kred[(q * 9 + 8) * WAVE + lane];
-        }
+        for (int k = 0; k < 8; ++k) acc8[k] += L.kred[(q * 9 + k) * WAVE + lane];
+        jc += L.kred[(q * 9 + 8) * WAVE + lane];
       }
-      __syncthreads();
     }
+    __syncthreads();
     const double gDx = acc8[4], gDy = acc8[5], gDz = acc8[6];
     const double lapD = acc8[7] - (gDx * gDx + gDy * gDy + gDz * gDz);
     const double tx = acc8[0] + gDx, ty = acc8[1] + gDy, tz = acc8[2] + gDz;
@@ -445,15 +429,13 @@ __device__ double el_kinetic(const Sys& s, const El2Lds& L, const double* __rest
   return tm.sum(kinetic);
 }
 
-// 5. per electron the nearest nucleus n, R - r_e and |R - r_e| (L.en) and the projector radial
-// factors V_t of its projected terms (L.Vt) when the system has non-local terms, and the J1 + J2
-// value at r_e (L.jold) for every electron when all_jold, else for the electrons with projected
-// terms.  Those electrons are listed in electron order in L.elist; returns their count on every
-// thread (the list is valid after the next team sync).
+// 5. per electron the nearest nucleus n, R - r_e and |R - r_e| (L.en), the projector radial factors V_t of
+// its projected terms (L.Vt) and, where it has any, the J1 + J2 value at r_e (L.jold).  Those electrons
+// are listed in electron order in L.elist; returns their count on every thread (the list is valid after
+// the next barrier).
 template <int NW>
-__device__ int el_ecp_electrons(const Sys& s, const El2Lds& L, const Team<NW>& tm, bool all_jold) {
+__device__ int el_ecp_electrons(const Sys& s, const El2Lds& L, const Team<NW>& tm) {
   const int ne = s.n_el, lane = tm.lane;
-  const bool nonlocal = s.ecp_on && s.nv > 0;
   const int mt = s.ecp_max_terms > 0 ? s.ecp_max_terms : 1;
   int n_ecp = 0;
   for (int e0 = 0; e0 < ne; e0 += tm.N) {
@@ -461,27 +443,25 @@ __device__ int el_ecp_electrons(const Sys& s, const El2Lds& L, const Team<NW>& t
     bool has = false;
     if (e < ne) {
       const double x = L.rr[3 * e], y = L.rr[3 * e + 1], z = L.rr[3 * e + 2];
-      if (nonlocal) {
-        EcpElec E;
-        E.n = nearest_nucleus(s, x, y, z);
-        E.nt = s.ecp_nt[E.n];
-        E.rx = s.nuc_pos[3 * E.n] - x;
-        E.ry = s.nuc_pos[3 * E.n + 1] - y;
-        E.rz = s.nuc_pos[3 * E.n + 2] - z;
-        E.rn = sqrt(E.rx * E.rx + E.ry * E.ry + E.rz * E.rz);
-        has = E.nt > 0;
-        L.en[5 * e] = (double)E.n;
-        L.en[5 * e + 1] = E.rx;
-        L.en[5 * e + 2] = E.ry;
-        L.en[5 * e + 3] = E.rz;
-        L.en[5 * e + 4] = E.rn;
-        for (int t = 0; t < E.nt; ++t) {
-          const int o = E.n * s.ecp_max_terms + t;
-          L.Vt[e * mt + t] =
-              (1.0 / (E.rn * E.rn)) * s.ecp_coef[o] * rpow(E.rn, s.ecp_pow[o]) * exp_nonpos(-s.ecp_exp[o] * (E.rn * E.rn));
-        }
+      EcpElec E;
+      E.n = nearest_nucleus(s, x, y, z);
+      E.nt = s.ecp_nt[E.n];
+      E.rx = s.nuc_pos[3 * E.n] - x;
+      E.ry = s.nuc_pos[3 * E.n + 1] - y;
+      E.rz = s.nuc_pos[3 * E.n + 2] - z;
+      E.rn = sqrt(E.rx * E.rx + E.ry * E.ry + E.rz * E.rz);
+      has = E.nt > 0;
+      L.en[5 * e] = (double)E.n;
+      L.en[5 * e + 1] = E.rx;
+      L.en[5 * e + 2] = E.ry;
+      L.en[5 * e + 3] = E.rz;
+      L.en[5 * e + 4] = E.rn;
+      for (int t = 0; t < E.nt; ++t) {
+        const int o = E.n * s.ecp_max_terms + t;
+        L.Vt[e * mt + t] =
+            (1.0 / (E.rn * E.rn)) * s.ecp_coef[o] * rpow(E.rn, s.ecp_pow[o]) * exp_nonpos(-s.ecp_exp[o] * (E.rn * E.rn));
       }
-      if (has || all_jold) {
+      if (has) {
         double old = 0.0;
         if (s.j2_type) {
           for (int f = 0; f < ne; ++f) {
@@ -495,19 +475,16 @@ __device__ int el_ecp_electrons(const Sys& s, const El2Lds& L, const Team<NW>& t
       }
     }
     const uint64_t mask = __ballot(has);
-    int before = 0, total = __popcll(mask);
-    if constexpr (NW > 1) {
-      // the waves' counts in order: this wave's offset and the round's total
-      if (lane == 0) L.red[tm.wid] = (double)total;
-      __syncthreads();
-      total = 0;
-      for (int q = 0; q < NW; ++q) {
-        const int c = (int)L.red[q];
-        before += q < tm.wid ? c : 0;
-        total += c;
-      }
-      __syncthreads();
+    // the waves' counts in order: this wave's offset and the round's total
+    if (lane == 0) L.red[tm.wid] = (double)__popcll(mask);
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int q = 0; q < NW; ++q) {
+      const int c = (int)L.red[q];
+      before += q < tm.wid ? c : 0;
+      total += c;
     }
+    __syncthreads();
     const int rank = n_ecp + before + __popcll(mask & ((1ull << lane) - 1ull));
     if (has) L.elist[rank] = e;
     n_ecp += total;
@@ -540,43 +517,42 @@ __device__ __forceinline__ void el_ecp_point(const Sys& s, const El2Lds& L, int 
 }
 
 // One fast shell (np primitives, canonical Cartesian AOs of angular momentum L) at a point (dx, dy, dz
-// from its centre, r2 = |.|^2): its AO values dotted into det (with the field row h, FP64) and dj3 (with
-// the J3 field row g, in T).  The record words are read unconditionally, so that they arrive with a
+// from its centre, r2 = |.|^2): its AO values dotted into det (with the field row h) and dj3 (with the
+// J3 field row g).  The record words are read unconditionally, so that they arrive with a
 // few wide loads and one wait.
-template <typename T, typename TC, int L>
-__device__ __forceinline__ void point_shell(const CPtr<double> rec, int np, T dx, T dy, T dz, T r2,
-                                            const double* __restrict__ h, const TC* g, double& det, T& dj3) {
+template <int L>
+__device__ __forceinline__ void point_shell(const CPtr<double> rec, int np, double dx, double dy, double dz, double r2,
+                                            const double* __restrict__ h, const double* g, double& det, double& dj3) {
   constexpr int NA = Cart<L>::N;
   double w[2 * SHR_PMAX], sc[NA], hv[NA];
-  TC gv[NA];
+  double gv[NA];
 #pragma unroll
   for (int k = 0; k < 2 * SHR_PMAX; ++k) w[k] = rec[SHR_P + k];
 #pragma unroll
   for (int k = 0; k < NA; ++k) {
     sc[k] = rec[SHR_SC + k];
     hv[k] = h[k];
-    gv[k] = g ? g[k] : (TC)0;
+    gv[k] = g ? g[k] : 0.0;
   }
-  T nr = 0;
+  double nr = 0;
 #pragma unroll
   for (int q = 0; q < SHR_PMAX; ++q)
-    if (q < np) nr += (T)w[2 * q + 1] * exp_nonpos(-(T)w[2 * q] * r2);
+    if (q < np) nr += w[2 * q + 1] * exp_nonpos(-w[2 * q] * r2);
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
-    const T P = cpow(Cart<L>::nx(i), dx) * cpow(Cart<L>::ny(i), dy) * cpow(Cart<L>::nz(i), dz);
-    const T v = (T)sc[i] * (nr * P);
-    det += (double)v * hv[i];
-    if (g) dj3 += v * (T)gv[i];
+    const double P = cpow(Cart<L>::nx(i), dx) * cpow(Cart<L>::ny(i), dy) * cpow(Cart<L>::nz(i), dz);
+    const double v = sc[i] * (nr * P);
+    det += v * hv[i];
+    if (g) dj3 += v * gv[i];
   }
 }
 
 // Electron e moved to (px, py, pz), every other electron in place: the determinant ratio
-// a(r') . h_e (FP64) and the log Jastrow ratio a(r') . g_e - c_e (J3, the AO values at r' in T) +
+// a(r') . h_e and the log Jastrow ratio a(r') . g_e - c_e (J3) +
 // J1 + J2 at r' - L.jold[e].  Each lane has its own point; the AO basis runs shell after shell with
 // the tables read at wave-uniform indices.
-template <typename T, typename TC>
 __device__ __forceinline__ void el_point(const Sys& s, const El2Lds& L, int e, double px, double py, double pz,
-                                         const double* __restrict__ Hw, const TC* gw, double& det_out,
+                                         const double* __restrict__ Hw, const double* gw, double& det_out,
                                          double& dj_out) {
   const int ne = s.n_el, na = s.n_ao, nsh = s.n_shell;
   double jn = 0.0;
@@ -591,51 +567,51 @@ __device__ __forceinline__ void el_point(const Sys& s, const El2Lds& L, int e, d
   const CPtr<int> sh0 = cview(s.sh_ao0);
   const CPtr<int> app = cview(s.ao_pp);
   const CPtr<int> meta = cview(s.ao_meta);
-  const RealTabs<T>& R = tabs<T>(s);
-  const CPtr<T> pz_ = cview(R.prim_exp);
-  const CPtr<T> pc = cview(R.prim_coef);
-  const CPtr<T> sc = cview(R.ao_scale);
+  const RealTabs<double>& R = s.td;
+  const CPtr<double> pz_ = cview(R.prim_exp);
+  const CPtr<double> pc = cview(R.prim_coef);
+  const CPtr<double> sc = cview(R.ao_scale);
   const double* hrow = Hw + (int64_t)e * na;
-  const TC* grow = gw ? gw + (int64_t)e * na : nullptr;
+  const double* grow = gw ? gw + (int64_t)e * na : nullptr;
   const CPtr<double> shr = cview(s.shrec);
   double det = 0.0;
-  T dj3 = 0;
+  double dj3 = 0;
   for (int sh = 0; sh < nsh; ++sh) {
     const CPtr<double> rec = shr + (int64_t)sh * SHREC;
     const int info = (int)rec[3];
     const int a0 = info >> 9;
-    const T dx = (T)(px - rec[0]), dy = (T)(py - rec[1]), dz = (T)(pz - rec[2]);
-    const T r2 = dx * dx + dy * dy + dz * dz;
-    T nr = 0;
+    const double dx = px - rec[0], dy = py - rec[1], dz = pz - rec[2];
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    double nr = 0;
     if (info & 256) {
       // fast shell: every table word from the record
       const int np = info & 15, l = (info >> 4) & 15;
-      const TC* gs = grow ? grow + a0 : nullptr;
+      const double* gs = grow ? grow + a0 : nullptr;
       if (l == 0)
-        point_shell<T, TC, 0>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
+        point_shell<0>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
       else if (l == 1)
-        point_shell<T, TC, 1>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
+        point_shell<1>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
       else
-        point_shell<T, TC, 2>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
+        point_shell<2>(rec, np, dx, dy, dz, r2, hrow + a0, gs, det, dj3);
       continue;
     }
     const int a1 = sh0[sh + 1];
     const int p1 = app[a0 + 1];
     for (int p = app[a0]; p < p1; ++p) nr += pc[p] * exp_nonpos(-pz_[p] * r2);
     for (int a = a0; a < a1; ++a) {
-      const T v = sc[a] * (nr * poly_uniform<T>(s, a, meta[a], dx, dy, dz));
-      det += (double)v * hrow[a];
-      if (grow) dj3 += v * (T)grow[a];
+      const double v = sc[a] * (nr * poly_uniform(s, a, meta[a], dx, dy, dz));
+      det += v * hrow[a];
+      if (grow) dj3 += v * grow[a];
     }
   }
   det_out = det;
-  dj_out = (grow ? (double)dj3 - L.jc[e] : 0.0) + (jn - L.jold[e]);
+  dj_out = (grow ? dj3 - L.jc[e] : 0.0) + (jn - L.jold[e]);
 }
 
 // 6. the non-local ECP (NN = 1, coulomb_potential.py:1477-1712) with the lanes owning the quadrature
 // points of the n_ecp listed electrons, 64 at a time.  Returns the lane's partial sum.
-template <typename T, typename TC, int NW>
-__device__ double el_nonlocal(const Sys& s, const El2Lds& L, int n_ecp, const double* __restrict__ Hw, const TC* gw,
+template <int NW>
+__device__ double el_nonlocal(const Sys& s, const El2Lds& L, int n_ecp, const double* __restrict__ Hw, const double* gw,
                               const Team<NW>& tm) {
   const int nv = s.nv, lane = tm.lane;
   const int P = n_ecp * nv;
@@ -647,7 +623,7 @@ __device__ double el_nonlocal(const Sys& s, const El2Lds& L, int n_ecp, const do
     const int e = L.elist[ie];
     double px, py, pz, pwt, det, dj;
     el_ecp_point(s, L, e, k, px, py, pz, pwt);
-    el_point<T, TC>(s, L, e, px, py, pz, Hw, gw, det, dj);
+    el_point(s, L, e, px, py, pz, Hw, gw, det, dj);
     vnl += valid ? pwt * (det * exp(dj)) : 0.0;
   }
   return vnl;
@@ -671,25 +647,24 @@ __device__ __forceinline__ double el_potential_partial(const Sys& s, const El2Ld
 }
 
 // The local energy of one walker by one team (phases 1-7 above).  Inputs: the walker's positions
-// r_up / r_dn, G^-1 (Giw), pair rows (Qw), J3 fields (gw, NULL without J3) in the cache type TC, its
-// rotation RTw (NULL: identity); workspace rows Hw (N x n_ao doubles) and, when the q rows do not fit
-// LDS, Qg (N x n_orb doubles).  T is the arithmetic type of the AO values at the quadrature points.
-// Returns kinetic and potential energy on every thread; the per-electron kinetic energies go to
-// t_elec_w when given.  A team of NW waves shares the walker's shells (kinetic phase) and its
-// quadrature points (non-local phase, 64-point rounds dealt to the waves in turn).
-template <typename T, typename TC, int NW>
+// r_up / r_dn, G^-1 (Giw), pair rows (Qw), J3 fields (gw, NULL without J3), its rotation RTw (NULL:
+// identity); workspace rows Hw (N x n_ao doubles) and, when the q rows do not fit LDS, Qg (N x n_orb
+// doubles).  Returns kinetic and potential energy on every thread; the per-electron kinetic energies go
+// to t_elec_w when given.  The waves share the walker's shells (kinetic phase) and its quadrature points
+// (non-local phase, 64-point rounds dealt to the waves in turn).
+template <int NW>
 __device__ void el_pts_walker(const Sys& s, const double* __restrict__ r_up, const double* __restrict__ r_dn,
-                              const double* __restrict__ Giw, const double* __restrict__ Qw, const TC* gw,
+                              const double* __restrict__ Giw, const double* __restrict__ Qw, const double* gw,
                               const double* __restrict__ RTw, double* Hw, double* Qg, const El2Lds& L,
                               const Team<NW>& tm, double* t_elec_w, double& kinetic_out, double& pot_out) {
   el_load_walker(s, r_up, r_dn, Giw, RTw, L, tm);
   el_det_fields(s, L, Qw, Qg, Hw, tm);
-  kinetic_out = el_kinetic<TC>(s, L, Hw, gw, tm, t_elec_w);
+  kinetic_out = el_kinetic(s, L, Hw, gw, tm, t_elec_w);
   double vnl = 0.0;
   if (s.ecp_on && s.nv > 0) {
-    const int n_ecp = el_ecp_electrons(s, L, tm, false);
-    tm.sync();
-    vnl = el_nonlocal<T, TC>(s, L, n_ecp, Hw, gw, tm);
+    const int n_ecp = el_ecp_electrons(s, L, tm);
+    __syncthreads();
+    vnl = el_nonlocal(s, L, n_ecp, Hw, gw, tm);
   }
   double red[2] = {el_potential_partial(s, L, tm), vnl};
   tm.template sum_k<2>(red);
@@ -740,7 +715,7 @@ __global__ void k_zero_int(int* p) {
 
 // The walkers listed by k_el_final<float> recomputed entirely in FP64 from their positions:
 // AO values at the electrons, orbital and pair rows, G and G^-1 (wave_gauss_jordan), the J3 fields
-// (jastrow_factor.py:4121-4135) from the products A J3 and A J3^T, then el_pts_walker<double, double>;
+// (jastrow_factor.py:4121-4135) from the products A J3 and A J3^T, then el_pts_walker;
 // e_L (and the optional parts) of those walkers are overwritten.  The GT / 64 waves of a block share
 // the AO, orbital, pair, G and J3-field work and, as one team, the local energy; the first wave runs
 // the inversion.  The pass takes as long as one walker's recomputation, so the host launches the
@@ -850,7 +825,7 @@ __global__ void __launch_bounds__(GT) k_local_energy_guard(Sys s, int64_t W, Wal
     }
     __syncthreads();
     double kin, pot;
-    el_pts_walker<double, double>(s, ru, rd, R.I, R.pair, s.j3_on ? R.g : nullptr, RTall ? RTall + 9 * w : nullptr,
+    el_pts_walker(s, ru, rd, R.I, R.pair, s.j3_on ? R.g : nullptr, RTall ? RTall + 9 * w : nullptr,
                                   R.H, R.Q, L, tm,
                                   t_elec ? t_elec + w * ne : nullptr, kin, pot);
     if (t == 0) {

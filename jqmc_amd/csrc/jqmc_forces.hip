@@ -162,7 +162,9 @@ inline int64_t fr_chunk(const Sys& s, int64_t W) {
   return parts > 0 ? (W + parts - 1) / parts : 0;
 }
 
-// Size bound of the systems taken, in bytes: one walker's vectors of every pass within the LDS of a CU.
+// Size limit of the systems taken, in bytes: one walker's vectors of every pass within 64 KiB, as one wave per
+// walker would hold them in LDS.  No launch needs this much (k_fr_pairing 16 n_up^2 bytes, at most 64 KiB with
+// n_up <= 64; the others fixed tiles); the limit stands, so that what is refused does not change.
 inline int64_t forces_lds_bytes(const Sys& s) {
   const int64_t ne = s.n_el, nv = std::max(s.nv, 1), na = s.n_ao, no = s.n_orb, nu = s.n_up, nn = s.n_nuc;
   return 8 * (6 * ne + nu * nu + 9 + 14 * nv + std::max(s.ecp_max_terms, 1) + no + 8 * na + std::max(no, nu) + 6 * nn +

@@ -101,8 +101,9 @@ inline LrState lr_state(const Sys& s, int64_t W, double* base) {
   return S;
 }
 
-// Size limit of a system: one walker's local-energy block of the guard's team form and its candidates.
-template <typename T>
+// Size limit of the systems that LRDMC takes: one walker's block of the guard's local energy and its candidates
+// within 64 KiB.  No launch needs this LDS any more (the candidates are in the workspace); the limit stands, so
+// that what is refused does not change.
 inline int64_t lr_ham_lds_bytes(const Sys& s) {
   return el2_lds_bytes(s) + 8 * (lr_cmax(s) > 0 ? lr_cmax(s) : 1);
 }
