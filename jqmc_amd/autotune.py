@@ -2,10 +2,10 @@
 
 The walkers per block of the move-synchronous proposal kernel are chosen per system by timing every
 candidate on the caller's walker count, on scratch walkers built at the caller's positions, so the
-caller's chain does not move.  The two knobs of the E_L kernel are timed and set along with it; the
-local energy runs over the electrons and points of all walkers and does not depend on them.  No knob
-(jqmc_system_set_tuning) changes a result bit (tests/test_gpu_autotune.py checks).  The reference
-has no counterpart (XLA picks its own launch shapes).
+caller's chain does not move.  The choice changes no result bit (tests/test_gpu_autotune.py checks).
+The two knobs of the local energy (``el_*``) can still be set and read back, and stand in older cache
+files; the local energy runs over the electrons and points of all walkers and does not depend on
+them, so they are not timed.  The reference has no counterpart (XLA picks its own launch shapes).
 """
 
 from __future__ import annotations
@@ -19,7 +19,7 @@ import torch
 from . import _lib
 
 KNOBS = {"el_walkers_per_block": 2, "sweep_walkers_per_block": 3, "el_waves_per_walker": 4}
-CANDIDATES = {"el_walkers_per_block": (1, 2, 4), "sweep_walkers_per_block": (1, 2, 4), "el_waves_per_walker": (1, 2)}
+CANDIDATES = {"sweep_walkers_per_block": (1, 2, 4)}
 
 
 def set_tuning(pack, **values) -> None:
@@ -54,10 +54,10 @@ def _key(pack, W):
 
 
 def autotune(ws, n_moves: int | None = None, reps: int = 3, seed: int = 1, cache_path: str | None = None) -> dict:
-    """Time every candidate walkers-per-block of the E_L kernel and of the proposal kernel for the
-    walkers ``ws`` (a WalkerState), apply the fastest to ``ws.pack`` and return {'best': {...},
-    'el_ms': {...}, 'sweep_ms': {...}}.  With ``cache_path`` the choice is stored in (and, when
-    present, read from) a JSON file keyed by the system shape, precision and walker count."""
+    """Time every candidate walkers-per-block of the proposal kernel for the walkers ``ws`` (a
+    WalkerState), apply the fastest to ``ws.pack`` and return {'best': {...}, 'sweep_ms': {...},
+    'cached': False}.  With ``cache_path`` the choice is stored in (and, when present, read from) a
+    JSON file keyed by the system shape, precision and walker count."""
     from ._api import WalkerState
 
     pack, W = ws.pack, ws.W
@@ -69,17 +69,6 @@ def autotune(ws, n_moves: int | None = None, reps: int = 3, seed: int = 1, cache
             set_tuning(pack, **cached)
             return {"best": cached, "cached": True}
     scratch = WalkerState(pack, W).init(ws.r_up, ws.r_dn)
-    RT = scratch.rotations(seed, 0)
-    el = {}
-    for wpb in CANDIDATES["el_walkers_per_block"]:
-        set_tuning(pack, el_walkers_per_block=wpb, el_waves_per_walker=1)
-        el[f"wpb{wpb}"] = ((wpb, 1), _time(lambda: scratch.local_energy(RT), reps))
-    for team in CANDIDATES["el_waves_per_walker"]:
-        if team == 1:  # the one-wave shapes above
-            continue
-        set_tuning(pack, el_walkers_per_block=1, el_waves_per_walker=team)
-        el[f"team{team}"] = ((1, team), _time(lambda: scratch.local_energy(RT), reps))
-    wpb_el, team_el = min(el.values(), key=lambda v: v[1])[0]
     n_moves = n_moves or pack.n_el
     sw = {}
     mv = [0]
@@ -91,8 +80,7 @@ def autotune(ws, n_moves: int | None = None, reps: int = 3, seed: int = 1, cache
     for wpb in CANDIDATES["sweep_walkers_per_block"]:
         set_tuning(pack, sweep_walkers_per_block=wpb)
         sw[wpb] = _time(sweep, reps)
-    wpb_sw = min(sw, key=sw.get)
-    best = {"el_walkers_per_block": wpb_el, "sweep_walkers_per_block": wpb_sw, "el_waves_per_walker": team_el}
+    best = {"sweep_walkers_per_block": min(sw, key=sw.get)}
     set_tuning(pack, **best)
     del scratch
     if cache_path:
@@ -103,5 +91,4 @@ def autotune(ws, n_moves: int | None = None, reps: int = 3, seed: int = 1, cache
         data[key] = best
         with open(cache_path, "w") as f:
             json.dump(data, f, indent=1)
-    return {"best": best, "el_ms": {name: t for name, (_, t) in el.items()},
-            "sweep_ms": {f"wpb{w}": t for w, t in sw.items()}, "cached": False}
+    return {"best": best, "sweep_ms": {f"wpb{w}": t for w, t in sw.items()}, "cached": False}

@@ -1,7 +1,7 @@
-"""Launch-shape knobs and the autotuner (jqmc_amd/autotune.py): every E_L walkers-per-block setting
-gives bit-identical local energies, every proposal walkers-per-block setting takes identical
-decisions (bit-identical positions), bad knob values are refused, and autotune() applies a valid
-choice and round-trips through its JSON cache."""
+"""Launch-shape knobs and the autotuner (jqmc_amd/autotune.py): every proposal walkers-per-block setting
+takes identical decisions (bit-identical positions), the local-energy knobs are taken and change
+nothing, bad knob values are refused, and autotune() applies a valid choice and round-trips through its
+JSON cache, older ones included."""
 
 import json
 
@@ -26,14 +26,6 @@ def _state(prec="fp64", W=96):
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 def test_knobs_change_no_result_bit(prec):
     pack, ru, rd = _state(prec)
-    ws = WalkerState(pack, len(ru)).init(ru, rd)
-    RT = ws.rotations(2, 0)
-    set_tuning(pack, el_walkers_per_block=0)
-    ref = ws.local_energy(RT).clone()
-    for w in CANDIDATES["el_walkers_per_block"]:
-        set_tuning(pack, el_walkers_per_block=w)
-        assert torch.equal(ws.local_energy(RT), ref), w
-    set_tuning(pack, el_walkers_per_block=0)
     pos = {}
     for w in (0,) + CANDIDATES["sweep_walkers_per_block"]:
         set_tuning(pack, sweep_walkers_per_block=w)
@@ -44,24 +36,19 @@ def test_knobs_change_no_result_bit(prec):
         assert all(torch.equal(a, b) for a, b in zip(pos[w], pos[0])), w
 
 
-@pytest.mark.parametrize("prec,rtol", [("fp64", 1e-11), ("mixed", 1e-5)])
-def test_el_team_matches_one_wave_within_rounding(prec, rtol):
-    """A team of 2 or 4 waves per walker adds its partial sums in wave order: e_L equals the one-wave
-    result up to rounding (FP64: 1e-11 of max(1, |e_L|); mixed: 1e-5, the FP32 J3 sums regrouped),
-    and repeats bit for bit."""
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_local_energy_knobs_are_taken_and_change_nothing(prec):
+    """Both knobs of the local energy keep their values and reach no launch."""
     pack, ru, rd = _state(prec)
     ws = WalkerState(pack, len(ru)).init(ru, rd)
     RT = ws.rotations(4, 0)
-    set_tuning(pack, el_walkers_per_block=0, el_waves_per_walker=0)
     ref = ws.local_energy(RT).clone()
-    for team in (2, 4):
-        set_tuning(pack, el_waves_per_walker=team)
-        assert get_tuning(pack)["el_waves_per_walker"] == team
-        e = ws.local_energy(RT).clone()
-        assert torch.equal(ws.local_energy(RT), e), team
-        err = ((e - ref).abs() / ref.abs().clamp(min=1.0)).max().item()
-        assert err <= rtol, (team, err)
-    set_tuning(pack, el_waves_per_walker=0)
+    for knob in ("el_walkers_per_block", "el_waves_per_walker"):
+        assert knob not in CANDIDATES
+        for v in (1, 2, 4, 0):
+            set_tuning(pack, **{knob: v})
+            assert get_tuning(pack)[knob] == v
+            assert torch.equal(ws.local_energy(RT), ref), (knob, v)
 
 
 def test_bad_knob_values_are_refused():
@@ -83,13 +70,17 @@ def test_autotune_applies_and_caches(tmp_path):
     cache = tmp_path / "tune.json"
     out = autotune(ws, reps=1, cache_path=str(cache))
     assert not out["cached"]
-    assert get_tuning(pack) == out["best"]
+    assert set(out["best"]) == set(CANDIDATES)
     for k, v in out["best"].items():
-        assert v in CANDIDATES[k], (k, v)
+        assert v in CANDIDATES[k] and get_tuning(pack)[k] == v, (k, v)
     assert torch.equal(ws.r_up, r0), "the caller's walkers do not move"
-    assert len(out["el_ms"]) == len(CANDIDATES["el_walkers_per_block"]) + len(CANDIDATES["el_waves_per_walker"]) - 1
     assert len(out["sweep_ms"]) == 3
-    set_tuning(pack, el_walkers_per_block=0, sweep_walkers_per_block=0)
+    set_tuning(pack, sweep_walkers_per_block=0)
     again = autotune(ws, cache_path=str(cache))
-    assert again["cached"] and get_tuning(pack) == out["best"]
-    assert list(json.loads(cache.read_text()).values())[0] == out["best"]
+    assert again["cached"] and get_tuning(pack)["sweep_walkers_per_block"] == out["best"]["sweep_walkers_per_block"]
+    (key, best), = json.loads(cache.read_text()).items()
+    assert best == out["best"]
+    # a file of an earlier version, with the local-energy knobs
+    older = {"el_walkers_per_block": 2, "sweep_walkers_per_block": 1, "el_waves_per_walker": 2}
+    cache.write_text(json.dumps({key: older}))
+    assert autotune(ws, cache_path=str(cache))["cached"] and get_tuning(pack) == older
