@@ -1776,9 +1776,9 @@ int launch_dlnpsi(const Sys& s, int64_t W, const jqmc_walkers* wk, const ParamLa
   };
   if (lay.lam >= 0) {
     outer(nu, nu, no, k.Ginv, (int64_t)nu * nu, 1, nu, k.orb, (int64_t)ne * no, no, Z, (int64_t)nu * no, no, 0);
-    if (nd > 0)
-      outer(nd, no, no, Z, (int64_t)nu * no, no, 1, k.orb + (int64_t)nu * no, (int64_t)ne * no, no, O, ld,
-            no + (nu - nd), lay.lam);
+    // without dn electrons a block of zeros (K = 0)
+    outer(nd, no, no, Z, (int64_t)nu * no, no, 1, k.orb + (int64_t)nu * no, (int64_t)ne * no, no, O, ld, no + (nu - nd),
+          lay.lam);
   }
   if (lay.j3 >= 0) {
     k_init_jsums<T><<<grid_for(W * na, 256), 256, 0, st>>>(s, W, k, S1, nullptr);

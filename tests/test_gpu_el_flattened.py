@@ -1,7 +1,7 @@
 """The flattened local energy (k_el_prep / k_el_kinetic / k_el_points) against the oracle where its tiles end:
 walker counts around the groups of four walkers and 64 electrons, meshes that fill a wave differently, every
-orbital form (up to 16, 32, 48 and more than 64 MOs, different MOs per spin, AO orbitals), f shells and
-spherical shells, open shells.  Tolerance: 1e-9 of 1 + |T| + |V| (the parts cancel in e_L; G^-1 of these small
+orbital form (up to 16, 32, 48, 64 and more MOs, different MOs per spin, AO orbitals), f shells; Cartesian closed
+shells (the other forms: test_gpu_forms.py).  Tolerance: 1e-9 of 1 + |T| + |V| (the parts cancel in e_L; G^-1 of these small
 random wavefunctions loses at most a few digits)."""
 
 import dataclasses
@@ -34,7 +34,8 @@ def _with_mos(system, n_up, same):
 CASES = [("water_ae", None, 6, 1), ("water_ae", None, 6, 13), ("chain10", None, 4, 9), ("chain10", None, 18, 7),
          ("benzene_ecp", None, 12, 5), ("chain56", None, 6, 3), ("chain96", None, 6, 2), ("water4_ecp", None, 12, 3),
          ("water4_jagp", None, 6, 2), ("chain30", (20, True), 6, 3), ("chain30", (17, False), 12, 3),
-         ("chain30", (70, True), 6, 3), ("chain30", (66, False), 4, 2)]
+         ("chain30", (50, False), 6, 2), ("chain30", (60, True), 6, 3), ("chain30", (70, True), 6, 3),
+         ("chain30", (66, False), 4, 2)]
 
 
 @pytest.mark.parametrize("name,mos,nv,W", CASES)

@@ -1,7 +1,7 @@
 """The flattened position derivatives (k_fr_kinetic / k_fr_points / k_fr_adjoint / k_fr_pairing / k_fr_orbital /
 k_fr_out) against the oracle where their tiles end: walker counts around the groups of four walkers and 64
-electrons, meshes that fill a wave differently, up to 16 and more than 64 MOs,
-different MOs per spin, open shells; and a call longer than the walkers taken at a time against short calls.
+electrons, meshes that fill a wave differently, up to 16 and more than 64 MOs, different MOs per spin, Cartesian
+closed shells (the other forms: test_gpu_forms.py); and a call longer than the walkers taken at a time against short calls.
 Tolerance: 1e-9 of the largest element, as for the other checks of these derivatives."""
 
 import numpy as np
