@@ -206,3 +206,39 @@ def test_meshes_of_many_points_match_oracle(nv, monkeypatch):
         ref = oracle.forces.local_energy_position_grads(ham, r_up[w], r_dn[w], RT[w].cpu().numpy(), Nv=nv)
         for k in ("dE_dr", "dE_dR", "dlnpsi_dr", "dlnpsi_dR"):
             assert float(np.abs(out[k][w] - ref[k]).max()) <= 1e-9 * max(1.0, float(np.abs(ref[k]).max())), (w, k)
+
+
+CHAINS = ["all_up", "doublet", "doublet_jagp", "g_shell", "no_j3", "no_jastrow", "one_electron", "pade_exp", "septet",
+          "six_primitives"]
+
+
+@pytest.mark.parametrize("name", CHAINS)
+def test_moves_match_oracle(name):
+    """Metropolis decisions and positions, then two lattice projections from there, on the oracle's stream (to
+    1e-10; the weights to 1e-8: G^-1 after the moves)."""
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+    from oracle import mcmc as om
+    from test_gpu_lrdmc import _oracle_chain
+
+    ham = _form(name)
+    W, n_moves, seed = 3, 30, 77
+    r_up, r_dn = _walkers(ham, W)
+    ws = WalkerState(SystemPack(ham), W).init(r_up, r_dn)
+    ws.sweep(n_moves, 0.5, 1e-4, seed, 0)
+    ru, rd = ws.r_up.cpu().numpy(), ws.r_dn.cpu().numpy()
+    for w in range(W):
+        G, Gi = om.init_walker(ham, r_up[w], r_dn[w])
+        acc, rej, ou, od, _, _ = om.metropolis_walker(ham, r_up[w], r_dn[w], Gi, G, seed, w, 0, n_moves, 0.5, 1e-4)
+        assert ws.accepted[w].item() == acc and ws.rejected[w].item() == rej
+        np.testing.assert_allclose(ru[w], ou, rtol=0, atol=1e-10)
+        np.testing.assert_allclose(rd[w], od, rtol=0, atol=1e-10)
+    ws.refresh()
+    for move in ("tmove", "dltmove"):
+        ws.init(ru, rd)
+        out = ws.lrdmc_projection(WalkerState.lrdmc_params(0.3, E_scf=-10.0, n_steps=2, non_local_move=move), seed, 5)
+        for w in range(W):
+            a, b, _, _, wgt, _, _, _ = _oracle_chain(ham, ru[w], rd[w], 2, 0.3, -10.0, seed, w, 5, move)
+            np.testing.assert_allclose(ws.r_up[w].cpu().numpy(), a, rtol=0, atol=1e-10)
+            np.testing.assert_allclose(ws.r_dn[w].cpu().numpy(), b, rtol=0, atol=1e-10)
+            assert abs(out["w_L"][w].item() - wgt) <= 1e-8 * abs(wgt)
