@@ -128,8 +128,7 @@ __device__ __forceinline__ double sqrt_nr(double x, double& inv) {
   return g;
 }
 
-// The same for every x, the reciprocal of 0 infinite: for Coulomb terms, so that the energy of coincident
-// particles is no number of ordinary size.
+// The same for every x, the reciprocal of 0 infinite.
 __device__ __forceinline__ double sqrt_inv(double x, double& inv) {
   double r = sqrt_nr(x, inv);
   if (!(x >= 1.0e-280 && x <= 1.0e300)) {
@@ -219,6 +218,24 @@ __device__ __forceinline__ double ecp_local_nr(CSys& s, int n, double d, double 
   return v;
 }
 
+// Bare Coulomb and local ECP terms of electron e (each pair of electrons half) by plain divisions: where the fast
+// reciprocals left no number of ordinary size, so that the energy of coincident particles is infinite.
+__device__ __forceinline__ double bare_terms(CSys& s, bool ions, const double* rr, int e) {
+  const double x = rr[3 * e], y = rr[3 * e + 1], z = rr[3 * e + 2];
+  double v = 0.0;
+  for (int n = 0; n < s.n_nuc; ++n) {
+    const double dx = s.nuc_pos[3 * n] - x, dy = s.nuc_pos[3 * n + 1] - y, dz = s.nuc_pos[3 * n + 2] - z;
+    const double d = sqrt(dx * dx + dy * dy + dz * dz);
+    if (ions) v += -s.nuc_charge[n] / d;
+    if (s.ecp_on) v += ecp_local_nr(s, n, d, 1.0 / d);
+  }
+  for (int f = 0; f < s.n_el; ++f) {
+    const double dx = x - rr[3 * f], dy = y - rr[3 * f + 1], dz = z - rr[3 * f + 2];
+    if (f != e) v += 0.5 / sqrt(dx * dx + dy * dy + dz * dz);
+  }
+  return v;
+}
+
 // Blocks [0, q_blocks) of a job: wave (w, row tile) forms q of 16 electrons of one spin block of walker
 // w.  The others: one wave per walker.
 template <typename T>
@@ -299,6 +316,7 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
     int best = 0;
     if (e < ne) {
       const double x = rr[3 * e], y = rr[3 * e + 1], z = rr[3 * e + 2];
+      const double pot0 = pot;
       double old = 0.0, bd = 1.0e300;
       for (int n = 0; n < s.n_nuc; ++n) {
         const double dx = np[3 * n] - x, dy = np[3 * n + 1] - y, dz = np[3 * n + 2] - z;
@@ -307,8 +325,7 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
           bd = d;
           best = n;
         }
-        double di = rcp_nr(d);
-        if (!(d >= 1.0e-140 && d <= 1.0e150)) di = 1.0 / d;  // 0: infinite
+        const double di = rcp_nr(d);
         if (!J.lr) pot += -nc[n] * di;
         if (s.ecp_on) pot += ecp_local_nr(s, n, d, di);
         if (JP.j1_type) old += j1_value(JP, s.j1_c[n], s.j1_A[n], d);
@@ -317,11 +334,12 @@ __global__ void __launch_bounds__(256) k_el_prep(ElJobs<T> M) {
         if (f == e) continue;
         const double dx = x - rr[3 * f], dy = y - rr[3 * f + 1], dz = z - rr[3 * f + 2];
         double ri;
-        const double r = sqrt_inv(dx * dx + dy * dy + dz * dz, ri);
+        const double r = sqrt_nr(dx * dx + dy * dy + dz * dz, ri);
         pot += 0.5 * ri;
         if (JP.j2_type) old += j2_value(JP, r);
       }
       J.jold[w * ne + e] = old;
+      if (!(fabs(pot) <= 1.0e120)) pot = pot0 + bare_terms(s, !J.lr, rr, e);
       if (nonlocal) has = s.ecp_nt[best] > 0;
     }
     const uint64_t mask = __ballot(has);

@@ -562,7 +562,8 @@ __global__ void __launch_bounds__(256) k_init_jfield_tile(Sys s, int64_t M, cons
 // 16384 walkers, at scattered rows) and by latency at small ones.  Blocks of 32 walkers x 64 AOs with barriers
 // took 32.7 us for 1024 benzene walkers, 175 us for 16384, 38.5 us for 2048 of 4 x H2O in FP32 and 9.3 us for
 // 256 of H2O; this 20.8, 173, 27.7 and 7.7 us.  Two AO tiles a wave: 31.4, 174 and 36.0 us, 32 movers a wave
-// 171 us for 16384.
+// 171 us for 16384.  A symmetric J3 takes the same product twice: a branch around the second put the operands
+// in scratch (274 us for 16384).
 template <typename T, bool kDirect = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_sweep_jfield_mfma(Sys s, int64_t W,
                                                                                                    WalkT<T> wk,
