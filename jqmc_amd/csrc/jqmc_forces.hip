@@ -372,7 +372,8 @@ struct NucSums {
 };
 
 // Lanes = 64 flattened electrons, the chunks of the AO range split over the four waves in order.  Bound by
-// the latency of the rows of h and g (22 % vector issue) and the FP64 vector rate (see k_el_kinetic).
+// the latency of the rows of h and g and of the sums per nucleus (14 % vector issue; 0.84 GB in 219 us for 2048
+// benzene walkers).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_fr_kinetic(FrJob J) {
   extern __shared__ double smem[];
   CSys& s = csys(J.sys);
@@ -678,7 +679,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 // A wave takes up to ten listed electrons of four walkers, one quadrature point per lane (an electron with
 // more than 64 points one part after the other).  Two AO sweeps: ratios, then the adjoints; per chunk of
 // twelve AOs the values at the points go through LDS and are summed per electron into w_e and gbar_e, per
-// run of AOs on one nucleus the gradients are summed into dE/dR.  Bound by the FP64 vector rate (40 %) and the
+// run of AOs on one nucleus the gradients are summed into dE/dR.  Bound by the FP64 vector rate (44 %) and the
 // latency of the staged rows: three waves per SIMD with some words spilled outside the sweeps took 829 us for
 // 2048 benzene walkers, two waves 1129 us.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_fr_points(FrJob J, int n_groups) {
