@@ -77,6 +77,11 @@ def kernel_work(pack, W, n_moves, accepted, n_ecp_el=None):
     return sweep, el
 
 
+# HBM bytes of one local-energy call from rocprofv3 FETCH_SIZE / WRITE_SIZE (each scaled by what the counter
+# reads for a plain 1 GiB device copy: x2.00 and x1.00), its four kernels together.
+EL_TRAFFIC = {("benzene_ecp", 16384, 12): (2.7e9, "profiles/cases_counters.md")}
+
+
 def cpu_model() -> str:
     try:
         with open("/proc/cpuinfo") as f:
@@ -635,7 +640,7 @@ def main(argv=None):
             "note": "FP64 vector ALU kernels (the determinant fields on the matrix cores) far above the machine balance "
                     f"({intensity:.0f} flop/B of compulsory traffic); peak = MI355X FP64 vector 78.6 TFLOP/s; "
                     "exp/sqrt/div count one op each"}
-    roof["traffic"] = None
+    roof["traffic"], roof["traffic_source"] = EL_TRAFFIC.get((args.workload, W, args.nv), (None, None))
     roof["avg_ms"] = ms
     roof["algorithmic"] = {"flops": work["flops"], "bytes": work["bytes"], "flop_per_byte": intensity,
                            "flops_per_walker": work["flops"] / W,
