@@ -667,7 +667,7 @@ int launch_forces(const jqmc_system* sys, int64_t W, const WalkT<double>& wk, co
       k_el_hrows<double><<<rows, 256, 0, st>>>(E);
   }
   k_fr_orbital<<<blocks, FR_WAVES * WAVE, FR_WAVES * 3 * tile, st>>>(J);
-  k_fr_out<<<(unsigned)W, fr_out_waves(s) * WAVE, 0, st>>>(J, out);
+  k_fr_out<<<(unsigned)W, fr_out_waves(s, W) * WAVE, 0, st>>>(J, out);
   return JQMC_OK;
 }
 

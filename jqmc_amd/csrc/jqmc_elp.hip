@@ -113,8 +113,8 @@ __device__ __forceinline__ double rcp_nr(double x) {
 }
 
 // sqrt(x) and its reciprocal for x >= 0 (below 1e-280: taken as that): one Goldschmidt step on the hardware
-// reciprocal square root, then one residual correction of each.  For distances whose reciprocal is not used,
-// or is cut off first.
+// reciprocal square root, then one residual correction of each.  For distances whose reciprocal is not used, is
+// cut off first, or is checked afterwards (bare_terms).
 __device__ __forceinline__ double sqrt_nr(double x, double& inv) {
   x = fmax(x, 1.0e-280);
   const double y = __builtin_amdgcn_rsq(x);

@@ -1373,10 +1373,13 @@ struct FrOut {
   int swct;
 };
 
-// One block per walker, lanes = electrons; its waves (fr_out_waves) share the partners, points and nuclei.  Three
-// waves fit a SIMD, so that waves without a partner of their own cost a round: the whole call for 2048 walkers of
-// H2 (2 electrons) 98 us with four waves in this kernel and k_fr_pairing, 89 with one.
-inline int fr_out_waves(const Sys& s) { return std::min(FR_WAVES, (std::max(s.n_el, s.n_nuc) + 3) / 4); }
+// One block per walker, lanes = electrons; the partners, points and nuclei in four parts shared by the block's waves,
+// whose number changes no bit.  Four waves as long as all walkers' fit the chip (three per SIMD), then no more than
+// the walker has partners for: 2048 walkers of H2 (2 electrons), whole call, 98 us with four waves and 87 with one
+// (k_fr_pairing alike); 64 walkers 69 and 74.
+inline int fr_out_waves(const Sys& s, int64_t W) {
+  return W * FR_WAVES <= 3 * 1024 ? FR_WAVES : std::min(FR_WAVES, (std::max(s.n_el, s.n_nuc) + 3) / 4);
+}
 __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
   __shared__ double p_sh[FR_WAVES][3][WAVE];
   CSys& s = csys(J.sys);
@@ -1402,7 +1405,6 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
     double re[3], dJ[3], dl[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      re[c] = wave == 0 ? J.re[c * M + i] : 0.0;
       dJ[c] = J.el[(3 + c) * M + i];
       dl[c] = -dJ[c];  // D1 + gJ = d ln|Psi| / d r_e
     }
@@ -1411,77 +1413,81 @@ __global__ void __launch_bounds__(256) k_fr_out(FrJob J, FrOut O) {
       en[0] += J.te[i];
       en[1] += S;
     }
-    // e-e pairs: e's own terms and those of its partners together (each is odd in r_e - r_f)
-    for (int f = wave; f < ne; f += nw) {
-      const CPtr<double> q = f < nu ? ru + 3 * f : rd + 3 * (f - nu);
-      const double ux = ex - q[0], uy = ey - q[1], uz = ez - q[2];
-      const double d2 = ux * ux + uy * uy + uz * uz;
-      if (f == e) continue;
-      const double d = sqrt(d2), c0 = -1.0 / (d2 * d);
-      re[0] += c0 * ux;
-      re[1] += c0 * uy;
-      re[2] += c0 * uz;
-      if (JP.j2_type) {
-        double f1, f2, f3;
-        const double r = fmax(d, 1.0e-12);
-        j2_f123(JP.j2_type, JP.a2, r, f1, f2, f3);
-        const double D[3] = {dJ[0] - el[3 * M + f], dJ[1] - el[4 * M + f], dJ[2] - el[5 * M + f]};
-        radial_adjoint(ux, uy, uz, f1, f2, f3, D, -1.0, re);
-        const double c = -(S + el[9 * M + f]) * f1 / r;
-        re[0] += c * ux;
-        re[1] += c * uy;
-        re[2] += c * uz;
-      }
-    }
-    // the other electrons' quadrature points move with r_e through J2
-    if (JP.j2_type)
-      for (int j = wave; j < n_ecp; j += nw) {
-        const int x = cview(J.elist)[w * ne + j] & 255;
-        const CPtr<double> q = cview(J.pt) + (w * ne + j) * (int64_t)nv * 4;
-        for (int k = 0; k < nv; ++k) {
-          const double ux = q[4 * k] - ex, uy = q[4 * k + 1] - ey, uz = q[4 * k + 2] - ez;
-          double ri;
-          const double r = sqrt_nr(fmax(ux * ux + uy * uy + uz * uz, 1.0e-24), ri);
-          const double c = x == e ? 0.0 : q[4 * k + 3] * j2_slope(JP, r, ri);
-          re[0] -= c * ux;
-          re[1] -= c * uy;
-          re[2] -= c * uz;
-        }
-      }
-    // nuclei
-    for (int n = wave; n < nn; n += nw) {
-      const double ux = ex - np[3 * n], uy = ey - np[3 * n + 1], uz = ez - np[3 * n + 2];
-      const double d2 = ux * ux + uy * uy + uz * uz, d = sqrt(d2);
-      double v[3] = {0.0, 0.0, 0.0}, c = s.nuc_charge[n] / (d2 * d);  // -Z / d
-      if (s.ecp_on)
-        for (int t = 0; t < s.ecpl_nt[n]; ++t) {
-          const int o = n * s.ecp_max_local + t;
-          const double Vl = (1.0 / d2) * s.ecpl_coef[o] * rpow(d, s.ecpl_pow[o]) * exp_nonpos(-s.ecpl_exp[o] * d2);
-          c += Vl * ((s.ecpl_pow[o] - 2.0) / d - 2.0 * s.ecpl_exp[o] * d) / d;
-        }
-      if (JP.j1_type) {
-        double f1, f2, f3;
-        const double r = fmax(d, 1.0e-12);
-        j1_f123(JP.j1_type, JP.a1, s.j1_c[n], s.j1_A[n], r, f1, f2, f3);
-        radial_adjoint(ux, uy, uz, f1, f2, f3, dJ, -0.5, v);
-        c -= S * f1 / r;
-      }
-      const double u[3] = {ux, uy, uz};
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        v[k] += c * u[k];
-        re[k] += v[k];
-        if (act) J.RA[(int64_t)(3 * n + k) * M + i] -= v[k];
-      }
-    }
     if (e0 > 0) __syncthreads();
+    for (int g = wave; g < FR_WAVES; g += nw) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) p_sh[wave][c][lane] = re[c];
+      for (int c = 0; c < 3; ++c) re[c] = g == 0 ? J.re[c * M + i] : 0.0;
+      // e-e pairs: e's own terms and those of its partners together (each is odd in r_e - r_f)
+      for (int f = g; f < ne; f += FR_WAVES) {
+        const CPtr<double> q = f < nu ? ru + 3 * f : rd + 3 * (f - nu);
+        const double ux = ex - q[0], uy = ey - q[1], uz = ez - q[2];
+        const double d2 = ux * ux + uy * uy + uz * uz;
+        if (f == e) continue;
+        const double d = sqrt(d2), c0 = -1.0 / (d2 * d);
+        re[0] += c0 * ux;
+        re[1] += c0 * uy;
+        re[2] += c0 * uz;
+        if (JP.j2_type) {
+          double f1, f2, f3;
+          const double r = fmax(d, 1.0e-12);
+          j2_f123(JP.j2_type, JP.a2, r, f1, f2, f3);
+          const double D[3] = {dJ[0] - el[3 * M + f], dJ[1] - el[4 * M + f], dJ[2] - el[5 * M + f]};
+          radial_adjoint(ux, uy, uz, f1, f2, f3, D, -1.0, re);
+          const double c = -(S + el[9 * M + f]) * f1 / r;
+          re[0] += c * ux;
+          re[1] += c * uy;
+          re[2] += c * uz;
+        }
+      }
+      // the other electrons' quadrature points move with r_e through J2
+      if (JP.j2_type)
+        for (int j = g; j < n_ecp; j += FR_WAVES) {
+          const int x = cview(J.elist)[w * ne + j] & 255;
+          const CPtr<double> q = cview(J.pt) + (w * ne + j) * (int64_t)nv * 4;
+          for (int k = 0; k < nv; ++k) {
+            const double ux = q[4 * k] - ex, uy = q[4 * k + 1] - ey, uz = q[4 * k + 2] - ez;
+            double ri;
+            const double r = sqrt_nr(fmax(ux * ux + uy * uy + uz * uz, 1.0e-24), ri);
+            const double c = x == e ? 0.0 : q[4 * k + 3] * j2_slope(JP, r, ri);
+            re[0] -= c * ux;
+            re[1] -= c * uy;
+            re[2] -= c * uz;
+          }
+        }
+      // nuclei
+      for (int n = g; n < nn; n += FR_WAVES) {
+        const double ux = ex - np[3 * n], uy = ey - np[3 * n + 1], uz = ez - np[3 * n + 2];
+        const double d2 = ux * ux + uy * uy + uz * uz, d = sqrt(d2);
+        double v[3] = {0.0, 0.0, 0.0}, c = s.nuc_charge[n] / (d2 * d);  // -Z / d
+        if (s.ecp_on)
+          for (int t = 0; t < s.ecpl_nt[n]; ++t) {
+            const int o = n * s.ecp_max_local + t;
+            const double Vl = (1.0 / d2) * s.ecpl_coef[o] * rpow(d, s.ecpl_pow[o]) * exp_nonpos(-s.ecpl_exp[o] * d2);
+            c += Vl * ((s.ecpl_pow[o] - 2.0) / d - 2.0 * s.ecpl_exp[o] * d) / d;
+          }
+        if (JP.j1_type) {
+          double f1, f2, f3;
+          const double r = fmax(d, 1.0e-12);
+          j1_f123(JP.j1_type, JP.a1, s.j1_c[n], s.j1_A[n], r, f1, f2, f3);
+          radial_adjoint(ux, uy, uz, f1, f2, f3, dJ, -0.5, v);
+          c -= S * f1 / r;
+        }
+        const double u[3] = {ux, uy, uz};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          v[k] += c * u[k];
+          re[k] += v[k];
+          if (act) J.RA[(int64_t)(3 * n + k) * M + i] -= v[k];
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) p_sh[g][c][lane] = re[c];
+    }
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       re[c] = p_sh[0][c][lane];
-      for (int q = 1; q < nw; ++q) re[c] += p_sh[q][c][lane];
+      for (int q = 1; q < FR_WAVES; ++q) re[c] += p_sh[q][c][lane];
     }
     if (act && wave == 0) {
 #pragma unroll

@@ -58,3 +58,24 @@ def test_long_call_matches_short_calls():
         for k, v in ref.items():
             scale = max(1.0, float(v.abs().max()))
             assert float((out[k][a:b] - v).abs().max()) <= 1e-9 * scale, k
+
+
+@pytest.mark.parametrize("name", ["h2", "water_ae", "chain10"])
+def test_number_of_walkers_changes_no_bit(name):
+    """The waves that k_fr_out and k_fr_pairing give a walker, the J3 product's form and the parts of a call depend on
+    how many walkers there are; their results do not."""
+    from jqmc_amd import synthetic
+    from jqmc_amd._api import WalkerState
+    from jqmc_amd._pack import SystemPack
+
+    if name == "h2":
+        st = synthetic._structure(["H", "H"], [[0.0, 0.0, 0.0], [0.0, 0.0, 1.4]])
+        system = synthetic._assemble("h2", st, {"H": "2s1p"}, 1)
+    else:
+        system = synthetic.chain_ecp(10, 1) if name == "chain10" else synthetic.water_ae(0)
+    pack, n, rep = SystemPack(system.hamiltonian_data), 5, 4000
+    r_up, r_dn = (torch.as_tensor(r, device="cuda") for r in system.initial_walkers(n, seed=2, sigma=0.8))
+    small = WalkerState(pack, n).init(r_up, r_dn).position_grads()
+    large = WalkerState(pack, n * rep).init(r_up.repeat(rep, 1, 1), r_dn.repeat(rep, 1, 1)).position_grads()
+    for k, v in small.items():
+        assert torch.equal(large[k].view(rep, *v.shape), v.expand(rep, *v.shape)), k

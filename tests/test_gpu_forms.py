@@ -80,7 +80,6 @@ FORMS = {
     "six_primitives": lambda: _shells("3s2p1d1f", n_prim=6),
     "one_primitive": lambda: _shells("3s2p1d1f", n_prim=1),
 }
-# the CN systems have up to 15 AOs on C and 12 on N: all of these forms reach the quadrature points
 
 
 @functools.lru_cache(maxsize=None)
