@@ -155,7 +155,7 @@ struct FrBuf {
 
 // Walkers that a call of W takes at a time, so that its workspace stays bounded (benzene: 1.3 GB): at most 2^17
 // electrons, 2048 blocks of the launches over electrons, in parts of equal size.  32768 walkers of N (7 electrons)
-// took 1286 us in parts of 4096 walkers and 797 so, H2 1122 and 459 us (with the waves of k_fr_out below).
+// took 1286 us in parts of 4096 walkers and 800 so, H2 1122 and 471 us (with the waves of k_fr_out below).
 constexpr int64_t FR_ELECTRONS = 1 << 17;
 inline int64_t fr_chunk(const Sys& s, int64_t W) {
   const int64_t most = FR_ELECTRONS / s.n_el, parts = (W + most - 1) / most;
