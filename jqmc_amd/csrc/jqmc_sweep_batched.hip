@@ -11,7 +11,7 @@
 //                     orbital / pair rows, G, G^-1) is updated in place and dA is left in the
 //                     workspace with the moved electron's index
 //     k_sweep_jfield_mfma  [T1 | T2] = [J3 | J3^T] x dA of the walkers that accepted on the matrix
-//                     cores, a wave per 16 of them and 16 AOs, then the J3 field increments of
+//                     cores, a wave per 16 of them and 16 or 32 AOs, then the J3 field increments of
 //                     jastrow_factor.py:4121-4135 on those
 //   k_sweep_flush     spin-block offsets added to every field row; R_AS stored
 //
@@ -381,6 +381,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 
 constexpr int JF_SEG = 64;      // walkers whose movers one block collects
 constexpr int JF_KC = 16;       // AO columns per step
+constexpr int64_t JF_WIDE_BLOCKS = 6 * 256;  // blocks of one AO tile from which a block takes two
 constexpr int JF_LD = 17;       // words per LDS row of the staged changes: no conflict over 16 rows
 
 // Matrix-core step of the J3 field products: D(16 x 16) += A(16 x 4) B(4 x 16) with A(i, k) from lane
@@ -551,32 +552,41 @@ __global__ void __launch_bounds__(256) k_init_jfield_tile(Sys s, int64_t M, cons
 // read by the next Hamiltonian launch), every row f != e of a moved walker takes its increment
 // instead: t1 for f < e, t2 for f > e, no offsets.
 //
-// The four waves of a block share 64 walkers and 16 AOs: wave t takes the movers 16 t .. 16 t + 15 of the 64
+// The four waves of a block share 64 walkers and 16 NT AOs: wave t takes the movers 16 t .. 16 t + 15 of the 64
 // (in order; a wave without any leaves at once) as the rows of D(mover, a) = sum_b dA(mover, b) J(b, a).
 // A(i, k) = dA of mover i at AO b0 + k through the wave's own LDS tile, B(k, j) = J3^T or J3 at (b0 + k, AO
-// a0 + j) straight from L2, both with the next sixteen b on their way during the current ones: no barrier, so
+// a0 + 16 y + j) straight from L2, both with the next sixteen b on their way during the current ones: no barrier, so
 // that the products of some waves overlap the row updates of others, and many small blocks, so that small
 // walker counts fill the chip.  The sums run over b in order in fours.  The AO tiles of a segment are eight
 // blocks apart (one XCD): the lines that two tiles share meet in its L2.
 // Bound by the row updates at large walker counts (104 bytes per AO and accepted move of benzene, 340 MB of
 // 16384 walkers, at scattered rows) and by latency at small ones.  Blocks of 32 walkers x 64 AOs with barriers
 // took 32.7 us for 1024 benzene walkers, 175 us for 16384, 38.5 us for 2048 of 4 x H2O in FP32 and 9.3 us for
-// 256 of H2O; this 20.8, 173, 27.7 and 7.7 us.  Two AO tiles a wave: 31.4, 174 and 36.0 us, 32 movers a wave
-// 171 us for 16384.  A symmetric J3 takes the same product twice: a branch around the second put the operands
-// in scratch (274 us for 16384).
-template <typename T, bool kDirect = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_sweep_jfield_mfma(Sys s, int64_t W,
-                                                                                                   WalkT<T> wk,
-                                                                                                   SweepWs<T> ws) {
+// 256 of H2O; one tile (NT = 1) 20.8, 173, 27.7 and 7.7 us.  Two tiles keep those small launches waiting (31.4 and
+// 36.0 us), 32 movers a wave give 171 us for 16384.
+// NT = 2 is for launches that stay many blocks all the same (JF_WIDE_BLOCKS: six of one tile per CU, so at least
+// three of two): then the pieces of rows bound, 64 bytes of FP32 or 128 of FP64 with one tile.  A move of the whole
+// sweep, one tile -> two: 4 x H2O, FP32, 4096 walkers (1216 blocks) 97.7 -> 99.5 us, 8192 (2432) 197 -> 181 us,
+// 16384 392 -> 350 us; benzene 8192 (1920) 152 -> 145 us; 30 electrons and 120 AOs 8192 (1024) 96.7 -> 99.9 us,
+// 16384 (2048) 190 -> 185 us.  In FP64 4 x H2O 16384 504 -> 485 us, benzene 362 -> 358 us (three waves a SIMD; held
+// to four it spills, 513 and 378 us).  Four tiles are slower (FP32 214 us for 8192 of 4 x H2O).  The LRDMC move
+// keeps one tile (its other launches outweigh it: 4096 walkers of 4 x H2O 874 -> 863 us).
+// A symmetric J3 takes the same product twice: a branch around the second put the operands in scratch (274 us for
+// 16384).
+template <typename T, bool kDirect, int NT>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(std::is_same<T, double>::value && NT == 2 ? 3 : 4)))
+    k_sweep_jfield_mfma(Sys s, int64_t W, WalkT<T> wk, SweepWs<T> ws) {
   using M = JfMfma<T>;
   typedef typename M::v4 v4;
   __shared__ T da_sh[4][2][JF_KC * JF_LD];
   __shared__ int mv_sh[4][JF_SEG], at_sh[4][JF_SEG];
   const int lane = threadIdx.x & 63, wave = wave_id(), il = lane & 15, ih = lane >> 4;
   const int nu = s.n_up, ne = s.n_el, na = s.n_ao;
-  const int n_ct = (na + 15) / 16;
+  constexpr int TA = 16 * NT, H = 4 / NT;  // AOs of a wave; rows of a pass of the epilogue
+  const int n_ct = (na + TA - 1) / TA;
   const int64_t blk = blockIdx.x, w0 = (blk / (8 * n_ct) * 8 + blk % 8) * JF_SEG;
-  const int a0 = (int)((blk / 8) % n_ct) * 16;
+  const int a0 = (int)((blk / 8) % n_ct) * TA;
   if (w0 >= W) return;
   const int e_l = w0 + lane < W ? ws.mv[w0 + lane] : -1;
   const uint64_t movers = __ballot(e_l >= 0);
@@ -598,27 +608,41 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   const int sr = lane >> 2, sk = lane & 3;
   const bool s_on = sr < n;
   const T* __restrict__ DA = ws.dA + (w0 + at_s[s_on ? sr : 0]) * na;
-  const int a = a0 + il < na ? a0 + il : na - 1;  // columns past the end are not used
-  T pa[4], pt[4], pj[4], ct[4], cj[4];
+  int a[NT];  // columns past the end are not used
+  bool in[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) {
+    in[y] = a0 + 16 * y + il < na;
+    a[y] = in[y] ? a0 + 16 * y + il : na - 1;
+  }
+  T pa[4], pt[NT][4], pj[NT][4], ct[NT][4], cj[NT][4];
   auto fetch = [&](int b0) {  // without branches: AOs past the end repeat the last one
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int ba = b0 + sk + 4 * q < na ? b0 + sk + 4 * q : na - 1;
       const int b = b0 + 4 * q + ih < na ? b0 + 4 * q + ih : na - 1;
       pa[q] = DA[ba];
-      pt[q] = JT[(int64_t)b * na + a];
-      pj[q] = JJ[(int64_t)b * na + a];
+#pragma unroll
+      for (int y = 0; y < NT; ++y) {
+        pt[y][q] = JT[(int64_t)b * na + a[y]];
+        pj[y][q] = JJ[(int64_t)b * na + a[y]];
+      }
     }
   };
-  v4 acc1 = {0, 0, 0, 0}, acc2 = {0, 0, 0, 0};
+  v4 acc1[NT], acc2[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) acc1[y] = acc2[y] = v4{0, 0, 0, 0};
   fetch(0);
   for (int b0 = 0, st = 0; b0 < na; b0 += JF_KC, st ^= 1) {
     T* da = da_sh[wave][st];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       da[(sk + 4 * q) * JF_LD + sr] = s_on && b0 + sk + 4 * q < na ? pa[q] : (T)0;  // zero against repeated rows of J
-      ct[q] = pt[q];
-      cj[q] = pj[q];
+#pragma unroll
+      for (int y = 0; y < NT; ++y) {
+        ct[y][q] = pt[y][q];
+        cj[y][q] = pj[y][q];
+      }
     }
     if (b0 + JF_KC < na) fetch(b0 + JF_KC);
     asm volatile("" ::: "memory");  // one wave's LDS accesses are taken in order
@@ -626,11 +650,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const T fa = da[(4 * q + ih) * JF_LD + il];
-      acc1 = M::mma(fa, ct[q], acc1);
-      acc2 = M::mma(fa, cj[q], acc2);
+#pragma unroll
+      for (int y = 0; y < NT; ++y) {
+        acc1[y] = M::mma(fa, ct[y][q], acc1[y]);
+        acc2[y] = M::mma(fa, cj[y][q], acc2[y]);
+      }
     }
   }
-  if (a0 + il >= na) return;  // no cross-lane work follows
+  if (!in[0]) return;  // no cross-lane work follows
   // epilogue: element q of this lane is mover row(q, ih) of the wave
   int ee[4];
   int64_t ww[4];
@@ -641,31 +668,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     ww[q] = w0 + at_s[r < n ? r : 0];
   }
   if constexpr (kDirect) {
-    // four rows of the four walkers per pass, all 16 loads in flight together
-    for (int f0 = 0; f0 < ne; f0 += 4) {
-      T v[4][4];
+    // H rows of the four walkers per pass, all 16 loads in flight together
+    for (int f0 = 0; f0 < ne; f0 += H) {
+      T v[H][4][NT];
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < H; ++h)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int f = f0 + h;
-          v[h][q] = (f < ne && ee[q] >= 0 && f != ee[q]) ? wk.jfield[(ww[q] * ne + f) * na + a] : (T)0;
-        }
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+          for (int y = 0; y < NT; ++y) {
+            const int f = f0 + h;
+            v[h][q][y] = (f < ne && ee[q] >= 0 && f != ee[q] && in[y]) ? wk.jfield[(ww[q] * ne + f) * na + a[y]] : (T)0;
+          }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int f = f0 + h;
-          if (f < ne && ee[q] >= 0 && f != ee[q])
-            wk.jfield[(ww[q] * ne + f) * na + a] = v[h][q] + (f < ee[q] ? acc1[q] : acc2[q]);
-        }
+      for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int y = 0; y < NT; ++y) {
+            const int f = f0 + h;
+            if (f < ne && ee[q] >= 0 && f != ee[q] && in[y])
+              wk.jfield[(ww[q] * ne + f) * na + a[y]] = v[h][q][y] + (f < ee[q] ? acc1[y][q] : acc2[y][q]);
+          }
     }
     return;
   }
   const bool sym = s.j3_sym != 0;
   int cs[4], cn[4];
   bool upm[4], lw[4];
-  T d4[4];
+  T d4[NT][4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int e = ee[q];
@@ -678,51 +709,68 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       cs[q] = lw[q] ? f0 : e + 1;
       cn[q] = (lw[q] ? e : f1) - cs[q];
     }
-    d4[q] = lw[q] ? acc1[q] - acc2[q] : acc2[q] - acc1[q];
+#pragma unroll
+    for (int y = 0; y < NT; ++y) d4[y][q] = lw[q] ? acc1[y][q] - acc2[y][q] : acc2[y][q] - acc1[y][q];
   }
   {
-    T go[4], ou[4], od[4];
+    T go[4][NT], ou[4][NT], od[4][NT];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const bool on = ee[q] >= 0;
-      go[q] = on ? wk.jfield[(ww[q] * ne + ee[q]) * na + a] : (T)0;
-      ou[q] = on ? ws.Oup[ww[q] * na + a] : (T)0;
-      od[q] = on ? ws.Odn[ww[q] * na + a] : (T)0;
-    }
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (ee[q] < 0) continue;
-      const T own = lw[q] ? acc2[q] : acc1[q];
-      wk.jfield[(ww[q] * ne + ee[q]) * na + a] = go[q] - own;
-      ws.Oup[ww[q] * na + a] = ou[q] + (upm[q] ? own : acc1[q]);
-      ws.Odn[ww[q] * na + a] = od[q] + (upm[q] ? acc2[q] : own);
-    }
+      for (int y = 0; y < NT; ++y) {
+        const bool on = ee[q] >= 0 && in[y];
+        go[q][y] = on ? wk.jfield[(ww[q] * ne + ee[q]) * na + a[y]] : (T)0;
+        ou[q][y] = on ? ws.Oup[ww[q] * na + a[y]] : (T)0;
+        od[q][y] = on ? ws.Odn[ww[q] * na + a[y]] : (T)0;
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int y = 0; y < NT; ++y) {
+        if (ee[q] < 0 || !in[y]) continue;
+        const T own = lw[q] ? acc2[y][q] : acc1[y][q];
+        wk.jfield[(ww[q] * ne + ee[q]) * na + a[y]] = go[q][y] - own;
+        ws.Oup[ww[q] * na + a[y]] = ou[q][y] + (upm[q] ? own : acc1[y][q]);
+        ws.Odn[ww[q] * na + a[y]] = od[q][y] + (upm[q] ? acc2[y][q] : own);
+      }
   }
-  // individual corrections: rows cs .. cs + cn - 1 of each walker get d, four rows per pass with all their
+  // individual corrections: rows cs .. cs + cn - 1 of each walker get d, H rows per pass with all their
   // loads in flight together
   int nmax = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) nmax = cn[q] > nmax ? cn[q] : nmax;
-  for (int r = 0; r < nmax; r += 4) {
-    T v[4][4];
+  for (int r = 0; r < nmax; r += H) {
+    T v[H][4][NT];
 #pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        v[h][q] = r + h < cn[q] ? wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a] : (T)0;
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
+    for (int h = 0; h < H; ++h)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (r + h < cn[q]) wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a] = v[h][q] + d4[q];
+#pragma unroll
+        for (int y = 0; y < NT; ++y)
+          v[h][q][y] = r + h < cn[q] && in[y] ? wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a[y]] : (T)0;
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int y = 0; y < NT; ++y)
+          if (r + h < cn[q] && in[y])
+            wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a[y]] = v[h][q][y] + d4[y][q];
   }
 }
 
 // The J3 field update of one move.
 template <typename T, bool kDirect>
 inline void launch_jfield_move(const Sys& s, int64_t W, const WalkT<T>& wk, const SweepWs<T>& ws, hipStream_t st) {
-  const int64_t segs = (W + JF_SEG - 1) / JF_SEG, n_ct = (s.n_ao + 15) / 16;
-  k_sweep_jfield_mfma<T, kDirect><<<(unsigned)((segs + 7) / 8 * 8 * n_ct), 256, 0, st>>>(s, W, wk, ws);
+  const int64_t segs = (W + JF_SEG - 1) / JF_SEG;
+  auto run = [&](auto N) {
+    constexpr int NT = decltype(N)::value;
+    const int64_t n_ct = (s.n_ao + 16 * NT - 1) / (16 * NT);
+    k_sweep_jfield_mfma<T, kDirect, NT><<<(unsigned)((segs + 7) / 8 * 8 * n_ct), 256, 0, st>>>(s, W, wk, ws);
+  };
+  if constexpr (!kDirect)
+    if (segs * ((s.n_ao + 15) / 16) >= JF_WIDE_BLOCKS) return run(std::integral_constant<int, 2>{});
+  run(std::integral_constant<int, 1>{});
 }
 
 // Offsets into every field row and the AS factor into the walker state (one thread per element).
