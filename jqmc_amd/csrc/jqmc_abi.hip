@@ -367,9 +367,10 @@ int launch_sweep_batched(const jqmc_system* sys, int64_t W, const jqmc_walkers* 
   const WalkT<T> k = to_walk<T>(wk);
   SweepWs<T> ws(workspace, s, W);
   k_sweep_begin<T><<<grid_for(W, wpb), wpb * WAVE, lds, st>>>(sys->s, W, k, ws, wpb, per_wave);
+  const auto propose = W > PROP_MANY ? &k_sweep_propose<T, true> : &k_sweep_propose<T, false>;
   for (int m = 0; m < n_moves; ++m) {
-    k_sweep_propose<T><<<grid_for(W, wpb), wpb * WAVE, lds, st>>>(sys->s, W, k, ws, m, Dt, epsilon_AS, seed,
-                                                                  move0, move_ctr, wpb, per_wave);
+    propose<<<grid_for(W, wpb), wpb * WAVE, lds, st>>>(sys->s, W, k, ws, m, Dt, epsilon_AS, seed, move0, move_ctr,
+                                                       wpb, per_wave);
     if (s.j3_on) launch_jfield_move<T, false>(sys->s, W, k, ws, st);
   }
   const int64_t n_flush = std::max<int64_t>(s.j3_on ? W * s.n_el * s.n_ao : 0, W);

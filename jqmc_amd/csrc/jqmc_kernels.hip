@@ -38,8 +38,8 @@ struct Carve {
 
 // y[k] = sum_a CT[a, k] x[a] for k < no, all 64 lanes busy: lanes split into groups of
 // lg >= no lanes, group g sums a = g, g + G, ...; groups combine by butterfly shuffles.  The sums
-// run in TY (FP64 for the orbital rows, whatever the type of the AO values x).
-template <typename TC, typename TX, typename TY>
+// run in TY (FP64 for the orbital rows, whatever the type of the AO values x), with kLoads steps in flight.
+template <typename TC, typename TX, typename TY, int kLoads = 8>
 __device__ inline void wave_matvec_T(const TC* __restrict__ CT, const TX* x, int na, int no, int lane, TY* y) {
   int lg = 64;
   while (lg / 2 >= no && lg > 1) lg >>= 1;
@@ -48,7 +48,7 @@ __device__ inline void wave_matvec_T(const TC* __restrict__ CT, const TX* x, int
     const int kk = kb + k;
     TY acc = 0;
     if (kk < no) {
-#pragma unroll 8
+#pragma unroll kLoads
       for (int a = grp; a < na; a += G) acc += (TY)CT[(int64_t)a * no + kk] * (TY)x[a];
     }
     for (int off = lg; off < WAVE; off <<= 1) acc += __shfl_xor(acc, off, WAVE);
@@ -419,10 +419,15 @@ inline int64_t sweep_lds_bytes(const Sys& s) {
 
 __device__ __forceinline__ double step_factor(double Z, double d) { return 1.0 / (Z * Z) * (1.0 + Z * Z * d) / (1.0 + d); }
 
+// Nuclei up to which the plain loop is no slower than the two reductions over the wave: a move for one
+// or two nuclei takes 0.3 to 0.8 of 21 us less, for three and four the same, for the six of H6 2.6 of 48 us more (8192
+// walkers, FP32).
+constexpr int NEAREST_SERIAL = 3;
+
 // nearest_nucleus by one wavefront, a nucleus per lane: the smallest distance, the first of equal ones (and the
 // first nucleus if no distance is a number).
 __device__ __forceinline__ int nearest_nucleus_wave(const Sys& s, double x, double y, double z, int lane) {
-  if (s.n_nuc > WAVE) return nearest_nucleus(s, x, y, z);
+  if (s.n_nuc <= NEAREST_SERIAL || s.n_nuc > WAVE) return nearest_nucleus(s, x, y, z);
   double d = __builtin_inf();
   if (lane < s.n_nuc) {
     const double dx = s.nuc_pos[3 * lane] - x, dy = s.nuc_pos[3 * lane + 1] - y, dz = s.nuc_pos[3 * lane + 2] - z;
@@ -449,7 +454,6 @@ __device__ inline double sweep_as_factor(const LdsT& L, int nu, int lane, int mo
   double smin = 1.0e300;
   for (int p = lane; p < nu; p += WAVE) {
     double rs = 0.0, cs = 0.0;
-#pragma unroll 8
     for (int q = 0; q < nu; ++q) {
       double gr = L.Gm[p * nu + q], gc = L.Gm[q * nu + p];
       if (mode == 1) {

@@ -155,15 +155,23 @@ __global__ void __launch_bounds__(256) k_sweep_begin(Sys s, int64_t W, WalkT<T> 
 }
 
 // Move m of the sweep for every walker (the body of k_vmc_sweep's move loop).
-// Registers capped at 128 (4 waves per SIMD): the per-walker chain is latency bound, and the LDS of 4
-// walkers per block allows 16 waves per CU.  The nearest nucleus by a nucleus per lane, shells from their
-// records and eight loads in flight in the orbital, pair-row and AS sums: 33 -> 27 us a move for 1024 benzene
-// walkers, 169 -> 163 for 16384, 40.5 -> 36.8 for 2048 of 4 x H2O (FP32), 18.4 -> 17.1 for 256 of H2O.
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_sweep_propose(Sys s, int64_t W, WalkT<T> wk,
-                                                       SweepWs<T> ws, int m, double Dt, double eps_AS, uint64_t seed,
-                                                       int64_t move_base, const int64_t* __restrict__ move_ctr,
-                                                       int wpb, int64_t lds_per_wave) {
+// A chain of dependent steps per walker, bound by latency while every wave has its place on the card at once and
+// by the waves in flight beyond that, so there are two forms.  Up to PROP_MANY walkers (kMany false; 82 registers
+// in FP32, 94 in FP64: five waves per SIMD) FP64 shells come from their records and eight loads are in flight in
+// the orbital sums and, in FP64, in those of the new pair row.  More walkers take four loads and the shell loop (66
+// and 69 registers, seven waves per SIMD), with the same bits.  Both find the nearest nucleus by a nucleus per lane.
+// The few against one form of the shell loop with four loads and a serial nearest nucleus: 33 -> 26 us for 1024
+// benzene walkers, 40.5 -> 36.8 for 2048 of 4 x H2O (FP32), 18.4 -> 17.1 for 256 of H2O.  A move of the whole sweep
+// with eight loads and records for all -> with the many: benzene FP64 6144 walkers 146 -> 136 us, mixed 120 -> 103;
+// 16384 357 -> 356 and 281 -> 268; 4 x H2O 16384 FP64 486 -> 466, mixed 351 -> 341; N2 16384 86.8 -> 82.1 and
+// 85.0 -> 76.6; one H 6144 36.2 -> 33.7 and 37.5 -> 32.3.  Around 7168 walkers, where the many just fit in one go,
+// FP64 takes up to 4 % longer (benzene 172 -> 176 us).  For 2048 walkers of 4 x H2O the many cost 2 of 66 us.
+template <typename T, bool kMany>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+    k_sweep_propose(Sys s, int64_t W, WalkT<T> wk, SweepWs<T> ws, int m, double Dt, double eps_AS, uint64_t seed,
+                    int64_t move_base, const int64_t* __restrict__ move_ctr, int wpb, int64_t lds_per_wave) {
+  constexpr bool kF64 = std::is_same<T, double>::value;
+  constexpr int kOrbLoads = kMany ? 4 : 8, kPairLoads = kF64 && !kMany ? 8 : 4;
   extern __shared__ double smem[];
   const RealTabs<T>& R = tabs<T>(s);
   const int wave = wave_id(), lane = lane_id();
@@ -237,7 +245,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 
   // ---- AO values at the new position, Jastrow log-ratio
   for (int sh = lane; sh < s.n_shell; sh += WAVE) {
-    if constexpr (std::is_same<T, double>::value)
+    if constexpr (kF64 && !kMany)
       shell_record_values(s, sh, nx, ny, nz, L.anew);
     else
       shell_values<T>(s, sh, nx, ny, nz, L.anew);
@@ -283,7 +291,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   // ---- orbitals at the new position (FP64 sums of the AO values) and their change
   const double* Pe = Pw + (int64_t)e * no;
   if (s.orb_is_mo) {
-    wave_matvec_T(is_up ? s.td.mo_upT : s.td.mo_dnT, L.anew, na, no, lane, L.phin);
+    wave_matvec_T<double, T, double, kOrbLoads>(is_up ? s.td.mo_upT : s.td.mo_dnT, L.anew, na, no, lane, L.phin);
     wave_sync();
   } else {
     for (int k = lane; k < no; k += WAVE) L.phin[k] = (double)L.anew[k];
@@ -298,7 +306,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       double v = 0.0;
       if (j < nd) {
         const double* pr = L.pr + (int64_t)j * no;
-#pragma unroll 8
+#pragma unroll 4
         for (int k = 0; k < no; ++k) v += L.dphi[k] * pr[k];
       } else {
         for (int k = 0; k < no; ++k) v += L.dphi[k] * s.td.lam_u[(int64_t)k * s.n_unp + (j - nd)];
@@ -310,7 +318,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     for (int i = lane; i < nu; i += WAVE) {
       const double* pr = L.pr + (int64_t)i * no;
       double u = 0.0;
-#pragma unroll 8
+#pragma unroll 4
       for (int k = 0; k < no; ++k) u += pr[k] * L.dphi[k];
       L.vv[i] = u;
       part += L.Gi[idx * nu + i] * u;
@@ -361,7 +369,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     for (int k = lane; k < no; k += WAVE) {
       Pem[k] = L.phin[k];
       double q = 0.0;
-#pragma unroll 8
+#pragma unroll kPairLoads
       for (int j = 0; j < no; ++j) q += Lm[(int64_t)j * no + k] * L.phin[j];
       Qem[k] = q;
     }
@@ -378,6 +386,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     wk.rejected[w] += 1;
   }
 }
+
+// Walkers up to which every wave of k_sweep_propose<T, false> is on the card at once: five on each of 4 x 256 SIMDs.
+constexpr int64_t PROP_MANY = 5 * 4 * 256;
 
 constexpr int JF_SEG = 64;      // walkers whose movers one block collects
 constexpr int JF_KC = 16;       // AO columns per step

@@ -54,10 +54,10 @@ def test_fields_after_moves(name, W, sym):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("sym", [False, True])
 @pytest.mark.parametrize("name,W", [("water_ae", 49153), ("benzene_ecp", 6593)])
-def test_two_tiles_give_the_bits_of_one(name, W, sym, precision):
-    """Many walkers take two tiles of 16 AOs a wave; the sums of an element stay the same, and the draws of a walker
-    depend on its index alone, so the first walkers of a large set end as those of a small one do.  25 and 228 AOs:
-    the last pair of tiles holds 25 and 4 columns."""
+def test_many_walkers_give_the_bits_of_few(name, W, sym, precision):
+    """Many walkers take two tiles of 16 AOs a wave and the proposal with fewer loads in flight; the sums of an element
+    stay the same, and the draws of a walker depend on its index alone, so the first walkers of a large set end as
+    those of a small one do.  25 and 228 AOs: the last pair of tiles holds 25 and 4 columns."""
     from jqmc_amd._api import WalkerState
     from jqmc_amd._pack import SystemPack
 
@@ -71,7 +71,7 @@ def test_two_tiles_give_the_bits_of_one(name, W, sym, precision):
         return ws
 
     many, few = run(W), run(300)
-    assert -(-W // 64) * -(-pack.n_ao // 16) >= 6 * 256 and int(few.accepted.sum()) > 0
+    assert W > 5 * 4 * 256 and -(-W // 64) * -(-pack.n_ao // 16) >= 6 * 256 and int(few.accepted.sum()) > 0
     assert torch.equal(many.r_up[:300], few.r_up) and torch.equal(many.jfield[:300], few.jfield)
     if precision == "fp64":
         ref = WalkerState(pack, W).init(many.r_up.cpu().numpy(), many.r_dn.cpu().numpy()).jfield
