@@ -419,15 +419,16 @@ inline int64_t sweep_lds_bytes(const Sys& s) {
 
 __device__ __forceinline__ double step_factor(double Z, double d) { return 1.0 / (Z * Z) * (1.0 + Z * Z * d) / (1.0 + d); }
 
-// Nuclei up to which the plain loop is no slower than the two reductions over the wave: a move for one
-// or two nuclei takes 0.3 to 0.8 of 21 us less, for three and four the same, for the six of H6 2.6 of 48 us more (8192
-// walkers, FP32).
+// Nuclei up to which the plain loop is no slower than the two reductions over the wave: a move for one or two nuclei
+// takes 0.3 to 0.8 of 21 us less, for three and four the same, for the six of H6 2.6 of 48 us more (8192 walkers,
+// FP32).  kLoop is false for few walkers in FP64, where the choice itself costs benzene 0.4 of 42 us and H2 gains 0.2.
 constexpr int NEAREST_SERIAL = 3;
 
 // nearest_nucleus by one wavefront, a nucleus per lane: the smallest distance, the first of equal ones (and the
 // first nucleus if no distance is a number).
+template <bool kLoop>
 __device__ __forceinline__ int nearest_nucleus_wave(const Sys& s, double x, double y, double z, int lane) {
-  if (s.n_nuc <= NEAREST_SERIAL || s.n_nuc > WAVE) return nearest_nucleus(s, x, y, z);
+  if ((kLoop && s.n_nuc <= NEAREST_SERIAL) || s.n_nuc > WAVE) return nearest_nucleus(s, x, y, z);
   double d = __builtin_inf();
   if (lane < s.n_nuc) {
     const double dx = s.nuc_pos[3 * lane] - x, dy = s.nuc_pos[3 * lane + 1] - y, dz = s.nuc_pos[3 * lane + 2] - z;

@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 
   // ---- proposal with nearest-nucleus step size (jqmc_mcmc.py:4339-4401)
   const double ox = L.rr[3 * e], oy = L.rr[3 * e + 1], oz = L.rr[3 * e + 2];
-  const int na0 = nearest_nucleus_wave(s, ox, oy, oz, lane);
+  const int na0 = nearest_nucleus_wave<!kF64 || kMany>(s, ox, oy, oz, lane);
   const double Z0 = s.nuc_charge[na0];
   double dxn = ox - s.nuc_pos[3 * na0], dyn = oy - s.nuc_pos[3 * na0 + 1], dzn = oz - s.nuc_pos[3 * na0 + 2];
   const double f_l = step_factor(Z0, sqrt(dxn * dxn + dyn * dyn + dzn * dzn));
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
   if (axis == 0) nx += g;
   else if (axis == 1) ny += g;
   else nz += g;
-  const int na1 = nearest_nucleus_wave(s, nx, ny, nz, lane);
+  const int na1 = nearest_nucleus_wave<!kF64 || kMany>(s, nx, ny, nz, lane);
   const double Z1 = s.nuc_charge[na1];
   dxn = nx - s.nuc_pos[3 * na1];
   dyn = ny - s.nuc_pos[3 * na1 + 1];
@@ -679,28 +679,27 @@ __global__ void __launch_bounds__(256)
     ww[q] = w0 + at_s[r < n ? r : 0];
   }
   if constexpr (kDirect) {
-    // H rows of the four walkers per pass, all 16 loads in flight together
-    for (int f0 = 0; f0 < ne; f0 += H) {
-      T v[H][4][NT];
+    static_assert(!kDirect || NT == 1);
+    const int a1 = a[0];
+    const v4 t1 = acc1[0], t2 = acc2[0];
+    // four rows of the four walkers per pass, all 16 loads in flight together
+    for (int f0 = 0; f0 < ne; f0 += 4) {
+      T v[4][4];
 #pragma unroll
-      for (int h = 0; h < H; ++h)
+      for (int h = 0; h < 4; ++h)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q) {
+          const int f = f0 + h;
+          v[h][q] = (f < ne && ee[q] >= 0 && f != ee[q]) ? wk.jfield[(ww[q] * ne + f) * na + a1] : (T)0;
+        }
 #pragma unroll
-          for (int y = 0; y < NT; ++y) {
-            const int f = f0 + h;
-            v[h][q][y] = (f < ne && ee[q] >= 0 && f != ee[q] && in[y]) ? wk.jfield[(ww[q] * ne + f) * na + a[y]] : (T)0;
-          }
+      for (int h = 0; h < 4; ++h)
 #pragma unroll
-      for (int h = 0; h < H; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int y = 0; y < NT; ++y) {
-            const int f = f0 + h;
-            if (f < ne && ee[q] >= 0 && f != ee[q] && in[y])
-              wk.jfield[(ww[q] * ne + f) * na + a[y]] = v[h][q][y] + (f < ee[q] ? acc1[y][q] : acc2[y][q]);
-          }
+        for (int q = 0; q < 4; ++q) {
+          const int f = f0 + h;
+          if (f < ne && ee[q] >= 0 && f != ee[q])
+            wk.jfield[(ww[q] * ne + f) * na + a1] = v[h][q] + (f < ee[q] ? t1[q] : t2[q]);
+        }
     }
     return;
   }
@@ -722,6 +721,44 @@ __global__ void __launch_bounds__(256)
     }
 #pragma unroll
     for (int y = 0; y < NT; ++y) d4[y][q] = lw[q] ? acc1[y][q] - acc2[y][q] : acc2[y][q] - acc1[y][q];
+  }
+  if constexpr (std::is_same<T, double>::value && NT == 1) {
+    // the updates below written without the loops over tiles, which take FP64 0.5 of 20 us more (1024 benzene walkers)
+    const int a1 = a[0];
+    const v4 t1 = acc1[0], t2 = acc2[0];
+    T go[4], ou[4], od[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bool on = ee[q] >= 0;
+      go[q] = on ? wk.jfield[(ww[q] * ne + ee[q]) * na + a1] : (T)0;
+      ou[q] = on ? ws.Oup[ww[q] * na + a1] : (T)0;
+      od[q] = on ? ws.Odn[ww[q] * na + a1] : (T)0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (ee[q] < 0) continue;
+      const T own = lw[q] ? t2[q] : t1[q];
+      wk.jfield[(ww[q] * ne + ee[q]) * na + a1] = go[q] - own;
+      ws.Oup[ww[q] * na + a1] = ou[q] + (upm[q] ? own : t1[q]);
+      ws.Odn[ww[q] * na + a1] = od[q] + (upm[q] ? t2[q] : own);
+    }
+    int nmax = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) nmax = cn[q] > nmax ? cn[q] : nmax;
+    for (int r = 0; r < nmax; r += 4) {
+      T v[4][4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[h][q] = r + h < cn[q] ? wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a1] : (T)0;
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (r + h < cn[q]) wk.jfield[(ww[q] * ne + cs[q] + r + h) * na + a1] = v[h][q] + d4[0][q];
+    }
+    return;
   }
   {
     T go[4][NT], ou[4][NT], od[4][NT];
