@@ -719,8 +719,12 @@ __global__ void __launch_bounds__(256)
       cs[q] = lw[q] ? f0 : e + 1;
       cn[q] = (lw[q] ? e : f1) - cs[q];
     }
+    if constexpr (NT == 1) {
+      d4[0][q] = lw[q] ? acc1[0][q] - acc2[0][q] : acc2[0][q] - acc1[0][q];
+    } else {
 #pragma unroll
-    for (int y = 0; y < NT; ++y) d4[y][q] = lw[q] ? acc1[y][q] - acc2[y][q] : acc2[y][q] - acc1[y][q];
+      for (int y = 0; y < NT; ++y) d4[y][q] = lw[q] ? acc1[y][q] - acc2[y][q] : acc2[y][q] - acc1[y][q];
+    }
   }
   if constexpr (std::is_same<T, double>::value && NT == 1) {
     // the updates below written without the loops over tiles, which take FP64 0.5 of 20 us more (1024 benzene walkers)
